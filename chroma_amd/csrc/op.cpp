@@ -191,7 +191,10 @@ Op* make_op(std::shared_ptr<GaugeData> gd, const cmx_op_params& p) {
                 "op_create: links are not SU(3) up to a per-direction boundary phase (deviation " +
                     std::to_string(gd->su3_dev) + "); use CMX_SINGLE with CMX_RECONS_18");
   CMX_HIP(hipStreamCreate(&op->stream));
-  op->npartials = std::max(2 * (int)((op->Vh + 63) / 64), blas_blocks((int)op->V)) * 4;
+  // three sums per work-group of two launches at most; the plane-grid kernel has at least one work-group
+  // per (z, t) plane, however few sites the plane holds
+  const int plane_wgs = (op->g.Lxh * op->g.L[1] + 63) / 64 * op->g.L[2] * op->g.L[3];
+  op->npartials = std::max(2 * std::max((int)((op->Vh + 63) / 64), plane_wgs), blas_blocks((int)op->V)) * 4;
   op->partials.alloc(sizeof(double) * op->npartials);
   op->state_S.alloc(sizeof(double) * S_NSLOTS);
   op->state_F.alloc(sizeof(int) * F_NFLAGS);
