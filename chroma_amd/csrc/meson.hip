@@ -6,8 +6,9 @@
 // the source, t_eff = (t - origin_t) mod L_t (mesons_w.cc:160-165).
 //
 // Every Gamma(n) and gamma_5 of the DeGrand-Rossi basis (docs/notes/gamma_conventions.tex:74-79) has one
-// non-zero entry, a power of i, per row, so each of the 16 spin blocks (a, b) of the trace reads one 3x3
-// colour block of S_2 and one of S_1 with a fixed coefficient; the host builds that table per Gamma.
+// non-zero entry, a power of i, per row: gamma_5 is diagonal, and Gamma(n) maps spin a to spin a ^ k(n) with
+// one of four masks k.  So the trace needs, for each of the 16 spin blocks (a, b) of S_2, the 3x3 colour
+// products with the four blocks (a^k, b^k) of S_1, and every Gamma is a signed sum of those 64 numbers.
 // Propagators: [site][sink spin*3 + colour][source spin*3 + colour] complex, sites in the host order.
 #include <algorithm>
 #include <cmath>
@@ -20,11 +21,6 @@
 namespace cmx {
 
 namespace {
-
-struct Term {  // one spin block (a, b) of the trace for one Gamma
-  double2 coef;
-  int r2, c2, r1, c1;  // spin row / column of the S_2 and S_1 colour blocks
-};
 
 // signed permutation: row a has its one non-zero entry ph[a] in column p[a]
 struct SPerm {
@@ -60,73 +56,33 @@ SPerm gamma_n(int n) {
   return g;
 }
 
-// c_n = sum_{a,b} sum_{ij} conj(anti_{(a,i),(b,j)}) (G S_1 G)_{(a,i),(b,j)} with anti = g5 S_2 g5:
-// anti_{(a,i),(b,j)} = g5ph[a] S_2[(p5[a],i),(q,j)] g5ph[q] where p5[q] = b, and
+// k(n): Gamma(n) maps spin a to a ^ k (gamma_1, gamma_2 flip with 3, gamma_3, gamma_4 with 2)
+__host__ __device__ constexpr int meson_mask(int n) {
+  return (((n ^ (n >> 1)) & 1) ? 3 : 0) ^ ((((n >> 2) ^ (n >> 3)) & 1) ? 2 : 0);
+}
+
+// c_n = sum_{a,b} coef[n][a][b] T_k(a,b), T_k(a,b) = sum_{ij} conj(S_2[(a,i),(b,j)]) S_1[(a^k,i),(b^k,j)]:
+// anti_{(a,i),(b,j)} = g5ph[a] S_2[(a,i),(b,j)] g5ph[b] (gamma_5 diagonal) and
 // (G S_1 G)_{(a,i),(b,j)} = Gph[a] S_1[(pG[a],i),(r,j)] Gph[r] where pG[r] = b.
-std::vector<Term> meson_terms() {
+std::vector<double2> meson_coefs() {
   const SPerm g5 = gamma_n(15);
-  std::vector<Term> t;
+  std::vector<double2> t;
   for (int n = 0; n < 16; ++n) {
     const SPerm G = gamma_n(n);
+    const int k = meson_mask(n);
     for (int a = 0; a < 4; ++a)
       for (int b = 0; b < 4; ++b) {
-        int q = -1, r = -1;
-        for (int k = 0; k < 4; ++k) {
-          if (g5.p[k] == b) q = k;
-          if (G.p[k] == b) r = k;
-        }
-        // conj(g5ph[a] g5ph[q]) Gph[a] Gph[r]
-        const double ar = g5.ph_re[a] * g5.ph_re[q] - g5.ph_im[a] * g5.ph_im[q];
-        const double ai = -(g5.ph_re[a] * g5.ph_im[q] + g5.ph_im[a] * g5.ph_re[q]);
+        const int r = b ^ k;
+        CMX_REQUIRE(g5.p[a] == a && G.p[a] == (a ^ k) && G.p[r] == b, CMX_ERR_STATE, "meson_2pt: gamma table");
+        // conj(g5ph[a] g5ph[b]) Gph[a] Gph[r]
+        const double ar = g5.ph_re[a] * g5.ph_re[b] - g5.ph_im[a] * g5.ph_im[b];
+        const double ai = -(g5.ph_re[a] * g5.ph_im[b] + g5.ph_im[a] * g5.ph_re[b]);
         const double br = G.ph_re[a] * G.ph_re[r] - G.ph_im[a] * G.ph_im[r];
         const double bi = G.ph_re[a] * G.ph_im[r] + G.ph_im[a] * G.ph_re[r];
-        t.push_back(Term{make_double2(ar * br - ai * bi, ar * bi + ai * br), g5.p[a], q, G.p[a], r});
+        t.push_back(make_double2(ar * br - ai * bi, ar * bi + ai * br));
       }
   }
   return t;
-}
-
-// MESON_SITES sites per block, one lane per (site, Gamma): the block first copies its sites' two
-// propagators (2 x 2304 B per site, contiguous) into LDS with coalesced loads, then each lane forms its
-// trace from LDS, so HBM sees each propagator once instead of the 16 re-reads a lane per (site, Gamma)
-// would make through the caches.  The block range is the nsite sites from s1/s2 (already offset to the
-// range's first site); c[n * cstride + coff + i] for the range's site i.
-constexpr int MESON_SITES = 8;
-
-__global__ void __launch_bounds__(16 * MESON_SITES) k_meson_sites(long nsites, const double2* __restrict__ s1,
-                                                                  const double2* __restrict__ s2,
-                                                                  const Term* __restrict__ terms,
-                                                                  double2* __restrict__ c, long cstride, long coff) {
-  __shared__ double2 sh1[MESON_SITES * 144], sh2[MESON_SITES * 144];
-  const long site0 = (long)blockIdx.x * MESON_SITES;
-  const int nsite = nsites - site0 < MESON_SITES ? (int)(nsites - site0) : MESON_SITES;
-  for (int q = threadIdx.x; q < nsite * 144; q += blockDim.x) {
-    sh1[q] = s1[site0 * 144 + q];
-    sh2[q] = s2[site0 * 144 + q];
-  }
-  __syncthreads();
-  const int ls = (int)threadIdx.x >> 4;
-  const int n = (int)threadIdx.x & 15;
-  if (ls >= nsite) return;
-  const double2* p1 = sh1 + ls * 144;
-  const double2* p2 = sh2 + ls * 144;
-  double cr = 0, ci = 0;
-  for (int k = 0; k < 16; ++k) {
-    const Term tm = terms[n * 16 + k];
-    double sr = 0, si = 0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double2 x = p2[(tm.r2 * 3 + i) * 12 + tm.c2 * 3 + j];
-        const double2 y = p1[(tm.r1 * 3 + i) * 12 + tm.c1 * 3 + j];
-        sr += x.x * y.x + x.y * y.y;  // conj(x) y
-        si += x.x * y.y - x.y * y.x;
-      }
-    cr += tm.coef.x * sr - tm.coef.y * si;
-    ci += tm.coef.x * si + tm.coef.y * sr;
-  }
-  c[(size_t)n * cstride + coff + site0 + ls] = make_double2(cr, ci);
 }
 
 struct ProjGeom {
@@ -135,51 +91,181 @@ struct ProjGeom {
   int org[4];
 };
 
-// Where k_meson_project finds the correlator of a site (cb, lex) of time slice t0 + blockIdx.x:
-// c[n * cstride + cb * cb_off + lex / 2 - lex_off].  Whole lattice: cstride V, cb_off Vh, lex_off 0.
-struct CorrIndex {
-  int t0;
-  long cstride, cb_off, lex_off;
+// Contraction and projection in one pass over the propagators, which it reads once (HBM-bound: 2304 B per
+// site and propagator against 4352 FP64 FMAs and 11.5 KB of LDS reads).  A work-group walks a range of one
+// time slice MESON_SITES sites at a time: the sites go to LDS with direct loads (double-buffered: the next
+// group is on its way while this one is contracted, and no registers hold it, which the 4 NM complex sums
+// per lane need), lane (site, a, b) forms T_0..T_3 of its spin block and adds phase_m(x) T_k to its sums;
+// Gamma and the momenta never meet per site.  At the end the lanes' sums are combined over sites and spins
+// (fixed order) and the work-group writes its 16 x NM partial correlators.
+// 24^3x48, 7 momenta, S_1 = S_2: two kernels that stored the 16 site correlators (one trace per lane and
+// Gamma, 256 colour products per site) and read them back per momentum took 2.17 ms.
+constexpr int MESON_SITES = 16;
+constexpr int MESON_NM = 8;  // momenta per pass over the propagators
+
+struct MesonArgs {
+  ProjGeom g;
+  const double2 *s1, *s2, *coef;
+  const int* moms;
+  int nmom;    // momenta of this launch
+  int t0;      // first time slice of this launch
+  int nchunk;  // work-groups per time slice
+  int groups;  // groups of MESON_SITES sites per work-group
+  double2* phase;  // [momentum][x, then y, then z]: exp(i 2 pi k (x - origin) / L) of each direction
+  double2* part;   // [slice of this launch][chunk][momentum][n]
 };
 
-// one block per (time slice, momentum): out[n][m][t_eff] = sum over the slice of phase(x) c[n][x], summed in
-// a fixed order (strided per lane, then a tree over the block), so the result is deterministic
-__global__ void __launch_bounds__(256) k_meson_project(ProjGeom g, CorrIndex ci, const double2* __restrict__ c,
-                                                       const int* __restrict__ moms, int nmom,
-                                                       double2* __restrict__ out) {
-  __shared__ double2 red[256];
-  const int t = ci.t0 + (int)blockIdx.x, m = blockIdx.y;
-  const long Vs = (long)g.L[0] * g.L[1] * g.L[2];
-  const double k0 = 6.283185307179586 * moms[3 * m] / g.L[0], k1 = 6.283185307179586 * moms[3 * m + 1] / g.L[1],
-               k2 = 6.283185307179586 * moms[3 * m + 2] / g.L[2];
-  double2 acc[16];
+// the phase factors of each direction, from the product k (x - origin) reduced mod L in integers
+__global__ void __launch_bounds__(256) k_meson_phase(MesonArgs A) {
+  const int nx = A.g.L[0] + A.g.L[1] + A.g.L[2];
+  const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x), m = blockIdx.y;
+  if (q >= nx) return;
+  const int d = q < A.g.L[0] ? 0 : (q < A.g.L[0] + A.g.L[1] ? 1 : 2);
+  const int x = q - (d > 0 ? A.g.L[0] : 0) - (d > 1 ? A.g.L[1] : 0);
+  const long L = A.g.L[d];
+  long r = ((long)A.moms[3 * m + d] * (x - A.g.org[d])) % L;
+  double2 p;
+  sincospi(2.0 * (double)r / (double)L, &p.y, &p.x);
+  A.phase[(size_t)m * nx + q] = p;
+}
+
+__device__ __forceinline__ double2 cmul2(double2 a, double2 b) {
+  return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
+}
+
+template <int NM, bool SAME> __global__ void __launch_bounds__(256, 2) k_meson(MesonArgs A) {
+  constexpr int SB = MESON_SITES * 144;  // 256 threads x 9 elements of 16 B
+  __shared__ __align__(16) double2 stage[2][SAME ? 1 : 2][SB];
+  __shared__ double2 shp[2][MESON_SITES * NM];
+  static_assert(4 * NM * 4 * 16 <= SB, "the final combination re-uses a staging buffer");
+  const int tid = threadIdx.x, ab = tid & 15, slot = tid >> 4, a = ab >> 2, b = ab & 3;
+  const int t = A.t0 + (int)blockIdx.x / A.nchunk, chunk = (int)blockIdx.x % A.nchunk;
+  const int m0 = (int)blockIdx.y * NM;
+  const int Lxh = A.g.L[0] / 2, Ly = A.g.L[1];
+  const int Vsh = Lxh * Ly * A.g.L[2];  // sites of the slice per checkerboard
+  const int vbeg = chunk * A.groups * MESON_SITES;
+  const int vend = min(2 * Vsh, vbeg + A.groups * MESON_SITES);
+  const int nx = A.g.L[0] + A.g.L[1] + A.g.L[2];
+  // stages the MESON_SITES sites from v0 (site v of the slice: even sites first, each checkerboard a
+  // contiguous range of the host order).  Lanes past the range re-read its last site: their phase is zero.
+  auto fetch = [&](int v0, int buf) {
 #pragma unroll
-  for (int n = 0; n < 16; ++n) acc[n] = make_double2(0, 0);
-  for (long v = threadIdx.x; v < Vs; v += blockDim.x) {
-    const int x0 = (int)(v % g.L[0]), x1 = (int)(v / g.L[0] % g.L[1]), x2 = (int)(v / ((long)g.L[0] * g.L[1]));
-    const long lex = v + Vs * t;
-    const long idx = ((x0 + x1 + x2 + t) & 1) * ci.cb_off + lex / 2 - ci.lex_off;
-    double sn, cs;
-    sincos(k0 * (x0 - g.org[0]) + k1 * (x1 - g.org[1]) + k2 * (x2 - g.org[2]), &sn, &cs);
+    for (int j = 0; j < 9; ++j) {
+      const int q = tid + 256 * j, sl = q / 144, e = q - sl * 144;
+      const int v = min(v0 + sl, vend - 1);
+      const int cb = v >= Vsh ? 1 : 0;
+      const size_t at = ((size_t)cb * A.g.Vh + (size_t)t * Vsh + (v - cb * Vsh)) * 144 + e;
+      const int w = (tid & ~63) + 256 * j;  // a wave's 64 elements are consecutive in LDS
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s1 + at),
+                                       (__attribute__((address_space(3))) void*)&stage[buf][0][w], 16, 0, 0);
+      if constexpr (!SAME)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s2 + at),
+                                         (__attribute__((address_space(3))) void*)&stage[buf][1][w], 16, 0, 0);
+    }
+    if (tid < MESON_SITES * NM) {
+      const int m = m0 + tid % NM, v = v0 + tid / NM;
+      double2 p = make_double2(0, 0);
+      if (v < vend && m < A.nmom) {
+        const int cb = v >= Vsh ? 1 : 0;
+        int r = v - cb * Vsh;
+        const int xh = r % Lxh;
+        r /= Lxh;
+        const int y = r % Ly, z = r / Ly;
+        const int x = 2 * xh + ((cb + y + z + t) & 1);
+        const double2* f = A.phase + (size_t)m * nx;
+        p = cmul2(cmul2(f[x], f[A.g.L[0] + y]), f[A.g.L[0] + Ly + z]);
+      }
+      shp[buf][tid] = p;  // [site][momentum]
+    }
+  };
+  double2 acc[NM][4];
 #pragma unroll
-    for (int n = 0; n < 16; ++n) {
-      const double2 z = c[(size_t)n * ci.cstride + idx];
-      acc[n].x += cs * z.x - sn * z.y;
-      acc[n].y += cs * z.y + sn * z.x;
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[m][k] = make_double2(0, 0);
+  if (vbeg < vend) fetch(vbeg, 0);
+  int buf = 0;
+  for (int v0 = vbeg; v0 < vend; v0 += MESON_SITES, buf ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's direct loads have reached LDS
+    __syncthreads();
+    if (v0 + MESON_SITES < vend) fetch(v0 + MESON_SITES, buf ^ 1);
+    const double2* p1 = stage[buf][0] + slot * 144;
+    const double2* p2 = stage[buf][SAME ? 0 : 1] + slot * 144 + a * 36 + b * 3;
+    double2 x[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) x[3 * i + j] = p2[i * 12 + j];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double2* q = p1 + (a ^ k) * 36 + (b ^ k) * 3;
+      double sr = 0, si = 0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const double2 u = x[3 * i + j], w = q[i * 12 + j];
+          sr = fma(u.x, w.x, fma(u.y, w.y, sr));
+          si = fma(u.x, w.y, fma(-u.y, w.x, si));
+        }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const double2 p = shp[buf][slot * NM + m];
+        acc[m][k].x = fma(p.x, sr, fma(-p.y, si, acc[m][k].x));
+        acc[m][k].y = fma(p.x, si, fma(p.y, sr, acc[m][k].y));
+      }
     }
   }
-  const int teff = (t - g.org[3] % g.L[3] + g.L[3]) % g.L[3];
-  for (int n = 0; n < 16; ++n) {
-    red[threadIdx.x] = acc[n];
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w)
-        red[threadIdx.x] = make_double2(red[threadIdx.x].x + red[threadIdx.x + w].x, red[threadIdx.x].y + red[threadIdx.x + w].y);
-      __syncthreads();
+  __syncthreads();
+  double2* sh1 = stage[0][0];
+  // over the wave's four sites, then the four waves and the spins
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int off = 16; off < 64; off <<= 1) {
+        acc[m][k].x += __shfl_xor(acc[m][k].x, off, 64);
+        acc[m][k].y += __shfl_xor(acc[m][k].y, off, 64);
+      }
+      if ((tid & 63) < 16) sh1[(((tid >> 6) * NM + m) * 4 + k) * 16 + ab] = acc[m][k];
     }
-    if (threadIdx.x == 0) out[((size_t)n * nmom + m) * g.L[3] + teff] = red[0];
-    __syncthreads();
+  __syncthreads();
+  if (tid < 16 * NM) {
+    const int n = tid & 15, m = tid >> 4, k = meson_mask(n);
+    if (m0 + m < A.nmom) {
+      double cr = 0, ci = 0;
+      for (int s = 0; s < 16; ++s) {
+        double2 z = make_double2(0, 0);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const double2 u = sh1[((w * NM + m) * 4 + k) * 16 + s];
+          z.x += u.x;
+          z.y += u.y;
+        }
+        const double2 c = A.coef[n * 16 + s];
+        cr += c.x * z.x - c.y * z.y;
+        ci += c.x * z.y + c.y * z.x;
+      }
+      A.part[((size_t)blockIdx.x * A.nmom + m0 + m) * 16 + n] = make_double2(cr, ci);
+    }
   }
+}
+
+// out[n][m0 + m][t_eff] = sum over the slice's chunks, in order (deterministic); one lane per (m, n) of a slice
+__global__ void __launch_bounds__(256) k_meson_reduce(MesonArgs A, int m0, int nmom_all, double2* __restrict__ out) {
+  const int t = A.t0 + (int)blockIdx.x, q = (int)(blockIdx.y * blockDim.x + threadIdx.x);
+  if (q >= A.nmom * 16) return;
+  const int m = q >> 4, n = q & 15;
+  const double2* p = A.part + (size_t)blockIdx.x * A.nchunk * A.nmom * 16 + q;
+  double2 s = make_double2(0, 0);
+  for (int c = 0; c < A.nchunk; ++c) {
+    const double2 z = p[(size_t)c * A.nmom * 16];
+    s.x += z.x;
+    s.y += z.y;
+  }
+  const int teff = (t - A.g.org[3] % A.g.L[3] + A.g.L[3]) % A.g.L[3];
+  out[((size_t)n * nmom_all + m0 + m) * A.g.L[3] + teff] = s;
 }
 
 ProjGeom proj_geom(const int dims[4], const int origin[4]) {
@@ -193,24 +279,79 @@ ProjGeom proj_geom(const int dims[4], const int origin[4]) {
     CMX_REQUIRE(g.org[m] >= 0 && g.org[m] < dims[m], CMX_ERR_ARG, "meson_2pt: origin outside the lattice");
   }
   g.Vh = g.V / 2;
-  CMX_REQUIRE(g.V <= (long)INT32_MAX * MESON_SITES, CMX_ERR_ARG, "meson_2pt: lattice too large for one grid");
+  CMX_REQUIRE(g.V <= (long)INT32_MAX * 8, CMX_ERR_ARG, "meson_2pt: lattice too large for one grid");
   return g;
 }
 
-void launch_sites(long nsites, const double2* s1, const double2* s2, const Term* terms, double2* c, long cstride,
-                  long coff, hipStream_t st) {
-  hipLaunchKernelGGL(k_meson_sites, dim3((unsigned)((nsites + MESON_SITES - 1) / MESON_SITES)), dim3(16 * MESON_SITES), 0,
-                     st, nsites, s1, s2, terms, c, cstride, coff);
-  CMX_HIP(hipGetLastError());
+// The work-groups of a lattice: about 2048 in all (four rounds of the 512 that are resident), each with at
+// least one group of sites.  They depend on the lattice alone, so the sums have one order whatever scratch
+// they are cut to.
+void meson_chunks(const ProjGeom& g, int& nchunk, int& groups) {
+  const long Vs = (long)g.L[0] * g.L[1] * g.L[2], ng = (Vs + MESON_SITES - 1) / MESON_SITES;
+  const long want = std::max<long>(1, std::min<long>(ng, (2048 + g.L[3] - 1) / g.L[3]));
+  groups = (int)((ng + want - 1) / want);
+  nchunk = (int)((ng + groups - 1) / groups);
 }
 
-// The allocation-free variant's scratch: the correlators of up to MESON_SCRATCH_SITES sites (a pass of whole
-// time slices; 64 MiB) followed by the Gamma-term table (written once per device at set-up, never
-// overwritten).  Host code never uses this name as an address: it uses the per-device pointer that
-// hipGetSymbolAddress returns.
-constexpr long MESON_SCRATCH_SITES = 262144;  // 64^3: the largest spatial volume one pass holds
-constexpr size_t MESON_SCRATCH_CORR = sizeof(double2) * 16 * MESON_SCRATCH_SITES;
-constexpr size_t MESON_SCRATCH_BYTES = MESON_SCRATCH_CORR + sizeof(Term) * 256;
+// Scratch for nm momenta (the phase factors) and the partial correlators of nt slices
+size_t meson_bytes(const ProjGeom& g, int nchunk, int nm, int nt) {
+  return sizeof(double2) * (size_t)nm * ((size_t)(g.L[0] + g.L[1] + g.L[2]) + (size_t)16 * nchunk * nt);
+}
+
+template <int NM> void launch_meson(const MesonArgs& A, int nt, hipStream_t st) {
+  const dim3 grid((unsigned)(nt * A.nchunk), (unsigned)((A.nmom + NM - 1) / NM));
+  if (A.s1 == A.s2)
+    hipLaunchKernelGGL((k_meson<NM, true>), grid, dim3(256), 0, st, A);
+  else
+    hipLaunchKernelGGL((k_meson<NM, false>), grid, dim3(256), 0, st, A);
+}
+
+// All momenta and slices, in passes whose partial correlators fit `bytes` of scratch
+void run_meson(const ProjGeom& g, const double2* s1, const double2* s2, const double2* coef, const int* moms, int nmom,
+               double2* part, size_t bytes, double2* out, hipStream_t st) {
+  MesonArgs A;
+  A.g = g;
+  A.s1 = s1, A.s2 = s2, A.coef = coef;
+  meson_chunks(g, A.nchunk, A.groups);
+  const size_t slice = sizeof(double2) * 16 * (size_t)A.nchunk;  // per momentum
+  // up to 64 momenta per pass (the grid's second index walks them by MESON_NM; fewer where the phases of a
+  // very long lattice would fill the scratch), as many slices as fit
+  const int nx = g.L[0] + g.L[1] + g.L[2];
+  int mstep = std::min(nmom, 64);
+  while (mstep > 1 && meson_bytes(g, A.nchunk, mstep, 1) > bytes) mstep = (mstep + 1) / 2;
+  CMX_REQUIRE(meson_bytes(g, A.nchunk, mstep, 1) <= bytes, CMX_ERR_STATE, "meson_2pt: scratch too small");
+  const size_t table = sizeof(double2) * (size_t)nx * mstep;
+  const int tstep = (int)std::min<size_t>(g.L[3], (bytes - table) / (slice * mstep));
+  A.phase = part, A.part = part + (size_t)nx * mstep;
+  for (int m0 = 0; m0 < nmom; m0 += mstep) {
+    A.moms = moms + 3 * m0;
+    A.nmom = std::min(mstep, nmom - m0);
+    A.t0 = 0;
+    hipLaunchKernelGGL(k_meson_phase, dim3((unsigned)((nx + 255) / 256), (unsigned)A.nmom), dim3(256), 0, st, A);
+    CMX_HIP(hipGetLastError());
+    for (int t0 = 0; t0 < g.L[3]; t0 += tstep) {
+      const int nt = std::min(tstep, g.L[3] - t0);
+      A.t0 = t0;
+      switch (A.nmom) {
+        case 1: launch_meson<1>(A, nt, st); break;
+        case 2: launch_meson<2>(A, nt, st); break;
+        case 3: case 4: launch_meson<4>(A, nt, st); break;
+        default: launch_meson<MESON_NM>(A, nt, st); break;
+      }
+      CMX_HIP(hipGetLastError());
+      hipLaunchKernelGGL(k_meson_reduce, dim3((unsigned)nt, (unsigned)((A.nmom * 16 + 255) / 256)), dim3(256), 0, st, A,
+                         m0, nmom, out);
+      CMX_HIP(hipGetLastError());
+    }
+  }
+}
+
+// The allocation-free variant's scratch: the partial correlators of a pass (64 MiB), followed by the
+// Gamma coefficients (written once per device at set-up, never overwritten).  Host code never uses this
+// name as an address: it uses the per-device pointer that hipGetSymbolAddress returns.
+constexpr long MESON_SCRATCH_SITES = 262144;  // 64^3: the largest spatial volume accepted
+constexpr size_t MESON_SCRATCH_PART = (size_t)64 << 20;
+constexpr size_t MESON_SCRATCH_BYTES = MESON_SCRATCH_PART + sizeof(double2) * 256;
 static __device__ __align__(256) char scratch[MESON_SCRATCH_BYTES];
 
 constexpr int MESON_MAX_DEVICES = 64;
@@ -224,22 +365,20 @@ void meson_2pt(const int dims[4], const double* prop1, const double* prop2, cons
   CMX_REQUIRE(dims && prop1 && prop2 && corr, CMX_ERR_ARG, "meson_2pt: null array");
   CMX_REQUIRE(nmom >= 1 && nmom <= 4096 && moms, CMX_ERR_ARG, "meson_2pt: 1..4096 momenta");
   const ProjGeom g = proj_geom(dims, origin);
-  const std::vector<Term> terms = meson_terms();
+  const std::vector<double2> coefs = meson_coefs();
   const size_t pbytes = sizeof(double) * 288 * (size_t)g.V;
-  DevBuf d1(pbytes), d2(pbytes), dc(sizeof(double2) * 16 * (size_t)g.V), dt(sizeof(Term) * terms.size()),
+  const bool same = prop2 == prop1;
+  int nchunk, groups;
+  meson_chunks(g, nchunk, groups);
+  const size_t least = meson_bytes(g, nchunk, 1, 1), whole = meson_bytes(g, nchunk, std::min(nmom, 64), g.L[3]);
+  DevBuf d1(pbytes), d2(same ? 0 : pbytes), dp(std::max(least, std::min(whole, MESON_SCRATCH_PART))), dt(sizeof(double2) * coefs.size()),
       dm(sizeof(int) * 3 * (size_t)nmom), dout(sizeof(double2) * 16 * (size_t)nmom * g.L[3]);
   CMX_HIP(hipMemcpy(d1.p, prop1, pbytes, hipMemcpyHostToDevice));
-  if (prop2 == prop1)
-    CMX_HIP(hipMemcpy(d2.p, d1.p, pbytes, hipMemcpyDeviceToDevice));
-  else
-    CMX_HIP(hipMemcpy(d2.p, prop2, pbytes, hipMemcpyHostToDevice));
-  CMX_HIP(hipMemcpy(dt.p, terms.data(), dt.bytes, hipMemcpyHostToDevice));
+  if (!same) CMX_HIP(hipMemcpy(d2.p, prop2, pbytes, hipMemcpyHostToDevice));
+  CMX_HIP(hipMemcpy(dt.p, coefs.data(), dt.bytes, hipMemcpyHostToDevice));
   CMX_HIP(hipMemcpy(dm.p, moms, dm.bytes, hipMemcpyHostToDevice));
-  launch_sites(g.V, d1.as<double2>(), d2.as<double2>(), dt.as<Term>(), dc.as<double2>(), g.V, 0, 0);
-  const CorrIndex ci{0, g.V, g.Vh, 0};
-  hipLaunchKernelGGL(k_meson_project, dim3(g.L[3], nmom), dim3(256), 0, 0, g, ci, dc.as<double2>(), dm.as<int>(), nmom,
-                     dout.as<double2>());
-  CMX_HIP(hipGetLastError());
+  run_meson(g, d1.as<double2>(), same ? d1.as<double2>() : d2.as<double2>(), dt.as<double2>(), dm.as<int>(), nmom,
+            dp.as<double2>(), dp.bytes, dout.as<double2>(), 0);
   CMX_HIP(hipMemcpy(corr, dout.p, dout.bytes, hipMemcpyDeviceToHost));
 }
 
@@ -252,8 +391,8 @@ void meson_scratch_setup() {
   void* ptr = nullptr;
   CMX_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
   CMX_REQUIRE(ptr != nullptr, CMX_ERR_HIP, "meson_2pt_noalloc: no device address for the scratch array");
-  const std::vector<Term> terms = meson_terms();
-  CMX_HIP(hipMemcpy(static_cast<char*>(ptr) + MESON_SCRATCH_CORR, terms.data(), sizeof(Term) * terms.size(),
+  const std::vector<double2> coefs = meson_coefs();
+  CMX_HIP(hipMemcpy(static_cast<char*>(ptr) + MESON_SCRATCH_PART, coefs.data(), sizeof(double2) * coefs.size(),
                     hipMemcpyHostToDevice));
   g_scratch_ptr[dev] = ptr;
 }
@@ -270,25 +409,9 @@ void meson_2pt_noalloc(const int dims[4], const double* prop1, const double* pro
   int dev = 0;
   CMX_HIP(hipGetDevice(&dev));
   char* base = static_cast<char*>(g_scratch_ptr[dev]);
-  double2* c = reinterpret_cast<double2*>(base);
-  const Term* terms = reinterpret_cast<const Term*>(base + MESON_SCRATCH_CORR);
-  const double2* s1 = reinterpret_cast<const double2*>(prop1);
-  const double2* s2 = reinterpret_cast<const double2*>(prop2);
-  // passes of T whole time slices; the slice range [t0, t0 + T) is two contiguous site ranges, one per
-  // checkerboard, stored one after the other in the scratch
-  const int T = (int)std::min<long>(g.L[3], MESON_SCRATCH_SITES / Vs);
-  for (int t0 = 0; t0 < g.L[3]; t0 += T) {
-    const int nt = std::min(T, g.L[3] - t0);
-    const long half = Vs * nt / 2, lex0 = Vs * t0 / 2;
-    for (int cb = 0; cb < 2; ++cb) {
-      const size_t first = (size_t)(cb * g.Vh + lex0) * 144;
-      launch_sites(half, s1 + first, s2 + first, terms, c, Vs * nt, cb * half, stream);
-    }
-    const CorrIndex ci{t0, Vs * nt, half, lex0};
-    hipLaunchKernelGGL(k_meson_project, dim3(nt, nmom), dim3(256), 0, stream, g, ci, c, moms, nmom,
-                       reinterpret_cast<double2*>(corr));
-    CMX_HIP(hipGetLastError());
-  }
+  run_meson(g, reinterpret_cast<const double2*>(prop1), reinterpret_cast<const double2*>(prop2),
+            reinterpret_cast<const double2*>(base + MESON_SCRATCH_PART), moms, nmom, reinterpret_cast<double2*>(base),
+            MESON_SCRATCH_PART, reinterpret_cast<double2*>(corr), stream);
 }
 
 }  // namespace cmx
