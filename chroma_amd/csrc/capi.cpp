@@ -632,7 +632,8 @@ int cmx_op_get_hop_config(cmx_op h, int prec, int cfg[6]) {
     const cmx::HopConfig& c = op.hcfg[prec][which];
     // the kernel actually admitted for this operator (the plane-grid kernel needs 12-real links,
     // real boundary phases and a field below 2 GiB; otherwise the site-linear kernel runs)
-    cfg[0] = c.block, cfg[1] = c.tiled, cfg[2] = c.zb, cfg[3] = c.prefetch, cfg[4] = op.hop_base(prec, which).fast;
+    cfg[0] = c.block, cfg[1] = c.tiled, cfg[2] = c.zb, cfg[3] = c.prefetch;
+    cfg[4] = op.hop_base(prec, which).fast & 3;  // the direction-split kernel (small lattices) shows as plane-grid
   });
 }
 

@@ -332,6 +332,12 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
   return (b & 7) * per + (b >> 3);
 }
 
+// The same for any n: XCD k owns n/8 (+1 for the first n mod 8 XCDs) consecutive logical work-groups.
+__device__ __forceinline__ int xcd_range(int b, int n) {
+  const int k = b & 7, q = n >> 3, r = n & 7;
+  return k * q + (k < r ? k : r) + (b >> 3);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Batched launches: one grid covers the work-groups of several problems (solves on different
 // lattices, or several solves on one).  Work-group b runs work-group map[b].y (of map[b].z) of
@@ -388,14 +394,18 @@ struct HopLaunch {
                      // loads of data read once per launch (links, clover, the xpay input) carry the
                      // non-temporal hint
   float inv_lxh;     // 1 / (Lx/2), for the fast kernel's plane decomposition
+  float inv_ly, inv_lz;  // 1 / Ly, 1 / Lz (direction-split kernel)
   float sgn[4][2];   // real det(U) phase per direction: [bulk | last slice]
 };
 
 constexpr int HOP_FAST_STREAM = 2;
+constexpr int HOP_SPLIT = 4;  // with bit 0: the direction-split kernel of hop_split.h (64 sites per work-group)
 // Launch-shape choice for the hopping kernels of one lattice and precision
 struct HopConfig {
   int block = 256, tiled = 0, zb = 1, prefetch = 0, fast = 1;
 };
+// The shape of an operator that has not been tuned: see the definition in op.cpp
+HopConfig hop_default_config(const Geom& g, int prec, bool clover, int which);
 // Fills the shape fields of h from c, falling back to the linear order when the lattice does not
 // admit the tiling (returns the number of work-groups)
 int hop_apply_config(HopLaunch& h, const HopConfig& c);

@@ -1,8 +1,12 @@
 // Hopping-term kernels instantiated for FP16 storage (kernel template in hop_kernel.h).
-#include "hop_fast.h"
+#include "hop_split.h"
 
 namespace cmx {
 void launch_hop_p16(const HopLaunch& h, hipStream_t s, const BatchGrid* bg) {
+  if (h.fast & HOP_SPLIT) {
+    launch_hop_split_t<P16>(h, s, bg);
+    return;
+  }
   if (h.fast & 1) {
     launch_hop_fast_t<P16>(h, s, bg);
     return;

@@ -31,8 +31,48 @@ void launch_hop(const HopLaunch& h, hipStream_t s, const BatchGrid* bg) {
   }
 }
 int hop_num_blocks(const HopLaunch& h) {
+  if (h.fast & HOP_SPLIT) return (h.g.Vh + 63) / 64;
   if (h.fast & 1) return ((h.g.Lxh * h.g.L[1] + h.block - 1) / h.block) * h.g.L[2] * h.g.L[3];
   return (h.g.Vh + h.block - 1) / h.block;
+}
+
+// The launch shape before any tuning (which: 0 the EO operator's kernels, 1 the plain hopping term).
+// The direction-split kernel (hop_split.h) where a wave per 64 sites leaves the chip waiting on latency: at
+// FP64 and FP32 storage up to 340 MB per launch, at FP16 up to 40000 sites.  EO clover operator, us, split
+// against the best plane-grid shape: FP64 8^3x16 10.6 / 15.3, 12^3x24 17.6 / 24.0, 20^3x40 102 / 120,
+// 24^3x48 (605 MB) 267 / 248; FP32 8^3x16 8.7 / 14.0, 16^3x32 21.2 / 22.7, 24^3x48 (303 MB) 107 / 116;
+// FP16 8^3x16 9.5 / 14.5, 12^3x24 12.4 / 18.3, 16^4 (32768 sites) 13.3 / 13.4, 16^3x32 (65536) 18.2 / 16.1;
+// the plain FP16 hop stays on the plane-grid kernel, whose arithmetic the multi-source hop shares.
+// Else the plane-grid kernel: one wave per work-group where an xy plane is a multiple of 64 sites, else the
+// block that idles the fewest lanes of it (the larger of equals); XCD slabs in blocks of 8 z planes where
+// the lattice admits them; read-once loads streamed once a launch's data no longer fits the 256 MB Infinity
+// Cache, below which streaming throws away what the next launch re-reads (EO clover operator, us, streamed
+// against not: 24^3x48 FP16 67 / 55, 151 MB per launch; 32^3x64 FP16 182 / 212, 478 MB; the hop alone:
+// 24^3x48 FP64 81 / 87, 382 MB).
+HopConfig hop_default_config(const Geom& g, int prec, bool clover, int which) {
+  HopConfig c;
+  const int P = g.Lxh * g.L[1];
+  auto lanes = [&](int b) { return (P + b - 1) / b * b; };
+  c.block = 64;
+  if (P % 64 != 0)
+    for (int b : {128, 256})
+      if (lanes(b) <= lanes(c.block)) c.block = b;
+  c.tiled = g.L[3] % 8 == 0 ? 1 : 0;
+  c.zb = 1;
+  for (int zb : {2, 4, 8})
+    if (g.L[2] % zb == 0) c.zb = zb;
+  c.prefetch = 0;
+  const double s = prec == P16 ? 2 : (prec == P32 ? 4 : 8);
+  const double bytes = (which == 1 ? 144.0 : (clover ? 228.0 : 156.0)) * s * g.Vh;
+  if (prec == P16 ? which == 0 && g.Vh <= 40000 : bytes <= 340e6) {
+    c.block = 64;
+    c.tiled = 0;
+    c.zb = 1;
+    c.fast = 1 | HOP_SPLIT;
+    return c;
+  }
+  c.fast = 1 | (bytes > 310e6 ? HOP_FAST_STREAM : 0);
+  return c;
 }
 
 int hop_apply_config(HopLaunch& h, const HopConfig& c) {
@@ -53,6 +93,15 @@ int hop_apply_config(HopLaunch& h, const HopConfig& c) {
                      h.g.L[2] * h.g.L[3] < 65536 && site_bytes * (size_t)h.g.Vh < ((size_t)1 << 31);
   h.fast = plane ? c.fast : (c.fast & HOP_FAST_STREAM);  // the stream bit applies to both kernels
   h.inv_lxh = 1.0f / (float)h.g.Lxh;
+  h.inv_ly = 1.0f / (float)h.g.L[1];
+  h.inv_lz = 1.0f / (float)h.g.L[2];
+  if ((h.fast & HOP_SPLIT) && h.g.Vh >= (1 << 24)) h.fast &= ~HOP_SPLIT;
+  if (h.fast & HOP_SPLIT) {  // site-linear, 64 sites per work-group, no cache hints
+    h.fast &= ~HOP_FAST_STREAM;
+    h.block = 64;
+    h.prefetch = 0;
+    return hop_num_blocks(h);
+  }
   if (h.fast & 1) {  // the plane-grid kernel tiles whole planes: any block size, Lt % 8 and Lz % zb only
     if (c.tiled && h.g.L[3] % 8 == 0 && c.zb > 0 && h.g.L[2] % c.zb == 0) {
       h.tiled = 1;
@@ -186,6 +235,8 @@ Op* make_op(std::shared_ptr<GaugeData> gd, const cmx_op_params& p) {
   // FP64 links as 12 reals (third row rebuilt in FP64 on use) when they are SU(3) up to a boundary
   // phase to rounding, which makes the rebuilt row as exact as a stored one
   op->recon[P64] = gd->su3_dev <= 1e-14 ? 12 : 18;
+  for (int prec : {P64, P32, P16})
+    for (int which : {0, 1}) op->hcfg[prec][which] = hop_default_config(op->g, prec, op->clover(), which);
   if (gd->su3_dev > 1e-6)
     CMX_REQUIRE(p.sloppy_recon == 18 && p.sloppy_prec == CMX_SINGLE, CMX_ERR_ARG,
                 "op_create: links are not SU(3) up to a per-direction boundary phase (deviation " +
@@ -578,6 +629,7 @@ void Op::autotune() {
             for (int zb : {1, 4, 8}) cands.push_back(HopConfig{block, 1, zb, 0, fm});
           }
         }
+        if (block == 64) cands.push_back(HopConfig{64, 0, 1, 0, 1 | HOP_SPLIT});
         for (int pf : {0, 1}) {  // site-linear kernel; streamed loads on the single-buffered path
           if (pf && prec == P64) continue;
           for (int st : {0, HOP_FAST_STREAM}) {
@@ -593,7 +645,9 @@ void Op::autotune() {
       for (const HopConfig& c : cands) {
         HopLaunch probe = hop_base(prec, which);
         hop_apply_config(probe, c);
-        if ((c.tiled && !probe.tiled) || ((c.fast & 1) && !(probe.fast & 1))) continue;  // not admitted here
+        if ((c.tiled && !probe.tiled) || ((c.fast & 1) && !(probe.fast & 1)) ||
+            ((c.fast & HOP_SPLIT) && !(probe.fast & HOP_SPLIT)))
+          continue;  // not admitted here
         hcfg[prec][which] = c;
         auto run = [&]() {
           if (which == 0)

@@ -934,10 +934,25 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     for (Op* o : ops) o->hcfg[ps][0] = bestc;
     CMX_HIP(hipStreamSynchronize(s0));
   }
+  if (!bp.tune) {
+    // one kernel covers the batch: operators whose own shapes (which depend on their volumes) select
+    // different ones share the first operator's work-group size, without streamed loads
+    bool same = true;
+    for (Op* o : ops)
+      same = same && o->hcfg[ps][0].block == ops[0]->hcfg[ps][0].block && o->hcfg[ps][0].fast == ops[0]->hcfg[ps][0].fast &&
+             o->hcfg[ps][0].prefetch == ops[0]->hcfg[ps][0].prefetch;
+    if (!same)
+      for (Op* o : ops) {
+        HopConfig& c = o->hcfg[ps][0];
+        c.block = saved[0].block;
+        c.fast = saved[0].fast & ~(HOP_FAST_STREAM | HOP_SPLIT);
+        c.prefetch = saved[0].prefetch;
+      }
+  }
   {
     const HopLaunch h = ops[0]->hop_base(ps);
     bres.hop_block = h.block;
-    bres.hop_fast = h.fast;
+    bres.hop_fast = h.fast & 3;
   }
 
   // passes: every problem, then (true-residual mode) the problems whose FP64 residual is above target,
