@@ -43,10 +43,29 @@ void record_fin(Recorder& r, const FinLaunch& f) { r.recs.push_back(make_rec(REC
 void BatchPlan::build(const std::vector<Recorder>& recs) {
   st_.clear();
   CMX_REQUIRE(!recs.empty(), CMX_ERR_ARG, "batch: no problems");
+  // problems whose launches select the same kernels share batched grids; others get their own
+  std::vector<std::vector<Recorder>> groups;
+  auto alike = [](const Recorder& a, const Recorder& b) {
+    if (a.recs.size() != b.recs.size()) return false;
+    for (size_t j = 0; j < a.recs.size(); ++j)
+      if (a.recs[j].kind != b.recs[j].kind || std::memcmp(a.recs[j].key, b.recs[j].key, sizeof(a.recs[j].key)) != 0)
+        return false;
+    return true;
+  };
+  for (const Recorder& r : recs) {
+    CMX_REQUIRE(r.recs.size() == recs[0].recs.size(), CMX_ERR_ARG,
+                "batch: the problems' kernel sequences differ in length");
+    size_t k = 0;
+    while (k < groups.size() && !alike(groups[k][0], r)) ++k;
+    if (k == groups.size()) groups.emplace_back();
+    groups[k].push_back(r);
+  }
+  for (const auto& g : groups) add_group(g);
+}
+
+void BatchPlan::add_group(const std::vector<Recorder>& recs) {
   const size_t ns = recs[0].recs.size();
   const int np = (int)recs.size();
-  for (const Recorder& r : recs)
-    CMX_REQUIRE(r.recs.size() == ns, CMX_ERR_ARG, "batch: the problems' kernel sequences differ in length");
   for (size_t j = 0; j < ns; ++j) {
     const LaunchRec& r0 = recs[0].recs[j];
     Stage s;

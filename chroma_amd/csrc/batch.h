@@ -44,7 +44,8 @@ struct RecordScope {
 // The batched stages of one recorded sequence
 class BatchPlan {
  public:
-  // recs[p] is problem p's recording; every recording must hold the same kernels in the same order
+  // recs[p] is problem p's recording, all of one length; problems whose recordings select the same kernels
+  // are batched together, each such group into stages of its own
   void build(const std::vector<Recorder>& recs);
   // the same kernel sequence with new launch records (other fields, same kernels and work-group counts):
   // the records are copied to the device on stream s through pinned staging, the work-group maps kept;
@@ -55,6 +56,7 @@ class BatchPlan {
   long blocks() const;  // work-groups over all stages
 
  private:
+  void add_group(const std::vector<Recorder>& recs);
   struct Stage {
     int kind = 0, opc = 0;
     int prec[4] = {0, 0, 0, 0};

@@ -662,6 +662,7 @@ int cmx_op_set_hop_config(cmx_op h, int prec, const int cfg[6]) {
                 "set_hop_config: bad tiling / prefetch flags");
     CMX_REQUIRE(cfg[5] >= 0 && cfg[5] <= 2, CMX_ERR_ARG, "set_hop_config: target must be 0, 1 or 2");
     const cmx::HopConfig c{cfg[0], cfg[1], cfg[2], prec == cmx::P64 ? 0 : cfg[3], cfg[4]};
+    op.hop_shape_set[prec] = true;
     if (cfg[5] != 2) op.hcfg[prec][0] = c;
     if (cfg[5] != 1) op.hcfg[prec][1] = c;
   });

@@ -301,6 +301,7 @@ Op* clone_op(Op& o, int prec) {
   c->fact = o.fact;
   std::memcpy(c->recon, o.recon, sizeof(o.recon));
   std::memcpy(c->hcfg, o.hcfg, sizeof(o.hcfg));
+  std::memcpy(c->hop_shape_set, o.hop_shape_set, sizeof(o.hop_shape_set));
   c->multi_group = o.multi_group;
   for (int p_ = 0; p_ < 3; ++p_) {
     for (int q = 0; q < 2; ++q) c->gauge[p_][q].alias(o.gauge[p_][q]);
@@ -599,7 +600,8 @@ void Op::autotune() {
   hipEvent_t e0, e1;
   CMX_HIP(hipEventCreate(&e0));
   CMX_HIP(hipEventCreate(&e1));
-  for (int prec : precs)
+  for (int prec : precs) {
+    hop_shape_set[prec] = true;
     for (int which = 0; which < 2; ++which) {
       TuneKey key;
       std::memset(&key, 0, sizeof(key));
@@ -685,6 +687,7 @@ void Op::autotune() {
       std::lock_guard<std::mutex> lk(tune_mutex());
       tune_cache()[key] = hcfg[prec][which];
     }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   CMX_HIP(hipGetLastError());

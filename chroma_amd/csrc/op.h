@@ -85,6 +85,7 @@ struct Op {
   // hopping-kernel launch shape per precision: [0] the EO operator's fused kernels, [1] the plain
   // hopping term (tuned separately by autotune(): their best shapes differ)
   HopConfig hcfg[3][2];
+  bool hop_shape_set[3] = {false, false, false};  // hcfg[prec] was set or tuned
   int multi_group = 0;  // sources per multi-source hop kernel; 0: timed at first use
   // per precision: links (per parity) and the clover blocks used by the EO operator
   DevBuf gauge[3][2];

@@ -935,19 +935,17 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     CMX_HIP(hipStreamSynchronize(s0));
   }
   if (!bp.tune) {
-    // one kernel covers the batch: operators whose own shapes (which depend on their volumes) select
-    // different ones share the first operator's work-group size, without streamed loads
-    bool same = true;
-    for (Op* o : ops)
-      same = same && o->hcfg[ps][0].block == ops[0]->hcfg[ps][0].block && o->hcfg[ps][0].fast == ops[0]->hcfg[ps][0].fast &&
-             o->hcfg[ps][0].prefetch == ops[0]->hcfg[ps][0].prefetch;
-    if (!same)
-      for (Op* o : ops) {
-        HopConfig& c = o->hcfg[ps][0];
-        c.block = saved[0].block;
-        c.fast = saved[0].fast & ~(HOP_FAST_STREAM | HOP_SPLIT);
-        c.prefetch = saved[0].prefetch;
-      }
+    // Shapes that depend on the volumes alone may differ (the plan batches each kernel's problems apart);
+    // shapes that were set or tuned must select one kernel for the batch.
+    bool same = true, untouched = true;
+    const HopLaunch h0 = ops[0]->hop_base(ps);
+    for (Op* o : ops) {
+      const HopLaunch h = o->hop_base(ps);
+      same = same && h.fast == h0.fast && h.prefetch == h0.prefetch && h.block == h0.block;
+      untouched = untouched && !o->hop_shape_set[ps];
+    }
+    CMX_REQUIRE(same || untouched, CMX_ERR_ARG,
+                "batch: the operators' launch shapes select different kernels (launch shape, precision or epilogue)");
   }
   {
     const HopLaunch h = ops[0]->hop_base(ps);
