@@ -76,7 +76,10 @@ int cmx_init(int device) {
 
 int cmx_finalize(void) {
   return guarded([&] {
-    if (g_init) CMX_HIP(hipDeviceSynchronize());
+    if (g_init) {
+      CMX_HIP(hipDeviceSynchronize());
+      cmx::xfer_release();
+    }
     g_init = false;
   });
 }
@@ -135,7 +138,7 @@ int cmx_op_apply(cmx_op h, double* chi, const double* psi, int isign, int prec) 
     CMX_REQUIRE(isign == 1 || isign == -1, CMX_ERR_ARG, "op_apply: isign must be +1 or -1");
     CMX_REQUIRE(prec >= 0 && prec <= 2, CMX_ERR_ARG, "op_apply: bad precision");
     const int n = op.subset_sites();
-    cmx::Vec in(prec, n), out(prec, n);
+    cmx::ScratchVec in(prec, n), out(prec, n);
     op.pack(psi, n, in);
     op.apply(prec, out.view(), in.view(), isign, nullptr);
     op.unpack(chi, n, out);
@@ -151,7 +154,7 @@ int cmx_dslash_apply(cmx_op h, double* chi, const double* psi, int isign, int cb
     CMX_REQUIRE(cb == 0 || cb == 1, CMX_ERR_ARG, "dslash_apply: cb must be 0 or 1");
     CMX_REQUIRE(prec >= 0 && prec <= 2, CMX_ERR_ARG, "dslash_apply: bad precision");
     const int n = (int)op.Vh;
-    cmx::Vec in(prec, n), out(prec, n);
+    cmx::ScratchVec in(prec, n), out(prec, n);
     op.pack(psi, n, in);
     op.dslash(prec, out.view(), in.view(), isign, cb);
     op.unpack(chi, n, out);
@@ -168,11 +171,11 @@ int cmx_dslash_multi(cmx_op h, int nrhs, double* chi, const double* psi, int isi
     CMX_REQUIRE(prec >= 0 && prec <= 2, CMX_ERR_ARG, "dslash_multi: bad precision");
     const int n = (int)op.Vh;
     const size_t nd = (size_t)24 * n;
-    std::vector<std::unique_ptr<cmx::Vec>> in, out;
+    std::vector<std::unique_ptr<cmx::ScratchVec>> in, out;
     std::vector<cmx::VRef> vi, vo;
     for (int k = 0; k < nrhs; ++k) {
-      in.emplace_back(new cmx::Vec(prec, n));
-      out.emplace_back(new cmx::Vec(prec, n));
+      in.emplace_back(new cmx::ScratchVec(prec, n));
+      out.emplace_back(new cmx::ScratchVec(prec, n));
       op.pack(psi + k * nd, n, *in.back());
       vi.push_back(in.back()->view());
       vo.push_back(out.back()->view());
@@ -191,29 +194,26 @@ int cmx_dslash_deriv(cmx_op h, double* ds_u, const double* chi, const double* ps
     CMX_REQUIRE(isign == 1 || isign == -1, CMX_ERR_ARG, "dslash_deriv: isign must be +1 or -1");
     CMX_REQUIRE(cb >= -1 && cb <= 1, CMX_ERR_ARG, "dslash_deriv: cb must be 0, 1 or -1");
     const long Vh = op.Vh, V = op.V;
-    cmx::Vec a(cmx::P64, (int)Vh), b(cmx::P64, (int)Vh);
-    cmx::DevBuf ds((size_t)4 * 9 * 16 * Vh);
-    std::vector<double> host((size_t)4 * 18 * Vh);
+    cmx::ScratchVec a(cmx::P64, (int)Vh), b(cmx::P64, (int)Vh);
+    cmx::DevScratch ds((size_t)4 * 9 * 16 * Vh);
     std::memset(ds_u, 0, sizeof(double) * 4 * 18 * V);
     for (int c = 0; c < 2; ++c) {
       if (cb >= 0 && c != cb) continue;
       op.pack(chi + (size_t)c * 24 * Vh, (int)Vh, a);
       op.pack(psi + (size_t)(1 - c) * 24 * Vh, (int)Vh, b);
-      cmx::hop_deriv(op.g, c, isign, a.view(), b.view(), ds.p, op.stream);
+      cmx::hop_deriv(op.g, c, isign, a.view(), b.view(), ds.get(), op.stream);
       CMX_HIP(hipGetLastError());
-      CMX_HIP(hipMemcpyAsync(host.data(), ds.p, sizeof(double) * host.size(), hipMemcpyDeviceToHost, op.stream));
-      op.sync();
       for (int mu = 0; mu < 4; ++mu)
-        std::memcpy(ds_u + ((size_t)mu * V + (size_t)c * Vh) * 18, host.data() + (size_t)mu * Vh * 18,
-                    sizeof(double) * 18 * Vh);
+        cmx::device_to_host(ds_u + ((size_t)mu * V + (size_t)c * Vh) * 18, ds.as<double>() + (size_t)mu * Vh * 18,
+                            sizeof(double) * 18 * Vh, op.stream);
     }
   });
 }
 
 namespace {
 // ds (device, [4][V][9] double2) -> host ds_u [4][V][18] doubles
-void download_force(cmx::Op& op, const cmx::DevBuf& ds, double* ds_u) {
-  CMX_HIP(hipMemcpyAsync(ds_u, ds.p, sizeof(double) * 4 * 18 * op.V, hipMemcpyDeviceToHost, op.stream));
+void download_force(cmx::Op& op, const cmx::DevScratch& ds, double* ds_u) {
+  cmx::device_to_host(ds_u, ds.get(), sizeof(double) * 4 * 18 * op.V, op.stream);
   op.sync();
 }
 }  // namespace
@@ -227,14 +227,14 @@ int cmx_clover_deriv(cmx_op h, double* ds_u, const double* chi, const double* ps
     CMX_REQUIRE(isign == 1 || isign == -1, CMX_ERR_ARG, "clover_deriv: isign must be +1 or -1");
     CMX_REQUIRE(cb >= -1 && cb <= 1, CMX_ERR_ARG, "clover_deriv: cb must be 0, 1 or -1");
     const long Vh = op.Vh;
-    cmx::Vec a(cmx::P64, (int)Vh), b(cmx::P64, (int)Vh);
-    cmx::DevBuf ds((size_t)4 * 9 * 16 * op.V);
-    CMX_HIP(hipMemsetAsync(ds.p, 0, ds.bytes, op.stream));
+    cmx::ScratchVec a(cmx::P64, (int)Vh), b(cmx::P64, (int)Vh);
+    cmx::DevScratch ds((size_t)4 * 9 * 16 * op.V), lam((size_t)6 * 9 * 16 * Vh);
+    CMX_HIP(hipMemsetAsync(ds.get(), 0, ds.bytes(), op.stream));
     for (int c = 0; c < 2; ++c) {
       if (cb >= 0 && c != cb) continue;
       op.pack(chi + (size_t)c * 24 * Vh, (int)Vh, a);
       op.pack(psi + (size_t)c * 24 * Vh, (int)Vh, b);
-      cmx::clover_force(op, false, c, a.view(), b.view(), 1.0, ds.p);
+      cmx::clover_force(op, false, c, a.view(), b.view(), 1.0, ds.get(), lam.get());
     }
     download_force(op, ds, ds_u);
   });
@@ -246,9 +246,9 @@ int cmx_clover_deriv_trln(cmx_op h, double* ds_u) {
     cmx::Op& op = O(h);
     CMX_REQUIRE(op.clover(), CMX_ERR_ARG, "clover_deriv_trln: not a clover operator");
     CMX_REQUIRE(ds_u, CMX_ERR_ARG, "clover_deriv_trln: null array");
-    cmx::DevBuf ds((size_t)4 * 9 * 16 * op.V);
-    CMX_HIP(hipMemsetAsync(ds.p, 0, ds.bytes, op.stream));
-    cmx::clover_force(op, true, 0, cmx::VRef{}, cmx::VRef{}, 1.0, ds.p);
+    cmx::DevScratch ds((size_t)4 * 9 * 16 * op.V), lam((size_t)6 * 9 * 16 * op.Vh);
+    CMX_HIP(hipMemsetAsync(ds.get(), 0, ds.bytes(), op.stream));
+    cmx::clover_force(op, true, 0, cmx::VRef{}, cmx::VRef{}, 1.0, ds.get(), lam.get());
     download_force(op, ds, ds_u);
   });
 }
@@ -261,13 +261,13 @@ int cmx_op_deriv(cmx_op h, double* ds_u, const double* chi, const double* psi, i
     CMX_REQUIRE(ds_u && chi && psi, CMX_ERR_ARG, "op_deriv: null array");
     CMX_REQUIRE(isign == 1 || isign == -1, CMX_ERR_ARG, "op_deriv: isign must be +1 or -1");
     const int Vh = (int)op.Vh;
-    cmx::Vec co(cmx::P64, Vh), po(cmx::P64, Vh), t2(cmx::P64, Vh), t3(cmx::P64, Vh);
-    cmx::DevBuf ds((size_t)4 * 9 * 16 * op.V), dcb((size_t)4 * 9 * 16 * Vh);
-    CMX_HIP(hipMemsetAsync(ds.p, 0, ds.bytes, op.stream));
+    cmx::ScratchVec co(cmx::P64, Vh), po(cmx::P64, Vh), t2(cmx::P64, Vh), t3(cmx::P64, Vh);
+    cmx::DevScratch ds((size_t)4 * 9 * 16 * op.V), dcb((size_t)4 * 9 * 16 * Vh), lam((size_t)6 * 9 * 16 * Vh);
+    CMX_HIP(hipMemsetAsync(ds.get(), 0, ds.bytes(), op.stream));
     op.pack(chi, Vh, co);
     op.pack(psi, Vh, po);
     // t = A_ee^-1 D_eo(sign) v, the first kernel of the even-odd operator at FP64
-    auto ainv_d = [&](cmx::Vec& t, const cmx::Vec& v, int sign) {
+    auto ainv_d = [&](const cmx::Vec& t, const cmx::Vec& v, int sign) {
       cmx::HopLaunch hh = op.hop_base(cmx::P64);
       hh.isign = sign;
       hh.cb = 0;
@@ -287,14 +287,14 @@ int cmx_op_deriv(cmx_op h, double* ds_u, const double* chi, const double* psi, i
     //   ds -= -1/2 D.deriv(chi, tmp2, cb 1)     = -1/4 D.deriv(chi, t2, cb 1)
     //   ds += clov.deriv(tmp3, tmp2, cb 0)      = +1/4 clov.deriv(t3, t2, cb 0)
     //   ds -= -1/2 D.deriv(tmp3, psi, cb 0)     = -1/4 D.deriv(t3, psi, cb 0)
-    cmx::clover_force(op, false, 1, co.view(), po.view(), 1.0, ds.p);
+    cmx::clover_force(op, false, 1, co.view(), po.view(), 1.0, ds.get(), lam.get());
     ainv_d(t2, po, isign);
-    cmx::hop_deriv(op.g, 1, isign, co.view(), t2.view(), dcb.p, op.stream);
-    cmx::force_axpy(op, 1, -0.25, dcb.p, ds.p);
+    cmx::hop_deriv(op.g, 1, isign, co.view(), t2.view(), dcb.get(), op.stream);
+    cmx::force_axpy(op, 1, -0.25, dcb.get(), ds.get());
     ainv_d(t3, co, -isign);
-    cmx::clover_force(op, false, 0, t3.view(), t2.view(), 0.25, ds.p);
-    cmx::hop_deriv(op.g, 0, isign, t3.view(), po.view(), dcb.p, op.stream);
-    cmx::force_axpy(op, 0, -0.25, dcb.p, ds.p);
+    cmx::clover_force(op, false, 0, t3.view(), t2.view(), 0.25, ds.get(), lam.get());
+    cmx::hop_deriv(op.g, 0, isign, t3.view(), po.view(), dcb.get(), op.stream);
+    cmx::force_axpy(op, 0, -0.25, dcb.get(), ds.get());
     download_force(op, ds, ds_u);
   });
 }
@@ -302,14 +302,22 @@ int cmx_op_deriv(cmx_op h, double* ds_u, const double* chi, const double* psi, i
 int cmx_gauge_stout_smear(const int dims[4], double* links, int nstep, double rho) {
   return guarded([&] {
     require_init();
-    cmx::stout_smear(dims, links, nstep, rho, 15);
+    cmx::stout_smear(dims, links, links, nstep, rho, 15);
   });
 }
 
 int cmx_gauge_stout_smear_dirs(const int dims[4], double* links, int nstep, double rho, int smear_dirs) {
   return guarded([&] {
     require_init();
-    cmx::stout_smear(dims, links, nstep, rho, smear_dirs);
+    cmx::stout_smear(dims, links, links, nstep, rho, smear_dirs);
+  });
+}
+
+int cmx_gauge_stout_smear_to(const int dims[4], const double* links, double* out, int nstep, double rho,
+                             int smear_dirs) {
+  return guarded([&] {
+    require_init();
+    cmx::stout_smear(dims, links, out, nstep, rho, smear_dirs);
   });
 }
 
@@ -337,7 +345,7 @@ int cmx_op_eo_piece(cmx_op h, int which, double* chi, const double* psi, int isi
     CMX_REQUIRE(chi && psi, CMX_ERR_ARG, "op_eo_piece: null array");
     CMX_REQUIRE(which >= 0 && which <= 5, CMX_ERR_ARG, "op_eo_piece: bad block");
     const int Vh = (int)op.Vh;
-    cmx::Vec in(cmx::P64, 2 * Vh), out(cmx::P64, 2 * Vh);
+    cmx::ScratchVec in(cmx::P64, 2 * Vh), out(cmx::P64, 2 * Vh);
     op.pack(psi, 2 * Vh, in);
     cmx::HopLaunch h0 = op.hop_base(cmx::P64);
     h0.isign = isign;
@@ -356,8 +364,8 @@ int cmx_op_eo_piece(cmx_op h, int which, double* chi, const double* psi, int isi
     };
     // hop with a zero input gives b*D*0 = 0, so the "local" blocks below are the EPI_XPAY / EPI_CLOV_XPAY
     // epilogues with b = 0 applied to a zero neighbour field
-    cmx::Vec zero(cmx::P64, 2 * Vh);
-    op.blas(cmx::B_ZERO, {&zero});
+    cmx::ScratchVec zero(cmx::P64, 2 * Vh);
+    op.blas(cmx::B_ZERO, {&zero.v});
     auto local = [&](int cb, const void* clov, double a) {
       cmx::HopLaunch hh = h0;
       hh.cb = cb;
@@ -385,11 +393,9 @@ int cmx_op_eo_piece(cmx_op h, int which, double* chi, const double* psi, int isi
     }
     CMX_HIP(hipGetLastError());
     // write back only the target checkerboard(s)
-    std::unique_ptr<double[]> full(new double[(size_t)48 * Vh]);
-    op.unpack(full.get(), 2 * Vh, out);
     const int lo = (which <= 2) ? 0 : (which == 5 ? 0 : Vh);
     const int hi = (which <= 2) ? Vh : 2 * Vh;
-    std::memcpy(chi + (size_t)24 * lo, full.get() + (size_t)24 * lo, sizeof(double) * 24 * (hi - lo));
+    op.unpack(chi + (size_t)24 * lo, hi - lo, out, lo);
   });
 }
 
@@ -400,13 +406,11 @@ int cmx_clover_download(cmx_op h, int which, double* tri) {
     CMX_REQUIRE(op.clover(), CMX_ERR_ARG, "clover_download: not a clover operator");
     CMX_REQUIRE(tri && (which == 0 || which == 1), CMX_ERR_ARG, "clover_download: bad argument");
     const int Vh = (int)op.Vh;
-    cmx::DevBuf d((size_t)72 * sizeof(double) * Vh);
+    cmx::DevScratch d((size_t)72 * sizeof(double) * Vh);
     auto grab = [&](const cmx::DevBuf& src, int cb) {
       cmx::clover_unpack(Vh, src.as<double2>(), d.as<double>(), op.stream);
       CMX_HIP(hipGetLastError());
-      CMX_HIP(hipMemcpyAsync(tri + (size_t)72 * cb * Vh, d.p, (size_t)72 * sizeof(double) * Vh, hipMemcpyDeviceToHost,
-                             op.stream));
-      op.sync();
+      cmx::device_to_host(tri + (size_t)72 * cb * Vh, d.get(), (size_t)72 * sizeof(double) * Vh, op.stream);
     };
     if (which == 0) {
       grab(op.clov64_even, 0);
@@ -448,8 +452,7 @@ int cmx_clover_pack_quda(cmx_op h, int which, int cb, double* out) {
       const cmx::DevBuf& src = which == 1 ? op.clovinv_even[cmx::P64] : (cb == 0 ? op.clov64_even : op.clov_odd[cmx::P64]);
       cmx::clover_unpack(Vh, src.as<double2>(), d.as<double>(), op.stream);
     }
-    CMX_HIP(hipMemcpyAsync(tri.get(), d.p, (size_t)72 * sizeof(double) * Vh, hipMemcpyDeviceToHost, op.stream));
-    op.sync();
+    cmx::device_to_host(tri.get(), d.p, (size_t)72 * sizeof(double) * Vh, op.stream);
     // QUDAPackedClovSite: diag1[6], offDiag1[15][2], diag2[6], offDiag2[15][2]; the lower triangle
     // column by column (packForQUDA, clover_term_qdp_w.h:2185-2222), written at the full-lattice site
     // index of each site of checkerboard cb (quda_array[rb[cb].siteTable()[ssite]]); the other
@@ -473,25 +476,30 @@ int cmx_clover_pack_quda(cmx_op h, int which, int cb, double* out) {
   });
 }
 
-int cmx_solve(cmx_op h, const cmx_solver_params* p, double* psi, const double* chi, int nrhs, cmx_solver_result* res) {
+static int solve_all(cmx_op h, const cmx_solver_params* p, double* psi, const double* chi, int nrhs, bool mdagm,
+                     bool from_zero, cmx_solver_result* res) {
   return guarded([&] {
     require_init();
     cmx::Op& op = O(h);
-    CMX_REQUIRE(p && psi && chi && res && nrhs >= 1, CMX_ERR_ARG, "solve: bad argument");
+    CMX_REQUIRE(p && psi && chi && res && nrhs >= 1, CMX_ERR_ARG,
+                mdagm ? "solve_mdagm: bad argument" : "solve: bad argument");
     const long nd = 24L * op.subset_sites();
-    for (int k = 0; k < nrhs; ++k) cmx::solve(op, *p, psi + k * nd, chi + k * nd, false, res[k]);
+    for (int k = 0; k < nrhs; ++k) cmx::solve(op, *p, psi + k * nd, chi + k * nd, mdagm, from_zero, res[k]);
   });
+}
+
+int cmx_solve(cmx_op h, const cmx_solver_params* p, double* psi, const double* chi, int nrhs, cmx_solver_result* res) {
+  return solve_all(h, p, psi, chi, nrhs, false, false, res);
 }
 
 int cmx_solve_mdagm(cmx_op h, const cmx_solver_params* p, double* psi, const double* chi, int nrhs,
                     cmx_solver_result* res) {
-  return guarded([&] {
-    require_init();
-    cmx::Op& op = O(h);
-    CMX_REQUIRE(p && psi && chi && res && nrhs >= 1, CMX_ERR_ARG, "solve_mdagm: bad argument");
-    const long nd = 24L * op.subset_sites();
-    for (int k = 0; k < nrhs; ++k) cmx::solve(op, *p, psi + k * nd, chi + k * nd, true, res[k]);
-  });
+  return solve_all(h, p, psi, chi, nrhs, true, false, res);
+}
+
+int cmx_solve_from_zero(cmx_op h, const cmx_solver_params* p, double* psi, const double* chi, int nrhs, int mdagm,
+                        cmx_solver_result* res) {
+  return solve_all(h, p, psi, chi, nrhs, mdagm != 0, true, res);
 }
 
 int cmx_solve_multishift(cmx_op h, const cmx_solver_params* p, int nshift, const double* shifts, const double* rsd,
@@ -504,9 +512,9 @@ int cmx_solve_multishift(cmx_op h, const cmx_solver_params* p, int nshift, const
   });
 }
 
-int cmx_solve_batch(const cmx_op* hs, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
-                    double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
-                    cmx_batch_result* bres) {
+static int solve_batch_all(const cmx_op* hs, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
+                           double* const* psi, const double* const* chi, int mdagm, bool from_zero,
+                           cmx_solver_result* res, cmx_batch_result* bres) {
   return guarded([&] {
     require_init();
     CMX_REQUIRE(hs && n >= 1 && p && bp && psi && chi && res && bres, CMX_ERR_ARG, "solve_batch: bad argument");
@@ -529,8 +537,20 @@ int cmx_solve_batch(const cmx_op* hs, int n, const cmx_solver_params* p, const c
         ops[i] = &o;
       }
     }
-    cmx::solve_batch(ops, *p, *bp, psi, chi, mdagm != 0, res, *bres);
+    cmx::solve_batch(ops, *p, *bp, psi, chi, mdagm != 0, from_zero, res, *bres);
   });
+}
+
+int cmx_solve_batch(const cmx_op* hs, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
+                    double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
+                    cmx_batch_result* bres) {
+  return solve_batch_all(hs, n, p, bp, psi, chi, mdagm, false, res, bres);
+}
+
+int cmx_solve_batch_from_zero(const cmx_op* hs, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
+                              double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
+                              cmx_batch_result* bres) {
+  return solve_batch_all(hs, n, p, bp, psi, chi, mdagm, true, res, bres);
 }
 
 int cmx_op_time(cmx_op h, int what, int prec, int n, double* ms_per_call) {
@@ -681,7 +701,7 @@ int cmx_layout_roundtrip(cmx_op h, int prec, const double* in, double* out) {
     cmx::Op& op = O(h);
     CMX_REQUIRE(in && out && prec >= 0 && prec <= 2, CMX_ERR_ARG, "layout_roundtrip: bad argument");
     const int n = (int)op.Vh;
-    cmx::Vec v(prec, n);
+    cmx::ScratchVec v(prec, n);
     op.pack(in, n, v);
     op.unpack(out, n, v);
   });

@@ -277,22 +277,21 @@ void launch_loops(Op& op, const double2* Lam, int cb, double scale, double2* ds)
 
 }  // namespace
 
-void clover_force(Op& op, bool trln, int cb, VRef chi, VRef psi, double scale, void* ds_full) {
+void clover_force(Op& op, bool trln, int cb, VRef chi, VRef psi, double scale, void* ds_full, void* lam_) {
   CMX_REQUIRE(op.clover(), CMX_ERR_ARG, "clover force: not a clover operator");
   CMX_REQUIRE(cb == 0 || cb == 1, CMX_ERR_ARG, "clover force: cb must be 0 or 1");
   CMX_REQUIRE(!trln || cb == 0, CMX_ERR_ARG, "clover force: derivTrLn of the inverted even-even term only");
   const ForcePlanes P = force_planes(op.par);
-  DevBuf lam((size_t)6 * 9 * 16 * op.Vh);
+  double2* lam = static_cast<double2*>(lam_);
   const dim3 grid((unsigned)((op.Vh + 255) / 256));
   if (trln)
     hipLaunchKernelGGL(k_force_lambda<true>, grid, dim3(256), 0, op.stream, op.g, P, chi, psi,
-                       op.clovinv_even[P64].as<double2>(), lam.as<double2>());
+                       op.clovinv_even[P64].as<double2>(), lam);
   else
     hipLaunchKernelGGL(k_force_lambda<false>, grid, dim3(256), 0, op.stream, op.g, P, chi, psi, nullptr,
-                       lam.as<double2>());
+                       lam);
   CMX_HIP(hipGetLastError());
-  launch_loops(op, lam.as<double2>(), cb, scale, static_cast<double2*>(ds_full));
-  op.sync();  // the Lambda buffer is released on return
+  launch_loops(op, lam, cb, scale, static_cast<double2*>(ds_full));
 }
 
 void force_axpy(Op& op, int cb, double f, const void* ds_cb, void* ds_full) {

@@ -371,15 +371,15 @@ void meson_2pt(const int dims[4], const double* prop1, const double* prop2, cons
   int nchunk, groups;
   meson_chunks(g, nchunk, groups);
   const size_t least = meson_bytes(g, nchunk, 1, 1), whole = meson_bytes(g, nchunk, std::min(nmom, 64), g.L[3]);
-  DevBuf d1(pbytes), d2(same ? 0 : pbytes), dp(std::max(least, std::min(whole, MESON_SCRATCH_PART))), dt(sizeof(double2) * coefs.size()),
+  DevScratch d1(pbytes), d2(same ? 0 : pbytes), dp(std::max(least, std::min(whole, MESON_SCRATCH_PART))), dt(sizeof(double2) * coefs.size()),
       dm(sizeof(int) * 3 * (size_t)nmom), dout(sizeof(double2) * 16 * (size_t)nmom * g.L[3]);
-  CMX_HIP(hipMemcpy(d1.p, prop1, pbytes, hipMemcpyHostToDevice));
-  if (!same) CMX_HIP(hipMemcpy(d2.p, prop2, pbytes, hipMemcpyHostToDevice));
-  CMX_HIP(hipMemcpy(dt.p, coefs.data(), dt.bytes, hipMemcpyHostToDevice));
-  CMX_HIP(hipMemcpy(dm.p, moms, dm.bytes, hipMemcpyHostToDevice));
+  host_to_device(d1.get(), prop1, pbytes, 0);
+  if (!same) host_to_device(d2.get(), prop2, pbytes, 0);
+  CMX_HIP(hipMemcpy(dt.get(), coefs.data(), dt.bytes(), hipMemcpyHostToDevice));
+  CMX_HIP(hipMemcpy(dm.get(), moms, dm.bytes(), hipMemcpyHostToDevice));
   run_meson(g, d1.as<double2>(), same ? d1.as<double2>() : d2.as<double2>(), dt.as<double2>(), dm.as<int>(), nmom,
-            dp.as<double2>(), dp.bytes, dout.as<double2>(), 0);
-  CMX_HIP(hipMemcpy(corr, dout.p, dout.bytes, hipMemcpyDeviceToHost));
+            dp.as<double2>(), dp.bytes(), dout.as<double2>(), 0);
+  CMX_HIP(hipMemcpy(corr, dout.get(), dout.bytes(), hipMemcpyDeviceToHost));
 }
 
 void meson_scratch_setup() {

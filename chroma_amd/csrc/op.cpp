@@ -168,10 +168,9 @@ std::shared_ptr<GaugeData> make_gauge(const int dims[4], const double* const lin
   gd->g.Vh = (int)gd->Vh;
   // one copy per direction: the caller's arrays need not be contiguous (QUDA_QDP_GAUGE_ORDER)
   const size_t nd = (size_t)4 * V * 18;
-  DevBuf tmp(nd * sizeof(double));
+  DevScratch tmp(nd * sizeof(double));
   for (int mu = 0; mu < 4; ++mu)
-    CMX_HIP(hipMemcpy(tmp.as<double>() + (size_t)mu * V * 18, links[mu], (size_t)V * 18 * sizeof(double),
-                      hipMemcpyHostToDevice));
+    host_to_device(tmp.as<double>() + (size_t)mu * V * 18, links[mu], (size_t)V * 18 * sizeof(double), 0);
   for (int p = 0; p < 2; ++p) gd->g64[p].alloc((size_t)4 * 9 * 16 * gd->Vh);
   gauge_pack64(gd->g, tmp.as<double>(), gd->g64[0].as<double2>(), gd->g64[1].as<double2>(), 0);
   CMX_HIP(hipGetLastError());
@@ -510,12 +509,11 @@ bool Op::dslash_multi(int prec, const VRef* out, const VRef* in, int n, int isig
 
 void Op::upload(const double* host, size_t n) {
   CMX_REQUIRE(n * sizeof(double) <= staging.bytes, CMX_ERR_ARG, "upload: too large");
-  CMX_HIP(hipMemcpyAsync(staging.p, host, n * sizeof(double), hipMemcpyHostToDevice, stream));
+  host_to_device(staging.p, host, n * sizeof(double), stream);
 }
 void Op::download(double* host, size_t n) {
   CMX_REQUIRE(n * sizeof(double) <= staging.bytes, CMX_ERR_ARG, "download: too large");
-  CMX_HIP(hipMemcpyAsync(host, staging.p, n * sizeof(double), hipMemcpyDeviceToHost, stream));
-  CMX_HIP(hipStreamSynchronize(stream));
+  device_to_host(host, staging.p, n * sizeof(double), stream);
 }
 void Op::pack(const double* host, int nsites, const Vec& v, int off) {
   upload(host, (size_t)nsites * 24);

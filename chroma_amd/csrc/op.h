@@ -7,6 +7,7 @@
 #include "blas.h"
 #include "cmx_internal.h"
 #include "learned.h"
+#include "xfer.h"
 
 namespace cmx {
 
@@ -65,6 +66,21 @@ struct Vec {
     r.stride = n;
     return r;
   }
+};
+
+// A fermion vector of one call, from the scratch cache (its stream is synchronised before it goes)
+struct ScratchVec {
+  DevScratch mem;
+  Vec v;
+  ScratchVec(int prec, int n) : mem(spinor_bytes(prec, n)) {
+    v.prec = prec;
+    v.n = n;
+    v.buf.p = mem.get();
+    v.buf.bytes = mem.bytes();
+    v.buf.own = false;
+  }
+  operator const Vec&() const { return v; }
+  VRef view(int off = 0) const { return v.view(off); }
 };
 
 struct GaugeData {
@@ -182,20 +198,23 @@ void learned_precond_apply_batch(Op& op, int prec, const std::vector<const Vec*>
 // two must issue their work on one stream
 void learned_share(Op& from, Op& to);
 
-// mdagm: solve M^dag M psi = chi instead of M psi = chi
-void solve(Op& op, const cmx_solver_params& p, double* psi, const double* chi, bool mdagm, cmx_solver_result& res);
+// mdagm: solve M^dag M psi = chi instead of M psi = chi; from_zero: the initial guess is zero and psi is
+// only written
+void solve(Op& op, const cmx_solver_params& p, double* psi, const double* chi, bool mdagm, bool from_zero,
+           cmx_solver_result& res);
 // WilsonDslashBase::deriv (lwldslash_base_w.h:132-227) for the sites of cb, FP64 (deriv.hip): chi on cb,
 // psi on 1 - cb, ds = 4 * Vh * 9 double2 (direction, site of cb, 3x3 row-major)
 void hop_deriv(const Geom& g, int cb, int isign, VRef chi, VRef psi, void* ds, hipStream_t s);
 // Clover force (force.hip), FP64, accumulated into ds_full = [4][V][9] double2 (host site order) times
 // scale: trln = false: CloverTermBase::deriv on cb from chi, psi (views of cb); trln = true: derivTrLn
-// of the inverted even-even term (cb = 0; chi, psi unused).  force_axpy adds f times a hopping-term
+// of the inverted even-even term (cb = 0; chi, psi unused).  lam: 6 x 9 x 16 x Vh bytes of device work
+// space, in use until op's stream has passed the call.  force_axpy adds f times a hopping-term
 // derivative of one checkerboard (hop_deriv's layout) into ds_full.
-void clover_force(Op& op, bool trln, int cb, VRef chi, VRef psi, double scale, void* ds_full);
+void clover_force(Op& op, bool trln, int cb, VRef chi, VRef psi, double scale, void* ds_full, void* lam);
 void force_axpy(Op& op, int cb, double f, const void* ds_cb, void* ds_full);
-// nstep stout steps on the device over the directions in the bit mask dirs, in place on host-layout
-// links (stout.hip)
-void stout_smear(const int dims[4], double* links, int nstep, double rho, int dirs = 15);
+// nstep stout steps on the device over the directions in the bit mask dirs, from host-layout links to
+// host-layout links (stout.hip); out may be in
+void stout_smear(const int dims[4], const double* in, double* out, int nstep, double rho, int dirs = 15);
 // meson two-point functions of two host-layout propagators for the 16 gamma insertions (meson.hip)
 void meson_2pt(const int dims[4], const double* prop1, const double* prop2, const int origin[4], int nmom,
                const int* moms, double* corr);
@@ -215,7 +234,7 @@ void solve_multishift(Op& op, const cmx_solver_params& p, int ns, const double* 
 // The same for n problems at once (batch.h): problem i solves on ops[i] (distinct solver contexts,
 // one stream); solver RELIABLE_CG or CG
 void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const cmx_batch_params& bp,
-                 double* const* psi, const double* const* chi, bool mdagm, cmx_solver_result* res,
+                 double* const* psi, const double* const* chi, bool mdagm, bool from_zero, cmx_solver_result* res,
                  cmx_batch_result& bres);
 
 }  // namespace cmx

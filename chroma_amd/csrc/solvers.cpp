@@ -72,6 +72,14 @@ void read_state(Op& op) {
   op.sync();
 }
 
+// the initial guess on the device: a host field, or zero
+void set_guess(Op& op, const double* host, Vec& psi) {
+  if (host)
+    op.pack(host, psi.n, psi);
+  else
+    op.blas(B_ZERO, {&psi});
+}
+
 // |v|^2 on the host (one synchronisation)
 double norm2(Op& op, const Vec& v) {
   op.blas(B_NORM2, {&v});
@@ -383,8 +391,10 @@ void solve_relbicgstab(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& 
   CMX_REQUIRE(ps == P64 || ps == P32 || ps == P16, CMX_ERR_ARG, "reliable BiCGStab: bad sloppy precision");
   const int px = ps == P64 ? P64 : P32;
   const int nb = blas_blocks(n);
-  Vec b(P64, n), tmp(P64, n), r_dble(P64, n), x_dble(P64, n);
-  Vec r(ps, n), r0(ps, n), pv(ps, n), v(ps, n), t(ps, n), x(px, n);
+  Vec &b = op.work(50, P64, n), &tmp = op.work(51, P64, n), &r_dble = op.work(52, P64, n),
+      &x_dble = op.work(53, P64, n);
+  Vec &r = op.work(54, ps, n), &r0 = op.work(55, ps, n), &pv = op.work(56, ps, n), &v = op.work(57, ps, n),
+      &t = op.work(58, ps, n), &x = op.work(59, px, n);
   const double chi_sq = norm2(op, chi);  // rsd_sq = Rsd^2 |chi|^2 (:65)
   reset_state(op, p.rsd_target * p.rsd_target * chi_sq, p.max_iter, p.delta);
   Timer tm(op.stream);
@@ -555,7 +565,7 @@ size_t fgmres_workspace_bytes(const Op& op, const cmx_solver_params& p) {
 // solve performs exactly the kernels and host arithmetic of cmx_solve, so its result is the same bit for
 // bit.  As many solves run at once as their workspaces fit in free device memory; the others wait.
 void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p, int max_concurrent,
-                        double* const* psi_h, const double* const* chi_h, cmx_solver_result* res,
+                        double* const* psi_h, const double* const* chi_h, bool from_zero, cmx_solver_result* res,
                         cmx_batch_result& bres) {
   const int np = (int)ops.size();
   std::vector<hipStream_t> streams;
@@ -597,7 +607,7 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
     Op& op = *ctx[i];
     const int n = op.subset_sites();
     op.pack(chi_h[i], n, op.work(1, P64, n));
-    op.pack(psi_h[i], n, op.work(0, P64, n));
+    set_guess(op, from_zero ? nullptr : psi_h[i], op.work(0, P64, n));
     op.work(2, P64, n);
     op.work(3, P64, n);
     FgmresDR::reserve(op, q[i]);
@@ -827,7 +837,7 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
 }  // namespace
 
 void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const cmx_batch_params& bp,
-                 double* const* psi_h, const double* const* chi_h, bool mdagm, cmx_solver_result* res,
+                 double* const* psi_h, const double* const* chi_h, bool mdagm, bool from_zero, cmx_solver_result* res,
                  cmx_batch_result& bres) {
   const auto t0 = std::chrono::steady_clock::now();
   const int np = (int)ops.size();
@@ -841,7 +851,7 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
   if (p.solver == CMX_SOLVER_FGMRESDR) {
     CMX_REQUIRE(!mdagm, CMX_ERR_UNSUPPORTED, "FGMRES-DR is a LinOp system solver (no MdagM form)");
     std::memset(&bres, 0, sizeof(bres));
-    solve_batch_fgmres(ops, p, bp.max_concurrent, psi_h, chi_h, res, bres);
+    solve_batch_fgmres(ops, p, bp.max_concurrent, psi_h, chi_h, from_zero, res, bres);
     bres.total_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     for (int i = 0; i < np; ++i) {
       res[i].solve_seconds = bres.solve_seconds;
@@ -876,7 +886,7 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     op.work(2, P64, n);
     op.work(3, P64, n);
     op.pack(chi_h[i], n, *chi[i]);
-    op.pack(psi_h[i], n, *psi[i]);
+    set_guess(op, from_zero ? nullptr : psi_h[i], *psi[i]);
     std::memset(&res[i], 0, sizeof(res[i]));
     // true-residual mode aims the first pass a little below the target, as the single solve does
     if (p.true_residual) q[i].rsd_target = 0.5 * p.rsd_target;
@@ -1090,13 +1100,14 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
   for (int i = 0; i < np; ++i) res[i].total_seconds = bres.total_seconds;
 }
 
-void solve(Op& op, const cmx_solver_params& p, double* psi_h, const double* chi_h, bool mdagm, cmx_solver_result& res) {
+void solve(Op& op, const cmx_solver_params& p, double* psi_h, const double* chi_h, bool mdagm, bool from_zero,
+           cmx_solver_result& res) {
   CMX_REQUIRE(p.max_iter > 0 && p.rsd_target > 0, CMX_ERR_ARG, "solve: MaxIter and RsdTarget must be positive");
   const auto t0 = std::chrono::steady_clock::now();
   const int n = op.subset_sites();
   Vec &psi = op.work(0, P64, n), &chi = op.work(1, P64, n);
   op.pack(chi_h, n, chi);
-  op.pack(psi_h, n, psi);
+  set_guess(op, from_zero ? nullptr : psi_h, psi);
   std::memset(&res, 0, sizeof(res));
   cmx_solver_params q = p;
   // true-residual mode aims the first pass a little below the target, so that a restart is rare

@@ -16,6 +16,7 @@
 // that layout and the result is transposed back.  One lane per (mu, site); each link is read by 13 lanes
 // (its own, and as a staple leg of 12 others), mostly from L2.
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <utility>
 
@@ -245,8 +246,8 @@ __global__ void __launch_bounds__(256) k_stout_step(StoutGeom g, const double2* 
 
 }  // namespace
 
-void stout_smear(const int dims[4], double* links, int nstep, double rho, int dirs) {
-  CMX_REQUIRE(dims && links, CMX_ERR_ARG, "gauge_stout_smear: null array");
+void stout_smear(const int dims[4], const double* in, double* out, int nstep, double rho, int dirs) {
+  CMX_REQUIRE(dims && in && out, CMX_ERR_ARG, "gauge_stout_smear: null array");
   CMX_REQUIRE(dirs >= 0 && dirs <= 15, CMX_ERR_ARG, "gauge_stout_smear: smeared directions are a 4-bit mask");
   CMX_REQUIRE(nstep >= 0, CMX_ERR_ARG, "gauge_stout_smear: nstep must be >= 0");
   CMX_REQUIRE(std::isfinite(rho), CMX_ERR_ARG, "gauge_stout_smear: rho must be finite");
@@ -259,10 +260,13 @@ void stout_smear(const int dims[4], double* links, int nstep, double rho, int di
   }
   g.Vh = g.V / 2;
   CMX_REQUIRE(4 * g.V <= (long)INT32_MAX * 256, CMX_ERR_ARG, "gauge_stout_smear: lattice too large for one grid");
-  if (nstep == 0) return;
   const size_t bytes = sizeof(double) * 18 * 4 * (size_t)g.V;
-  DevBuf a(bytes), b(bytes);
-  CMX_HIP(hipMemcpy(a.p, links, bytes, hipMemcpyHostToDevice));
+  if (nstep == 0) {
+    if (out != in) std::memcpy(out, in, bytes);
+    return;
+  }
+  DevScratch a(bytes), b(bytes);
+  host_to_device(a.get(), in, bytes, 0);
   const dim3 grid((unsigned)((4 * g.V + 255) / 256));
   hipLaunchKernelGGL(k_links_to_soa, grid, dim3(256), 0, 0, g.V, a.as<double2>(), b.as<double2>());
   CMX_HIP(hipGetLastError());
@@ -275,7 +279,7 @@ void stout_smear(const int dims[4], double* links, int nstep, double rho, int di
   }
   hipLaunchKernelGGL(k_links_from_soa, grid, dim3(256), 0, 0, g.V, cur, nxt);
   CMX_HIP(hipGetLastError());
-  CMX_HIP(hipMemcpy(links, nxt, bytes, hipMemcpyDeviceToHost));
+  device_to_host(out, nxt, bytes, 0);
 }
 
 }  // namespace cmx

@@ -126,11 +126,17 @@ def lib():
                                      ctypes.POINTER(SolverResult)]),
         "cmx_solve_mdagm": (ctypes.c_int, [_vp, ctypes.POINTER(SolverParams), _dp, _dp, ctypes.c_int,
                                            ctypes.POINTER(SolverResult)]),
+        "cmx_solve_from_zero": (ctypes.c_int, [_vp, ctypes.POINTER(SolverParams), _dp, _dp, ctypes.c_int, ctypes.c_int,
+                                               ctypes.POINTER(SolverResult)]),
         "cmx_solve_multishift": (ctypes.c_int, [_vp, ctypes.POINTER(SolverParams), ctypes.c_int, _dp, _dp, _dp, _dp,
                                                 ctypes.POINTER(SolverResult)]),
         "cmx_solve_batch": (ctypes.c_int, [ctypes.POINTER(_vp), ctypes.c_int, ctypes.POINTER(SolverParams),
                                            ctypes.POINTER(BatchParams), ctypes.POINTER(_dp), ctypes.POINTER(_dp),
                                            ctypes.c_int, ctypes.POINTER(SolverResult), ctypes.POINTER(BatchResult)]),
+        "cmx_solve_batch_from_zero": (ctypes.c_int, [ctypes.POINTER(_vp), ctypes.c_int, ctypes.POINTER(SolverParams),
+                                                     ctypes.POINTER(BatchParams), ctypes.POINTER(_dp),
+                                                     ctypes.POINTER(_dp), ctypes.c_int, ctypes.POINTER(SolverResult),
+                                                     ctypes.POINTER(BatchResult)]),
         "cmx_net_create": (ctypes.c_int, [ctypes.POINTER(_vp)]),
         "cmx_net_destroy": (ctypes.c_int, [_vp]),
         "cmx_net_init_neumann": (ctypes.c_int, [_vp, ctypes.c_double]),
@@ -166,6 +172,7 @@ def lib():
         "cmx_plaquette": (ctypes.c_double, [_ip, _dp]),
         "cmx_gauge_stout_smear": (ctypes.c_int, [_ip, _dp, ctypes.c_int, ctypes.c_double]),
         "cmx_gauge_stout_smear_dirs": (ctypes.c_int, [_ip, _dp, ctypes.c_int, ctypes.c_double, ctypes.c_int]),
+        "cmx_gauge_stout_smear_to": (ctypes.c_int, [_ip, _dp, _dp, ctypes.c_int, ctypes.c_double, ctypes.c_int]),
         "cmx_meson_2pt": (ctypes.c_int, [_ip, _dp, _dp, _ip, ctypes.c_int, _ip, _dp]),
         "cmx_meson_2pt_noalloc": (ctypes.c_int, [_ip, _vp, _vp, _ip, ctypes.c_int, _vp, _vp, _vp]),
         "cmx_fill_z2": (ctypes.c_int, [ctypes.c_long, ctypes.c_ulonglong, _dp]),
@@ -231,11 +238,9 @@ def gauge_stout_smear(L, U, nstep, rho, smear_dirs=15):
     """nstep stout steps on the device (Stouting::smear_links, stout_utils.cc:936-962) over the directions
     whose bit is set in smear_dirs (15: all, 7: spatial); returns a new complex128[4, V, 3, 3]."""
     init()
-    out = np.array(U, np.complex128, order="C", copy=True)
-    if smear_dirs == 15:
-        check(lib().cmx_gauge_stout_smear(_dims(L), _d(out), int(nstep), float(rho)))
-    else:
-        check(lib().cmx_gauge_stout_smear_dirs(_dims(L), _d(out), int(nstep), float(rho), int(smear_dirs)))
+    U = np.ascontiguousarray(U, np.complex128)
+    out = np.empty_like(U)
+    check(lib().cmx_gauge_stout_smear_to(_dims(L), _d(U), _d(out), int(nstep), float(rho), int(smear_dirs)))
     return out
 
 
@@ -348,20 +353,20 @@ class Operator:
 
     def __call__(self, psi, isign=PLUS, prec=DOUBLE):
         psi = np.ascontiguousarray(psi, np.complex128)
-        chi = np.zeros_like(psi)
+        chi = np.empty_like(psi)
         check(lib().cmx_op_apply(self.h, _d(chi), _d(psi), int(isign), int(prec)))
         return chi
 
     def dslash(self, psi_cb, isign, cb, prec=DOUBLE):
         psi_cb = np.ascontiguousarray(psi_cb, np.complex128)
-        chi = np.zeros_like(psi_cb)
+        chi = np.empty_like(psi_cb)
         check(lib().cmx_dslash_apply(self.h, _d(chi), _d(psi_cb), int(isign), int(cb), int(prec)))
         return chi
 
     def dslash_multi(self, psis_cb, isign, cb, prec=HALF):
         """D on n sources at once: psis_cb complex[n, Vh, 4, 3]."""
         psis_cb = np.ascontiguousarray(psis_cb, np.complex128)
-        chi = np.zeros_like(psis_cb)
+        chi = np.empty_like(psis_cb)
         check(lib().cmx_dslash_multi(self.h, int(psis_cb.shape[0]), _d(chi), _d(psis_cb), int(isign), int(cb),
                                      int(prec)))
         return chi
@@ -369,27 +374,27 @@ class Operator:
     def dslash_deriv(self, chi_full, psi_full, isign=PLUS, cb=-1):
         """WilsonDslashBase::deriv (lwldslash_base_w.h:132-227): ds_u complex[4, V, 3, 3] from full-lattice
         chi, psi; cb 0/1 one checkerboard, -1 both."""
-        ds = np.zeros((4, self.V, 3, 3), np.complex128)
+        ds = np.empty((4, self.V, 3, 3), np.complex128)
         check(lib().cmx_dslash_deriv(self.h, _d(ds), _d(np.ascontiguousarray(chi_full, np.complex128)),
                                      _d(np.ascontiguousarray(psi_full, np.complex128)), int(isign), int(cb)))
         return ds
 
     def clover_deriv(self, chi_full, psi_full, isign=PLUS, cb=-1):
         """CloverTermBase::deriv: ds[4, V, 3, 3] of chi^dag A' psi over cb (-1: both checkerboards)."""
-        ds = np.zeros((4, self.V, 3, 3), np.complex128)
+        ds = np.empty((4, self.V, 3, 3), np.complex128)
         check(lib().cmx_clover_deriv(self.h, _d(ds), _d(np.ascontiguousarray(chi_full, np.complex128)),
                                      _d(np.ascontiguousarray(psi_full, np.complex128)), int(isign), int(cb)))
         return ds
 
     def clover_deriv_trln(self):
         """CloverTermBase::derivTrLn of the inverted even-even clover term (the even-even log det force)."""
-        ds = np.zeros((4, self.V, 3, 3), np.complex128)
+        ds = np.empty((4, self.V, 3, 3), np.complex128)
         check(lib().cmx_clover_deriv_trln(self.h, _d(ds)))
         return ds
 
     def deriv(self, chi_odd, psi_odd, isign=PLUS):
         """EvenOddPrecLogDetLinearOperator::deriv: ds[4, V, 3, 3] of chi^dag M'(isign) psi (odd arrays)."""
-        ds = np.zeros((4, self.V, 3, 3), np.complex128)
+        ds = np.empty((4, self.V, 3, 3), np.complex128)
         check(lib().cmx_op_deriv(self.h, _d(ds), _d(np.ascontiguousarray(chi_odd, np.complex128)),
                                  _d(np.ascontiguousarray(psi_odd, np.complex128)), int(isign)))
         return ds
@@ -397,7 +402,7 @@ class Operator:
     def piece(self, which, psi_full, isign=PLUS):
         names = {"evenEven": 0, "evenEvenInv": 1, "evenOdd": 2, "oddEven": 3, "oddOdd": 4, "unprec": 5}
         psi_full = np.ascontiguousarray(psi_full, np.complex128)
-        chi = np.zeros_like(psi_full)
+        chi = np.zeros(psi_full.shape, np.complex128)  # one checkerboard may stay unwritten
         check(lib().cmx_op_eo_piece(self.h, names[which], _d(chi), _d(psi_full), int(isign)))
         return chi
 
@@ -525,15 +530,18 @@ class Operator:
         chi = np.ascontiguousarray(chi, np.complex128)
         single = chi.ndim == 3
         chis = chi[None] if single else chi
-        psis = np.zeros_like(chis) if psi is None else np.ascontiguousarray(psi, np.complex128).reshape(chis.shape).copy()
+        psis = np.empty_like(chis) if psi is None else np.ascontiguousarray(psi, np.complex128).reshape(chis.shape).copy()
         nrhs = chis.shape[0]
         p = SolverParams(int(solver), int(maxit), float(rsd), float(delta), int(sloppy_prec), int(check_every),
                          int(bool(verbose)), int(bool(true_residual)), int(n_krylov), int(n_defl), int(precond),
                          int(precond_iters), float(precond_rsd), float(precond_omega), int(reorth), int(basis_prec),
                          float(cycle_reduction), int(bool(graph)))
         res = (SolverResult * nrhs)()
-        fn = lib().cmx_solve_mdagm if mdagm else lib().cmx_solve
-        check(fn(self.h, ctypes.byref(p), _d(psis), _d(chis), nrhs, res))
+        if psi is None:
+            check(lib().cmx_solve_from_zero(self.h, ctypes.byref(p), _d(psis), _d(chis), nrhs, int(bool(mdagm)), res))
+        else:
+            fn = lib().cmx_solve_mdagm if mdagm else lib().cmx_solve
+            check(fn(self.h, ctypes.byref(p), _d(psis), _d(chis), nrhs, res))
         out = [dict(n_count=r.n_count, resid=r.resid, rel_resid=r.rel_resid, n_reliable=r.n_reliable,
                     solve_seconds=r.solve_seconds, total_seconds=r.total_seconds, gflops=r.gflops,
                     n_restarts=r.n_restarts) for r in res]
@@ -546,7 +554,7 @@ class Operator:
         shifts = np.ascontiguousarray(shifts, np.float64)
         rsd = np.ascontiguousarray(np.broadcast_to(np.asarray(rsd, np.float64), shifts.shape))
         ns = len(shifts)
-        psis = np.zeros((ns,) + chi.shape, np.complex128)
+        psis = np.empty((ns,) + chi.shape, np.complex128)
         p = SolverParams(CG, int(maxit), float(rsd.max()), 0.1, DOUBLE, 0, int(bool(verbose)), 0, 16, 0, 0, 4,
                          1e-12, 1.0, 1, -1, 0.0, 0)
         res = (SolverResult * ns)()
@@ -566,7 +574,8 @@ def solve_batch(ops, chis, psis=None, solver=RELIABLE_CG, rsd=1e-10, maxit=10000
     n = len(ops)
     assert len(chis) == n
     chis = [np.ascontiguousarray(c, np.complex128) for c in chis]
-    psis = [np.zeros_like(c) for c in chis] if psis is None else \
+    fn = lib().cmx_solve_batch_from_zero if psis is None else lib().cmx_solve_batch
+    psis = [np.empty_like(c) for c in chis] if psis is None else \
         [np.ascontiguousarray(x, np.complex128).copy() for x in psis]
     p = SolverParams(int(solver), int(maxit), float(rsd), float(delta), int(sloppy_prec), int(check_every),
                      0, int(bool(true_residual)), int(n_krylov), int(n_defl), int(precond), int(precond_iters),
@@ -578,8 +587,7 @@ def solve_batch(ops, chis, psis=None, solver=RELIABLE_CG, rsd=1e-10, maxit=10000
     cp = (_dp * n)(*[_d(c) for c in chis])
     res = (SolverResult * n)()
     br = BatchResult()
-    check(lib().cmx_solve_batch(hs, n, ctypes.byref(p), ctypes.byref(bp), pp, cp, int(bool(mdagm)), res,
-                                ctypes.byref(br)))
+    check(fn(hs, n, ctypes.byref(p), ctypes.byref(bp), pp, cp, int(bool(mdagm)), res, ctypes.byref(br)))
     out = [dict(n_count=r.n_count, resid=r.resid, rel_resid=r.rel_resid, n_reliable=r.n_reliable,
                 solve_seconds=r.solve_seconds, total_seconds=r.total_seconds, gflops=r.gflops,
                 n_restarts=r.n_restarts) for r in res]
@@ -649,7 +657,7 @@ def net_set_variant(op, prec, variant):
 
 def net_apply(op, v, prec=SINGLE):
     v = np.ascontiguousarray(v, np.complex128)
-    out = np.zeros_like(v)
+    out = np.empty_like(v)
     check(lib().cmx_net_apply(op.h, int(prec), _d(out), _d(v)))
     return out
 

@@ -216,6 +216,11 @@ int cmx_solve(cmx_op op, const cmx_solver_params* p, double* psi, const double* 
 int cmx_solve_mdagm(cmx_op op, const cmx_solver_params* p, double* psi, const double* chi, int nrhs,
                     cmx_solver_result* res);
 
+/* cmx_solve (mdagm = 0) or cmx_solve_mdagm (1) from the initial guess zero: psi is only written, so the
+ * caller's array need not be cleared and is not sent to the device. */
+int cmx_solve_from_zero(cmx_op op, const cmx_solver_params* p, double* psi, const double* chi, int nrhs, int mdagm,
+                        cmx_solver_result* res);
+
 /* MdagMMultiSystemSolver with CG (multi_syssolver_mdagm_cg.h:58-100 -> MInvCG2, minvcg2.cc:72-355):
  * solves (M^dag M + shifts[s]) psi_s = chi for s < nshift (1..64) with one Krylov space, in FP64 --
  * the rational-approximation solves of RHMC.  Every psi_s starts at zero, as MInvCG2 requires (the
@@ -261,6 +266,10 @@ typedef struct {
 int cmx_solve_batch(const cmx_op* ops, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
                     double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
                     cmx_batch_result* bres);
+/* The same with every initial guess zero: the psi arrays are only written. */
+int cmx_solve_batch_from_zero(const cmx_op* ops, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
+                              double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
+                              cmx_batch_result* bres);
 
 /* ---- learned preconditioner (CMX_PRECOND_LEARNED): no counterpart in the reference ------------------
  * A gauge-equivariant parallel-transport network on the odd checkerboard, a chain of 1..4 blocks
@@ -427,6 +436,9 @@ int cmx_gauge_stout_smear(const int dims[4], double* links, int nstep, double rh
  * directions are left as they are and contribute no staples (rho(mu,nu) = 0 when either is unsmeared);
  * 15 is cmx_gauge_stout_smear, 7 the usual spatial smearing with no_smear_dir = 3. */
 int cmx_gauge_stout_smear_dirs(const int dims[4], double* links, int nstep, double rho, int smear_dirs);
+/* The same from links to out (which may be links), for callers that keep the unsmeared field. */
+int cmx_gauge_stout_smear_to(const int dims[4], const double* links, double* out, int nstep, double rho,
+                             int smear_dirs);
 /* Meson two-point functions on the device: mesons() (mesons_w.cc:97-180) for the 16 insertions
  * Gamma(n) = gamma_1^n0 gamma_2^n1 gamma_3^n2 gamma_4^n3 with the sink-momentum projection of
  * SftMom::sft (sftmom.cc:405-460), decay direction 3:
