@@ -1,8 +1,9 @@
 // Multishift CG (MInvCG2_a, minvcg2.cc:72-355; MdagMMultiSysSolverCG, multi_syssolver_mdagm_cg.h:58-100):
 // (M^dag M + shifts[s]) psi[s] = chi for every shift with one Krylov space (Jegerlehner,
-// hep-lat/9708029), in FP64 on the device.  The vectors live on the device; the scalar recurrences of
-// the shifted systems (z, bs, as) are a few flops per shift and run on the host in double, as the
-// reference runs them, from the two reductions each iteration reads back (d = |M p|^2, c = |r|^2).
+// hep-lat/9708029), in FP64 on the device.  Vectors and the shifted recurrences (z, bs, as) live there, so
+// an iteration is nine launches with no host value between them; the host polls the stop flag every few
+// iterations (two read-backs and three coefficient copies per iteration when the recurrences ran on the
+// host left the device idle for 50 to 70 us of each 0.4 ms at 16^3x32).
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -10,33 +11,19 @@
 #include <memory>
 #include <vector>
 
-#include "blas.h"
+#include "multishift.h"
 #include "op.h"
 
 namespace cmx {
 
 namespace {
 
-constexpr int MS_MAX = 64;             // shifts per solve
-constexpr int MS_D = S_KRY;            // device-written: d = |M p0|^2
-constexpr int MS_C = S_KRY + 1;        // device-written: c = |r|^2
-constexpr int MS_B = S_KRY + 2;        // host-written: b
-constexpr int MS_SIG = S_KRY + 3;      // host-written: the shift of the residual check
-constexpr int MS_X = S_KRY + 8;        // host-written: a, then (z_s, as_s) for every shift
-constexpr int MS_NBS = MS_X + 1 + 2 * MS_MAX;  // host-written: -bs_s
-static_assert(MS_NBS + MS_MAX <= S_MR, "multishift slots overlap the MR slots");
-
-void put(Op& op, int slot, const double* v, int n) {
-  std::memcpy(op.hS + slot, v, sizeof(double) * n);
-  CMX_HIP(hipMemcpyAsync(static_cast<double*>(op.state_S.p) + slot, op.hS + slot, sizeof(double) * n,
-                         hipMemcpyHostToDevice, op.stream));
-}
-double get(Op& op, int slot) {
-  CMX_HIP(hipMemcpyAsync(op.hS + slot, static_cast<double*>(op.state_S.p) + slot, sizeof(double),
-                         hipMemcpyDeviceToHost, op.stream));
-  op.sync();
-  return op.hS[slot];
-}
+constexpr int MS_A = S_KRY;        // a, b of the p0 and r updates
+constexpr int MS_B = S_KRY + 1;
+constexpr int MS_C = S_KRY + 2;    // |chi|^2
+constexpr int MS_SIG = S_KRY + 8;  // the shifts, for the residual checks
+constexpr int MS_RES = MS_SIG + MS_MAX;  // |chi - (M^dag M + shift_s) psi_s|^2
+static_assert(MS_RES + MS_MAX <= S_MR, "multishift slots overlap the MR slots");
 
 }  // namespace
 
@@ -51,11 +38,18 @@ void solve_multishift(Op& op, const cmx_solver_params& p, int ns, const double* 
   const int nb = blas_blocks(n);
   Vec &chi = op.work(1, P64, n), &r = op.work(11, P64, n), &p0 = op.work(12, P64, n), &mp = op.work(13, P64, n),
       &mmp = op.work(14, P64, n);
-  std::vector<std::unique_ptr<Vec>> psi, pv;
-  for (int s = 0; s < ns; ++s) {
-    psi.emplace_back(new Vec(P64, n));
-    pv.emplace_back(new Vec(P64, n));
-  }
+  // p_s and psi_s of all shifts in one allocation
+  const size_t vb = spinor_bytes(P64, n);
+  DevScratch vecs(2 * vb * ns), state(sizeof(MsState));
+  auto psi_of = [&](int s) {
+    Vec v;
+    v.prec = P64;
+    v.n = n;
+    v.buf.p = vecs.as<char>() + vb * (ns + s);
+    v.buf.bytes = vb;
+    v.buf.own = false;
+    return v;
+  };
   op.pack(chi_h, n, chi);
   hipEvent_t e0, e1;
   CMX_HIP(hipEventCreate(&e0));
@@ -73,111 +67,96 @@ void solve_multishift(Op& op, const cmx_solver_params& p, int ns, const double* 
   int isz = 0;
   for (int s = 1; s < ns; ++s)
     if (shifts[s] < shifts[isz]) isz = s;
-  for (int s = 0; s < ns; ++s) op.blas(B_ZERO, {psi[s].get()});  // (:118-121)
+  MsLaunch L;
+  std::memset(&L, 0, sizeof(L));
+  L.ne = 12L * n;
+  L.ns = ns;
+  L.isz = isz;
+  L.max_iter = p.max_iter;
+  L.st = state.as<MsState>();
+  L.S = op.state_S.as<double>();
+  L.F = op.state_F.as<int>();
+  L.slot_a = MS_A;
+  L.slot_b = MS_B;
+  L.partials = op.partials.as<double>();
+  L.r = r.buf.as<double2>();
+  L.p0 = p0.buf.as<double2>();
+  L.p = vecs.as<double2>();
+  L.psi = vecs.as<double2>() + L.ne * ns;
+  ms_init(L, chi.buf.as<double2>(), op.stream);  // r = p0 = p_s = chi, psi_s = 0 (:118-121, :161-175)
   op.blas(B_NORM2, {&chi});
   op.finalize(nb, 1, PG_STORE, MS_C);
-  const double chi_norm_sq = get(op, MS_C);
+  CMX_HIP(hipMemcpyAsync(op.hS + MS_C, static_cast<double*>(op.state_S.p) + MS_C, sizeof(double),
+                         hipMemcpyDeviceToHost, op.stream));
+  op.sync();
+  const double chi_norm_sq = op.hS[MS_C];
   int n_count = 0;
   if (std::sqrt(chi_norm_sq) >= 1e-10) {  // a zero source returns the zero solutions (:133-153)
-    std::vector<double> rsd_sq(ns), bs(ns), z[2] = {std::vector<double>(ns), std::vector<double>(ns)};
-    for (int s = 0; s < ns; ++s) rsd_sq[s] = chi_norm_sq * rsd[s] * rsd[s];
-    double cp = chi_norm_sq;
-    // r = p0 = p_s = chi (:161-175)
-    op.blas(B_COPY, {&r, &chi});
-    op.blas(B_COPY, {&p0, &chi});
-    for (int s = 0; s < ns; ++s) op.blas(B_COPY, {pv[s].get(), &chi});
-    // b = -|r|^2 / |M p0|^2 ; r += b M^dag M p0 (:179-194)
-    int np = op.apply(P64, mp.view(), p0.view(), +1, op.partials.as<double>());
-    op.finalize(np, 1, PG_STORE, MS_D);
-    op.apply(P64, mmp.view(), mp.view(), -1, nullptr);
-    double d = get(op, MS_D);
-    CMX_REQUIRE(d > 0 && std::isfinite(d), CMX_ERR_BREAKDOWN, "multishift CG: |M p| = 0 or not finite");
-    double b = -cp / d;
-    put(op, MS_B, &b, 1);
-    op.blas(B_AXPY_NORM, {&r, &mmp}, MS_B);
-    op.finalize(nb, 1, PG_STORE, MS_C);
-    // shifted bs and z (:197-217); psi_s = -bs_s chi (:221-225)
-    int iz = 1;
-    std::vector<double> nbs(ns);
-    for (int s = 0; s < ns; ++s) {
-      z[1 - iz][s] = 1.0;
-      z[iz][s] = 1.0 / (1.0 - shifts[s] * b);
-      bs[s] = b * z[iz][s];
-      nbs[s] = -bs[s];
-    }
-    put(op, MS_NBS, nbs.data(), ns);
-    for (int s = 0; s < ns; ++s) op.blas(B_SCALE, {psi[s].get(), &chi}, MS_NBS + s);
-    double c = get(op, MS_C);
-    std::vector<char> conv(ns, 0);
-    bool convP = c < rsd_sq[isz];
-    std::vector<double> x(1 + 2 * ns);
-    for (int k = 1; k <= p.max_iter && !convP; ++k) {
-      // p0 = r + a p0 ; p_s = z_s r + as_s p_s (:253-273)
-      const double a = c / cp;
-      x[0] = a;
-      for (int s = 0; s < ns; ++s) {
-        x[1 + 2 * s] = z[iz][s];
-        x[2 + 2 * s] = conv[s] ? 0.0 : a * z[iz][s] * bs[s] / (z[1 - iz][s] * b);
+    MsState h;
+    std::memset(&h, 0, sizeof(h));
+    h.cp = chi_norm_sq;
+    for (int s = 0; s < ns; ++s) h.sigma[s] = shifts[s], h.rsd_sq[s] = chi_norm_sq * rsd[s] * rsd[s];
+    CMX_HIP(hipMemcpy(state.get(), &h, sizeof(h), hipMemcpyHostToDevice));
+    std::memset(op.hF, 0, sizeof(int) * F_NFLAGS);
+    CMX_HIP(hipMemcpyAsync(op.state_F.p, op.hF, sizeof(int) * F_NFLAGS, hipMemcpyHostToDevice, op.stream));
+    op.sync();
+    int* F = op.state_F.as<int>();
+    // b = -|r|^2 / |M p0|^2 ; r += b M^dag M p0 ; c = |r|^2 and the recurrences (:179-217, :275-339)
+    auto step = [&](int phase) {
+      L.nb = op.apply(P64, mp.view(), p0.view(), +1, op.partials.as<double>(), F + F_DONE);
+      ms_scalars(L, 1, op.stream);
+      op.apply(P64, mmp.view(), mp.view(), -1, nullptr, F + F_DONE);
+      op.blas(B_AXPY_NORM, {&r, &mmp}, MS_B, 0, F_DONE);
+      L.nb = nb;
+      ms_scalars(L, phase, op.stream);
+    };
+    auto poll = [&]() {
+      CMX_HIP(hipMemcpyAsync(op.hF, op.state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, op.stream));
+      if (p.verbose) CMX_HIP(hipMemcpyAsync(&h.c, &L.st->c, sizeof(double), hipMemcpyDeviceToHost, op.stream));
+      op.sync();
+      CMX_REQUIRE(op.hF[F_ERR] != CMX_ERR_BREAKDOWN, CMX_ERR_BREAKDOWN, "multishift CG: |M p| = 0 or not finite");
+      return op.hF[F_CONV] != 0;
+    };
+    step(0);
+    const int batch = p.verbose ? 1 : 6;
+    for (long k = 0; !poll() && k <= (long)p.max_iter + batch; k += batch) {
+      if (p.verbose && k > 0) std::printf("MInvCG2: k = %ld |r| = %g\n", k, std::sqrt(h.c));
+      for (int j = 0; j < batch; ++j) {
+        ms_update(L, op.stream);  // p0 = r + a p0 ; psi_s -= bs_s p_s ; p_s = z_s r + as_s p_s (:253-273, :312-322)
+        step(2);
       }
-      put(op, MS_X, x.data(), 1 + 2 * ns);
-      op.blas(B_XPAY, {&p0, &r}, MS_X);
-      for (int s = 0; s < ns; ++s)
-        if (!conv[s]) op.blas(B_AXPBY, {pv[s].get(), &r}, MS_X + 1 + 2 * s, MS_X + 2 + 2 * s);
-      cp = c;
-      // b = -cp / |M p0|^2 ; r += b M^dag M p0 ; c = |r|^2 (:275-294)
-      np = op.apply(P64, mp.view(), p0.view(), +1, op.partials.as<double>());
-      op.finalize(np, 1, PG_STORE, MS_D);
-      op.apply(P64, mmp.view(), mp.view(), -1, nullptr);
-      d = get(op, MS_D);
-      CMX_REQUIRE(d > 0 && std::isfinite(d), CMX_ERR_BREAKDOWN, "multishift CG: |M p| = 0 or not finite");
-      const double bp = b;
-      b = -cp / d;
-      put(op, MS_B, &b, 1);
-      op.blas(B_AXPY_NORM, {&r, &mmp}, MS_B);
-      op.finalize(nb, 1, PG_STORE, MS_C);
-      c = get(op, MS_C);
-      // shifted z and bs (:297-308) ; psi_s -= bs_s p_s (:312-322)
-      iz = 1 - iz;
-      for (int s = 0; s < ns; ++s)
-        if (!conv[s]) {
-          const double z0 = z[1 - iz][s], z1 = z[iz][s];
-          z[iz][s] = z0 * z1 * bp / (b * a * (z1 - z0) + z1 * bp * (1.0 - shifts[s] * b));
-          bs[s] = b * z[iz][s] / z0;
-          nbs[s] = -bs[s];
-        }
-      put(op, MS_NBS, nbs.data(), ns);
-      for (int s = 0; s < ns; ++s)
-        if (!conv[s]) op.blas(B_AXPY, {psi[s].get(), pv[s].get()}, MS_NBS + s);
-      // per-shift test on the shifted residual estimate c z_s^2 (:326-339)
-      convP = true;
-      for (int s = 0; s < ns; ++s) {
-        if (!conv[s]) conv[s] = c * z[iz][s] * z[iz][s] < rsd_sq[s];
-        convP = convP && conv[s];
-      }
-      n_count = k;
-      if (p.verbose) std::printf("MInvCG2: k = %d |r| = %g\n", k, std::sqrt(c));
     }
+    n_count = op.hF[F_NCOUNT];
+    if (p.verbose && n_count > 0) std::printf("MInvCG2: k = %d |r| = %g\n", n_count, std::sqrt(h.c));
+    ms_finish(L, op.stream);
   }
   CMX_HIP(hipEventRecord(e1, op.stream));
   CMX_HIP(hipEventSynchronize(e1));
   float ms = 0;
   CMX_HIP(hipEventElapsedTime(&ms, e0, e1));
   // FP64 residual of every shifted system: |chi - (M^dag M + shift_s) psi_s|
+  std::memcpy(op.hS + MS_SIG, shifts, sizeof(double) * ns);
+  CMX_HIP(hipMemcpyAsync(static_cast<double*>(op.state_S.p) + MS_SIG, op.hS + MS_SIG, sizeof(double) * ns,
+                         hipMemcpyHostToDevice, op.stream));
   for (int s = 0; s < ns; ++s) {
-    op.apply(P64, mp.view(), psi[s]->view(), +1, nullptr);
+    const Vec x = psi_of(s);
+    op.apply(P64, mp.view(), x.view(), +1, nullptr);
     op.apply(P64, mmp.view(), mp.view(), -1, nullptr);
-    put(op, MS_SIG, &shifts[s], 1);
-    op.blas(B_AXPY, {&mmp, psi[s].get()}, MS_SIG);
+    op.blas(B_AXPY, {&mmp, &x}, MS_SIG + s);
     op.blas(B_XMY_NORM, {&r, &chi, &mmp});
-    op.finalize(nb, 1, PG_STORE, MS_C);
-    const double rr = get(op, MS_C);
+    op.finalize(nb, 1, PG_STORE, MS_RES + s);
+  }
+  CMX_HIP(hipMemcpyAsync(op.hS + MS_RES, static_cast<double*>(op.state_S.p) + MS_RES, sizeof(double) * ns,
+                         hipMemcpyDeviceToHost, op.stream));
+  op.sync();
+  for (int s = 0; s < ns; ++s) {
     cmx_solver_result& q = res[s];
     std::memset(&q, 0, sizeof(q));
     q.n_count = n_count;
-    q.resid = std::sqrt(rr);
+    q.resid = std::sqrt(op.hS[MS_RES + s]);
     q.rel_resid = chi_norm_sq > 0 ? q.resid / std::sqrt(chi_norm_sq) : q.resid;
     q.solve_seconds = ms * 1e-3;
-    op.unpack(psi_h + (size_t)s * 24 * n, n, *psi[s]);
+    op.unpack(psi_h + (size_t)s * 24 * n, n, psi_of(s));
   }
   const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   for (int s = 0; s < ns; ++s) res[s].total_seconds = wall;
