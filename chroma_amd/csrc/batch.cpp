@@ -42,6 +42,7 @@ void record_fin(Recorder& r, const FinLaunch& f) { r.recs.push_back(make_rec(REC
 
 void BatchPlan::build(const std::vector<Recorder>& recs) {
   st_.clear();
+  mem_.clear();
   CMX_REQUIRE(!recs.empty(), CMX_ERR_ARG, "batch: no problems");
   // problems whose launches select the same kernels share batched grids; others get their own
   std::vector<std::vector<Recorder>> groups;
@@ -66,6 +67,24 @@ void BatchPlan::build(const std::vector<Recorder>& recs) {
 void BatchPlan::add_group(const std::vector<Recorder>& recs) {
   const size_t ns = recs[0].recs.size();
   const int np = (int)recs.size();
+  // all stages' records and maps go to the device in one copy; stages with the same work-group counts share
+  // a map
+  std::vector<unsigned char> blob;
+  auto place = [&](const void* p, size_t n) {
+    const size_t at = (blob.size() + 255) & ~(size_t)255;
+    blob.resize(at + n);
+    std::memcpy(blob.data() + at, p, n);
+    return at;
+  };
+  struct MapAt {
+    bool hop;
+    std::vector<int> nb;
+    size_t at;
+    int n;
+  };
+  std::vector<MapAt> maps;
+  std::vector<size_t> tab_at(ns), map_at(ns, (size_t)-1);
+  const size_t first = st_.size();
   for (size_t j = 0; j < ns; ++j) {
     const LaunchRec& r0 = recs[0].recs[j];
     Stage s;
@@ -81,6 +100,9 @@ void BatchPlan::add_group(const std::vector<Recorder>& recs) {
     std::vector<unsigned char> tab;
     tab.reserve(r0.bytes.size() * np);
     std::vector<int4> map;
+    const MapAt* known = nullptr;
+    for (const MapAt& m : maps)
+      if (s.kind != REC_FIN && m.hop == (s.kind == REC_HOP) && m.nb == s.nb) known = &m;
     int maxnb = 0;
     for (int p = 0; p < np; ++p) {
       const LaunchRec& r = recs[p].recs[j];
@@ -89,11 +111,11 @@ void BatchPlan::add_group(const std::vector<Recorder>& recs) {
                   "batch: stage " + std::to_string(j) + " selects a different kernel for problem " + std::to_string(p) +
                       " (launch shape, precision or epilogue)");
       tab.insert(tab.end(), r.bytes.begin(), r.bytes.end());
-      if (s.kind == REC_BLAS)
+      if (s.kind == REC_BLAS && !known)
         for (int b = 0; b < r.nblocks; ++b) map.push_back(make_int4(p, b, r.nblocks, 0));
       maxnb = std::max(maxnb, r.nblocks);
     }
-    if (s.kind == REC_HOP) {
+    if (s.kind == REC_HOP && !known) {
       // Hopping stages interleave the problems in runs of 8 work-groups: the work-groups of every
       // problem over the same 8 local blocks follow each other, and global work-group g lands on XCD
       // g mod 8 = local block mod 8.  Problems on one gauge field (the sources of a propagator) then
@@ -110,14 +132,26 @@ void BatchPlan::add_group(const std::vector<Recorder>& recs) {
           }
         }
     }
-    s.nblocks = s.kind == REC_FIN ? np : (int)map.size();
-    s.tab.alloc(tab.size());
-    CMX_HIP(hipMemcpy(s.tab.p, tab.data(), tab.size(), hipMemcpyHostToDevice));
-    if (!map.empty()) {
-      s.map.alloc(sizeof(int4) * map.size());
-      CMX_HIP(hipMemcpy(s.map.p, map.data(), sizeof(int4) * map.size(), hipMemcpyHostToDevice));
+    tab_at[j] = place(tab.data(), tab.size());
+    if (s.kind == REC_FIN) {
+      s.nblocks = np;
+    } else if (known) {
+      s.nblocks = known->n;
+      map_at[j] = known->at;
+    } else {
+      s.nblocks = (int)map.size();
+      map_at[j] = place(map.data(), sizeof(int4) * map.size());
+      maps.push_back(MapAt{s.kind == REC_HOP, s.nb, map_at[j], s.nblocks});
     }
     st_.push_back(std::move(s));
+  }
+  mem_.emplace_back(new DevScratch(blob.size()));
+  char* base = mem_.back()->as<char>();
+  host_to_device(base, blob.data(), blob.size(), 0);
+  CMX_HIP(hipStreamSynchronize(0));
+  for (size_t j = 0; j < ns; ++j) {
+    st_[first + j].tab = base + tab_at[j];
+    if (map_at[j] != (size_t)-1) st_[first + j].map = reinterpret_cast<const int4*>(base + map_at[j]);
   }
 }
 
@@ -149,7 +183,7 @@ void BatchPlan::refresh(const std::vector<Recorder>& recs, hipStream_t strm) {
     unsigned char* h = static_cast<unsigned char*>(s.htab.get());
     for (int p = 0; p < np; ++p) std::memcpy(h + rb * p, recs[p].recs[j].bytes.data(), rb);
     s.rec0 = recs[0].recs[j].bytes;
-    CMX_HIP(hipMemcpyAsync(s.tab.p, h, bytes, hipMemcpyHostToDevice, strm));
+    CMX_HIP(hipMemcpyAsync(s.tab, h, bytes, hipMemcpyHostToDevice, strm));
   }
 }
 
@@ -162,7 +196,7 @@ long BatchPlan::blocks() const {
 void BatchPlan::run(hipStream_t strm) const {
   CMX_REQUIRE(active_recorder() == nullptr, CMX_ERR_ARG, "batch: replay while recording");
   for (const Stage& s : st_) {
-    const BatchGrid bg{s.tab.p, s.map.as<int4>(), s.nblocks};
+    const BatchGrid bg{s.tab, s.map, s.nblocks};
     switch (s.kind) {
       case REC_HOP: {
         HopLaunch h;
@@ -177,7 +211,7 @@ void BatchPlan::run(hipStream_t strm) const {
         break;
       }
       default:
-        launch_finalize_batch(s.tab.as<FinLaunch>(), s.nprob, strm);
+        launch_finalize_batch(static_cast<const FinLaunch*>(s.tab), s.nprob, strm);
         break;
     }
   }

@@ -62,12 +62,14 @@ class BatchPlan {
     int prec[4] = {0, 0, 0, 0};
     int nprob = 0, nblocks = 0;
     std::vector<unsigned char> rec0;  // the first problem's record: selects the kernel
-    DevBuf tab, map;
+    void* tab = nullptr;              // in the group's memory
+    const int4* map = nullptr;
     int key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     std::vector<int> nb;              // work-groups of each problem's own launch
     std::shared_ptr<void> htab;       // pinned staging of the records (refresh)
   };
   std::vector<Stage> st_;
+  std::vector<std::unique_ptr<DevScratch>> mem_;  // launch records and work-group maps, one block per group
 };
 
 }  // namespace cmx

@@ -26,7 +26,8 @@ enum Slot {
 };
 // Flags (ints)
 enum Flag {
-  F_DONE = 0,   // iteration kernels return immediately once set
+  F_DONE = 0,   // iteration kernels return immediately while set: the solve has stopped, or (reliable solvers)
+                // waits for its FP64 update (F_UPDR), which clears it
   F_CONV,       // converged (or stopped); copied into F_DONE by the next finalize
   F_NCOUNT,     // iteration count at convergence
   F_K,          // iterations completed
@@ -46,18 +47,20 @@ enum Prog {
   PG_CG_D,           // after |M p|^2: F_DONE = F_CONV; d; a = c/d; -a
   PG_CG_R,           // after r -= a A p, |r|^2: k++, convergence, b = cp/c, c = cp
   PG_RCG_INIT,       // reliable CG start: r_sq, rNorm = r0Norm = maxrx = maxrr
-  PG_RCG_D,          // F_DONE = F_CONV; d; a = c/d
-  PG_RCG_R,          // r_sq, rNorm, maxrx/maxrr, updateX/updateR decision, convergence if no update
-  PG_RCG_UPD,        // after the FP64 reliable update: r_sq, rNorm, maxrr, (r0Norm, maxrx), convergence
+  PG_RCG_D,          // d; a = c/d
+  PG_RCG_R,          // r_sq, rNorm, maxrx/maxrr, updateX/updateR decision: hold for the update, or k++, beta,
+                     // convergence
+  PG_RCG_UPD,        // after the FP64 reliable update (F_UPDR): r_sq, rNorm, maxrr, (r0Norm, maxrx); ends the
+                     // hold; k++, beta, convergence
   PG_BICG_RHO,       // rho = <r0,r>; breakdown test; beta = (rho/rho_prev)(alpha/omega)
   PG_BICG_ALPHA,     // ctmp = <r0,v>; alpha = rho/ctmp; rho_prev = rho
   PG_BICG_OMEGA,     // |t|^2, <t,r>: omega = <t,r>/|t|^2
   PG_BICG_R,         // |r|^2: k++, convergence
   // reliable BiCGStab (reliable_bicgstab.cc:14-290)
   PG_RBICG_INIT,     // after b = chi - A psi: r_sq, norms, rho = r_sq, rho_prev = alpha = omega = 1, beta = 0
-  PG_RBICG_ALPHA,    // F_DONE = F_CONV; ctmp = <r0,v>; alpha = rho/ctmp; rho_prev = rho
-  PG_RBICG_R,        // |r|^2, rho = <r0,r>: updateX / updateR; without an update: k++, convergence, beta
-  PG_RBICG_UPD,      // after the FP64 update of r: r_sq, norms; k++, convergence, beta
+  PG_RBICG_ALPHA,    // ctmp = <r0,v>; alpha = rho/ctmp; rho_prev = rho
+  PG_RBICG_R,        // |r|^2, rho = <r0,r>: updateX / updateR: hold for the update, or k++, convergence, beta
+  PG_RBICG_UPD,      // after the FP64 update of r: r_sq, norms; ends the hold; k++, convergence, beta
   // MR (invmr.cc:100-160), run with the F_MRDONE skip flag
   PG_MR_INIT,        // cp = |r|^2; rsd_sq = RsdMR^2 |v|^2; F_MRDONE = cp <= rsd_sq
   PG_MR_A,           // d = |Mr|^2, c = <Mr, r>: a = omega c / d
@@ -149,6 +152,8 @@ struct FinLaunch {
   int prog, slot;
 };
 void launch_finalize(const FinLaunch& L, hipStream_t s);
+// out[F_NFLAGS * i ..] = the flags of problem i, i < n: one read-back for a batch
+void launch_gather_flags(const int* const* flags, int n, int* out, hipStream_t s);
 // one finalize per problem: tab is a device array of nproblems records
 void launch_finalize_batch(const FinLaunch* tab, int nproblems, hipStream_t s);
 

@@ -320,6 +320,21 @@ void dispatch(const BlasLaunch& b, const int p[4], hipStream_t s, const BatchGri
 }
 
 // ------------------------------------------------------------------------------------------------
+// the end of a reliable CG iteration (reliable_cg.cc:150-170)
+__device__ __forceinline__ void rcg_end(double* S, int* F) {
+  const int k = F[F_K];
+  F[F_K] = k + 1;
+  S[S_BETA] = S[S_RSQ] / S[S_C];
+  if (S[S_RSQ] < S[S_RSDSQ]) {
+    F[F_CONV] = F[F_DONE] = 1;
+    F[F_NCOUNT] = k;
+  } else if (k + 1 >= F[F_MAXIT] || !isfinite(S[S_RSQ])) {
+    F[F_CONV] = F[F_DONE] = 1;
+    F[F_NCOUNT] = k + 1;
+    F[F_ERR] = CMX_ERR_NOCONV;
+  }
+}
+
 __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
   const double* partials = L.partials;
   const int nb = L.nb, nred = L.nred, prog = L.prog, slot = L.slot;
@@ -403,7 +418,6 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       break;
     }
     case PG_RCG_D: {  // reliable_cg.cc:84-96: c = r_sq; d = |mp|^2; a = c/d
-      F[F_DONE] = F[F_CONV];
       if (F[F_DONE]) break;
       S[S_C] = S[S_RSQ];
       S[S_D] = red[0];
@@ -429,31 +443,26 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       const int updR = (rn < S[S_DELTA] * S[S_MAXRR] && S[S_R0NORM] <= S[S_MAXRR]) || updX;
       F[F_UPDX] = updX;
       F[F_UPDR] = updR;
-      if (updR) F[F_NUPD]++;
+      if (updR) {  // the host launches the FP64 update, then PG_RCG_UPD finishes the iteration
+        F[F_NUPD]++;
+        F[F_DONE] = 1;
+        break;
+      }
+      rcg_end(S, F);
       break;
     }
     case PG_RCG_UPD: {  // reliable_cg.cc:120-170 (update part, then the convergence test)
-      if (F[F_DONE]) break;
-      if (F[F_UPDR]) {
-        S[S_RSQ] = red[0];
-        S[S_RNORM] = sqrt(red[0]);
-        S[S_MAXRR] = S[S_RNORM];
-        if (F[F_UPDX]) {
-          S[S_R0NORM] = S[S_RNORM];
-          S[S_MAXRX] = S[S_RNORM];
-        }
+      if (!F[F_UPDR]) break;
+      S[S_RSQ] = red[0];
+      S[S_RNORM] = sqrt(red[0]);
+      S[S_MAXRR] = S[S_RNORM];
+      if (F[F_UPDX]) {
+        S[S_R0NORM] = S[S_RNORM];
+        S[S_MAXRX] = S[S_RNORM];
       }
-      const int k = F[F_K];
-      F[F_K] = k + 1;
-      S[S_BETA] = S[S_RSQ] / S[S_C];
-      if (S[S_RSQ] < S[S_RSDSQ]) {
-        F[F_CONV] = 1;
-        F[F_NCOUNT] = k;
-      } else if (k + 1 >= F[F_MAXIT] || !isfinite(S[S_RSQ])) {
-        F[F_CONV] = 1;
-        F[F_NCOUNT] = k + 1;
-        F[F_ERR] = CMX_ERR_NOCONV;
-      }
+      F[F_UPDR] = 0;
+      F[F_DONE] = 0;
+      rcg_end(S, F);
       break;
     }
     case PG_BICG_RHO: {  // invbicgstab.cc:72-95
@@ -544,7 +553,6 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       break;
     }
     case PG_RBICG_ALPHA: {  // reliable_bicgstab.cc:135-150
-      F[F_DONE] = F[F_CONV];
       if (F[F_DONE]) break;
       const double cr = red[0], ci = red[1];
       if (cr == 0.0 && ci == 0.0) {
@@ -564,7 +572,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
     }
     case PG_RBICG_R:      // reliable_bicgstab.cc:199-214
     case PG_RBICG_UPD: {  // reliable_bicgstab.cc:216-271
-      if (F[F_DONE]) break;
+      if (prog == PG_RBICG_R ? F[F_DONE] : !F[F_UPDR]) break;
       if (prog == PG_RBICG_R) {
         S[S_RSQ] = red[0];
         S[S_RHO] = red[1];
@@ -579,6 +587,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
         F[F_UPDR] = updR;
         if (updR) {  // the host launches the FP64 update, then PG_RBICG_UPD finishes the iteration
           F[F_NUPD]++;
+          F[F_DONE] = 1;
           break;
         }
       } else {  // r = b - A x in FP64 (rho keeps the value from the sloppy r, as the reference does)
@@ -589,16 +598,18 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
           S[S_R0NORM] = S[S_RNORM];
           S[S_MAXRX] = S[S_RNORM];
         }
+        F[F_UPDR] = 0;
+        F[F_DONE] = 0;
       }
       const int k = F[F_K];
       F[F_K] = k + 1;
       if (S[S_RSQ] < S[S_RSDSQ]) {
-        F[F_CONV] = 1;
+        F[F_CONV] = F[F_DONE] = 1;
         F[F_NCOUNT] = k;
         break;
       }
       if (k + 1 >= F[F_MAXIT] || !isfinite(S[S_RSQ])) {
-        F[F_CONV] = 1;
+        F[F_CONV] = F[F_DONE] = 1;
         F[F_NCOUNT] = k + 1;
         F[F_ERR] = CMX_ERR_NOCONV;
         break;
@@ -648,6 +659,9 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
 }
 
 __global__ void __launch_bounds__(256) k_finalize(FinLaunch L) { finalize_body(L); }
+__global__ void __launch_bounds__(256) k_gather_flags(const int* const* __restrict__ flags, int n, int* out) {
+  for (int t = threadIdx.x; t < n * F_NFLAGS; t += 256) out[t] = flags[t / F_NFLAGS][t % F_NFLAGS];
+}
 // one work-group per problem
 __global__ void __launch_bounds__(256) k_finalize_b(const FinLaunch* __restrict__ tab) { finalize_body(tab[blockIdx.x]); }
 
@@ -699,6 +713,9 @@ void launch_blas(int op, const BlasLaunch& b, const int prec[4], hipStream_t s, 
 }
 
 void launch_finalize(const FinLaunch& L, hipStream_t s) { hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, L); }
+void launch_gather_flags(const int* const* flags, int n, int* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_gather_flags, dim3(1), dim3(256), 0, s, flags, n, out);
+}
 void launch_finalize_batch(const FinLaunch* tab, int nproblems, hipStream_t s) {
   hipLaunchKernelGGL(k_finalize_b, dim3(nproblems), dim3(256), 0, s, tab);
 }

@@ -210,8 +210,12 @@ std::shared_ptr<GaugeData> make_gauge(const int dims[4], const double* const lin
 Op::~Op() {
   for (auto& e : graphs) (void)hipGraphExecDestroy(e.exec);
   if (stream && !shared_stream) (void)hipStreamDestroy(stream);
-  if (hS) (void)hipHostFree(hS);
-  if (hF) (void)hipHostFree(hF);
+  if (shared_stream) {
+    pinned_give(hS);
+  } else {
+    if (hS) (void)hipHostFree(hS);
+    if (hF) (void)hipHostFree(hF);
+  }
 }
 
 Op* make_op(std::shared_ptr<GaugeData> gd, const cmx_op_params& p) {
@@ -249,7 +253,7 @@ Op* make_op(std::shared_ptr<GaugeData> gd, const cmx_op_params& p) {
   op->state_S.alloc(sizeof(double) * S_NSLOTS);
   op->state_F.alloc(sizeof(int) * F_NFLAGS);
   CMX_HIP(hipHostMalloc((void**)&op->hS, sizeof(double) * S_NSLOTS, 0));
-  CMX_HIP(hipHostMalloc((void**)&op->hF, sizeof(int) * F_NFLAGS, 0));
+  CMX_HIP(hipHostMalloc((void**)&op->hF, sizeof(int) * 2 * F_NFLAGS, 0));
   op->staging.alloc(sizeof(double) * 24 * op->V);
   if (op->clover()) {
     // QDPCloverTermT::create (clover_term_qdp_w.h:244-294): coefficients x 1/2; planes
@@ -313,11 +317,14 @@ Op* clone_op(Op& o, int prec) {
   c->stream = o.stream;
   c->shared_stream = true;
   c->npartials = o.npartials;
-  c->partials.alloc(sizeof(double) * c->npartials);
-  c->state_S.alloc(sizeof(double) * S_NSLOTS);
-  c->state_F.alloc(sizeof(int) * F_NFLAGS);
-  CMX_HIP(hipHostMalloc((void**)&c->hS, sizeof(double) * S_NSLOTS, 0));
-  CMX_HIP(hipHostMalloc((void**)&c->hF, sizeof(int) * F_NFLAGS, 0));
+  // a clone lives for one batched call: its buffers come from the scratch cache, its mirrors of the scalars
+  // and flags share a cached pinned block
+  c->partials.alloc_scratch(sizeof(double) * c->npartials);
+  c->state_S.alloc_scratch(sizeof(double) * S_NSLOTS);
+  c->state_F.alloc_scratch(sizeof(int) * F_NFLAGS);
+  static_assert(sizeof(double) * S_NSLOTS + sizeof(int) * 2 * F_NFLAGS <= PINNED_BLOCK, "pinned block too small");
+  c->hS = static_cast<double*>(pinned_take());
+  c->hF = reinterpret_cast<int*>(c->hS + S_NSLOTS);
   c->staging.alias(o.staging);
   c->mg = o.mg;  // the multigrid state is read-only in a solve, but for its coarse work space (one stream)
   return c.release();
@@ -345,7 +352,7 @@ Vec& Op::work(int slot, int prec, int n) {
   if ((int)ws.size() <= slot) ws.resize(slot + 1);
   auto& v = ws[slot];
   if (!v || v->prec != prec || v->n != n) {
-    v.reset(new Vec(prec, n));
+    v.reset(new Vec(prec, n, shared_stream));
     ++ws_gen;
   }
   return *v;
@@ -353,7 +360,7 @@ Vec& Op::work(int slot, int prec, int n) {
 
 Vec& Op::tmp(int prec, int k) {
   auto& v = tmp_even[prec];
-  while ((int)v.size() <= k) v.emplace_back(new Vec(prec, (int)Vh));
+  while ((int)v.size() <= k) v.emplace_back(new Vec(prec, (int)Vh, shared_stream));
   return *v[k];
 }
 

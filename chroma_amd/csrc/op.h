@@ -1,5 +1,6 @@
 // Device-resident operator state behind the cmx_gauge / cmx_op handles.
 #pragma once
+#include <exception>
 #include <memory>
 #include <string>
 #include <vector>
@@ -11,7 +12,6 @@
 
 namespace cmx {
 
-// Owning device allocation
 // Owning device allocation (or, after alias(), a non-owning view of another one)
 struct DevBuf {
   void* p = nullptr;
@@ -21,20 +21,30 @@ struct DevBuf {
   explicit DevBuf(size_t n) { alloc(n); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), own(o.own) { o.p = nullptr, o.bytes = 0, o.own = true; }
+  DevBuf(DevBuf&& o) noexcept { take(o); }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
       release();
-      p = o.p, bytes = o.bytes, own = o.own;
-      o.p = nullptr, o.bytes = 0, o.own = true;
+      take(o);
     }
     return *this;
   }
   ~DevBuf() { release(); }
   void alloc(size_t n) {
     release();
-    if (n) CMX_HIP(hipMalloc(&p, n));
+    if (n && hipMalloc(&p, n) != hipSuccess) {
+      (void)hipGetLastError();
+      xfer_release();  // cached scratch may be what is missing
+      CMX_HIP(hipMalloc(&p, n));
+    }
     bytes = n;
+  }
+  // from the scratch cache; work on it must have completed when it is released
+  void alloc_scratch(size_t n) {
+    release();
+    p = scratch_take(n, cap_, dev_);
+    bytes = n;
+    scratch_ = true;
   }
   // refers to o's memory without owning it (o must outlive this buffer)
   void alias(const DevBuf& o) {
@@ -42,10 +52,24 @@ struct DevBuf {
     p = o.p, bytes = o.bytes, own = false;
   }
   void release() {
-    if (p && own) (void)hipFree(p);
-    p = nullptr, bytes = 0, own = true;
+    if (p && own) {
+      if (scratch_ && std::uncaught_exceptions() == 0)
+        scratch_give(p, cap_, dev_);
+      else
+        (void)hipFree(p);
+    }
+    p = nullptr, bytes = 0, own = true, scratch_ = false;
   }
   template <typename T> T* as() const { return static_cast<T*>(p); }
+
+ private:
+  void take(DevBuf& o) {
+    p = o.p, bytes = o.bytes, own = o.own, scratch_ = o.scratch_, cap_ = o.cap_, dev_ = o.dev_;
+    o.p = nullptr, o.bytes = 0, o.own = true, o.scratch_ = false;
+  }
+  bool scratch_ = false;
+  size_t cap_ = 0;
+  int dev_ = 0;
 };
 
 // A fermion vector over n sites (one checkerboard, or a full lattice stored even-then-odd)
@@ -54,7 +78,12 @@ struct Vec {
   int prec = P64;
   int n = 0;
   Vec() = default;
-  Vec(int prec_, int n_) : prec(prec_), n(n_) { buf.alloc(spinor_bytes(prec_, n_)); }
+  Vec(int prec_, int n_, bool scratch = false) : prec(prec_), n(n_) {
+    if (scratch)
+      buf.alloc_scratch(spinor_bytes(prec_, n_));
+    else
+      buf.alloc(spinor_bytes(prec_, n_));
+  }
   float* nrm() const {
     return prec == P16 ? reinterpret_cast<float*>(buf.as<char>() + (size_t)spinor_chunks(prec) * 16 * n) : nullptr;
   }
@@ -116,7 +145,7 @@ struct Op {
   int npartials = 0;
   DevBuf state_S, state_F;
   double* hS = nullptr;  // pinned mirrors
-  int* hF = nullptr;
+  int* hF = nullptr;     // two snapshots of the flags
   DevBuf staging;        // V*24 doubles
   std::vector<std::unique_ptr<Vec>> tmp_even[3];  // scratch even-checkerboard vectors
   // solver workspace kept across solves (so that captured iteration graphs stay valid), and the

@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -162,6 +163,53 @@ int run_batches(Op& op, const cmx_solver_params& p, long tag, const Vec& psi, co
     if (p.check_every <= 0 && batch < 32) batch *= 2;
   }
   return op.hF[F_NCOUNT];
+}
+
+// The iterations of a reliable solver.  The device decides after each whether its FP64 update is due and then
+// holds (F_DONE with F_UPDR: the next iterations' kernels return at once) until update() has run, so the
+// host needs the flags only to launch the update.  On small lattices it reads them one iteration behind the
+// launches, which keeps the device busy over the read-back (15 to 20 us of a 60 to 90 us iteration); the
+// one iteration queued behind a held one exits at once.  On large ones such an exit costs more (20 us per
+// launch of 16384 work-groups, against an iteration of 0.5 ms) and the host waits for each iteration.
+template <typename Inner, typename Update, typename Say>
+void run_held(Op& op, const cmx_solver_params& p, Inner&& inner, Update&& update, Say&& say) {
+  const bool ahead = op.subset_sites() <= 200000 && !p.verbose;
+  struct Ev {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    ~Ev() {
+      for (hipEvent_t x : e)
+        if (x) (void)hipEventDestroy(x);
+    }
+  } ev;
+  for (hipEvent_t& e : ev.e) CMX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  long issued = 0;
+  auto issue = [&]() {
+    inner();
+    const int q = (int)(issued++ & 1);
+    CMX_HIP(hipMemcpyAsync(op.hF + q * F_NFLAGS, op.state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost,
+                           op.stream));
+    if (p.verbose)
+      CMX_HIP(hipMemcpyAsync(op.hS, op.state_S.p, sizeof(double) * 40, hipMemcpyDeviceToHost, op.stream));
+    CMX_HIP(hipEventRecord(ev.e[q], op.stream));
+  };
+  issue();
+  for (long seen = 0;; ++seen) {
+    if (ahead && issued == seen + 1) issue();
+    CMX_HIP(hipEventSynchronize(ev.e[seen & 1]));
+    CMX_HIP(hipGetLastError());
+    const int* f = op.hF + (seen & 1) * F_NFLAGS;
+    if (p.verbose) {
+      if (f != op.hF) std::memcpy(op.hF, f, sizeof(int) * F_NFLAGS);
+      say();
+    }
+    if (f[F_DONE]) {
+      if (!f[F_UPDR]) break;  // converged or stopped
+      update(f[F_UPDX] != 0);
+      seen = issued - 1;  // an iteration queued meanwhile held too: its flags say nothing new
+    }
+    if (issued > 2L * p.max_iter + 8) break;  // the device stops itself at MaxIter
+    if (issued == seen + 1) issue();
+  }
 }
 
 double flops_per_apply(const Op& op) {
@@ -320,20 +368,20 @@ struct RelCGState {
     op.blas(B_AXPY2_NORM, {&x, &r, &pv, &mmp}, S_A, 0, F_DONE);                             // x += a p; r -= a mmp
     op.finalize(nb, 1, PG_RCG_R);                                                           // updateX / updateR
   }
-  // r = b - A^dag A x in FP64 (reliable_cg.cc:120-136)
-  void update_r(int skip, int run) {
+  // The FP64 update of an iteration that holds for it: r = b - A^dag A x (reliable_cg.cc:120-136), the norms
+  // and the convergence test, and (F_UPDX) psi += x; x = 0; b = r.  gated: every launch asks the flags (a
+  // batch, where only some problems hold); else the host has seen that the update is due.
+  void update(bool gated, bool updx) {
     int* F = op.state_F.as<int>();
-    op.blas(B_COPY, {&x_dble, &x}, 0, 0, skip, run);
-    op.apply(P64, tmp1.view(), x_dble.view(), +1, nullptr, skip >= 0 ? F + skip : nullptr, run >= 0 ? F + run : nullptr);
-    op.apply(P64, tmp2.view(), tmp1.view(), -1, nullptr, skip >= 0 ? F + skip : nullptr, run >= 0 ? F + run : nullptr);
-    op.blas(B_XMY_NORM_COPY, {&r_dble, &b, &tmp2, &r}, 0, 0, skip, run);
-  }
-  // The update step with the decisions taken on the device: the FP64 kernels run when the flags ask
-  // for them and return at once otherwise (same arithmetic as the host-decided step)
-  void update_gated() {
-    update_r(F_DONE, F_UPDR);
-    op.finalize(nb, 1, PG_RCG_UPD);                                                         // norms, convergence
-    op.blas(B_ADD_ZERO_COPY, {&psi, &x, &b, &r_dble}, 0, 0, F_DONE, F_UPDX);                // psi += x; x = 0; b = r
+    const int run = gated ? F_UPDR : -1;
+    const int* runp = gated ? F + F_UPDR : nullptr;
+    op.blas(B_COPY, {&x_dble, &x}, 0, 0, -1, run);
+    op.apply(P64, tmp1.view(), x_dble.view(), +1, nullptr, nullptr, runp);
+    op.apply(P64, tmp2.view(), tmp1.view(), -1, nullptr, nullptr, runp);
+    op.blas(B_XMY_NORM_COPY, {&r_dble, &b, &tmp2, &r}, 0, 0, -1, run);
+    op.finalize(nb, 1, PG_RCG_UPD);
+    // a converged solve keeps its last x: psi += x follows at the end in any case
+    if (gated || updx) op.blas(B_ADD_ZERO_COPY, {&psi, &x, &b, &r_dble}, 0, 0, F_DONE, F_UPDX);
   }
   void finish(double seconds, cmx_solver_result& res) {
     res.n_count = op.hF[F_NCOUNT];
@@ -350,30 +398,21 @@ void solve_relcg(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& chi, b
   RelCGState st(op, p, psi, chi, mdagm);
   Timer tm(op.stream);
   st.setup(&tm);
-  // One host synchronisation per iteration: the flags of the updateR / updateX decision are read
-  // back, and the FP64 reliable-update kernels are launched only when the device asks for them
-  // (an early-exit launch of a full-lattice grid costs tens of microseconds, more than the read-back).
-  long launched = 0;
   GraphCache gc(op, p.graph != 0, 3 + 10 * st.ps + (mdagm ? 100 : 0), psi, chi);
-  auto inner = [&]() { st.inner(); };
-  while (true) {
-    if (launched == 0)
-      inner();  // eager: performs the lazy allocations of the operator's scratch vectors
-    else
-      gc.run(0, inner);
-    CMX_HIP(hipMemcpyAsync(op.hF, op.state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, op.stream));
-    if (p.verbose)
-      CMX_HIP(hipMemcpyAsync(op.hS, op.state_S.p, sizeof(double) * 16, hipMemcpyDeviceToHost, op.stream));
-    op.sync();
-    if (p.verbose)  // reliable_cg.cc:108-110
-      std::printf("RelCG: k = %d  r_sq = %.6e  d = %.6e  a = %.6e  updateR %d updateX %d err %d\n", op.hF[F_K],
-                  op.hS[S_RSQ], op.hS[S_D], op.hS[S_A], op.hF[F_UPDR], op.hF[F_UPDX], op.hF[F_ERR]);
-    if (op.hF[F_DONE]) break;  // converged (or stopped) in the previous iteration
-    if (op.hF[F_UPDR]) st.update_r(-1, -1);
-    op.finalize(st.nb, 1, PG_RCG_UPD);                                                      // norms, convergence
-    if (op.hF[F_UPDX]) op.blas(B_ADD_ZERO_COPY, {&psi, &st.x, &st.b, &st.r_dble});          // psi += x; x = 0; b = r
-    if (++launched > (long)p.max_iter + 4) break;                                           // device stops at MaxIter
-  }
+  long launched = 0;
+  run_held(
+      op, p,
+      [&] {
+        if (launched++ == 0)
+          st.inner();  // eager: performs the lazy allocations of the operator's scratch vectors
+        else
+          gc.run(0, [&] { st.inner(); });
+      },
+      [&](bool updx) { st.update(false, updx); },
+      [&] {  // reliable_cg.cc:108-110
+        std::printf("RelCG: k = %d  r_sq = %.6e  d = %.6e  a = %.6e  updateR %d updateX %d err %d\n", op.hF[F_K],
+                    op.hS[S_RSQ], op.hS[S_D], op.hS[S_A], op.hF[F_UPDR], op.hF[F_UPDX], op.hF[F_ERR]);
+      });
   op.blas(B_ADD, {&psi, &st.x});                                                            // psi += x (reliable_cg.cc:158-163)
   read_state(op);
   st.finish(tm.stop(), res);
@@ -408,36 +447,31 @@ void solve_relbicgstab(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& 
   op.blas(B_ZERO, {&x});
   op.blas(B_ZERO, {&pv});
   op.blas(B_ZERO, {&v});
-  long launched = 0;
-  while (true) {
-    op.blas(B_BICG_P, {&pv, &r, &v}, S_OMEGA, S_BETAC);                        // p = r + beta (p - omega v)
-    op.apply(ps, v.view(), pv.view(), isign, nullptr);                         // v = A p
-    op.blas(B_CDOT, {&r0, &v});
-    op.finalize(nb, 2, PG_RBICG_ALPHA);                                        // alpha = rho / <r0|v>
-    op.blas(B_CAXPY2, {&r, &v, &x, &pv}, S_NALPHA, S_ALPHA, F_DONE);           // s = r - alpha v; x += alpha p
-    op.apply(ps, t.view(), r.view(), isign, nullptr, F + F_DONE);              // t = A s
-    op.blas(B_TNORM_TDOT, {&t, &r}, 0, 0, F_DONE);
-    op.finalize(nb, 3, PG_BICG_OMEGA);                                         // omega = <t|s> / |t|^2
-    op.blas(B_RBICG_UPDATE, {&x, &r, &t, &r0}, S_OMEGA, 0, F_DONE);            // x += omega s; r = s - omega t
-    op.finalize(nb, 3, PG_RBICG_R);                                            // updateX / updateR
-    CMX_HIP(hipMemcpyAsync(op.hF, op.state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, op.stream));
-    op.sync();
-    if (op.hF[F_DONE] || op.hF[F_ERR]) break;  // breakdown inside this iteration
-    if (op.hF[F_UPDR]) {                       // r = b - A x in FP64 (:216-256)
-      op.blas(B_COPY, {&x_dble, &x});
-      op.apply(P64, tmp.view(), x_dble.view(), isign, nullptr);
-      op.blas(B_XMY_NORM_COPY, {&r_dble, &b, &tmp, &r});
-      op.finalize(nb, 1, PG_RBICG_UPD);
-      if (op.hF[F_UPDX]) op.blas(B_ADD_ZERO_COPY, {&psi, &x, &b, &r_dble});  // psi += x; x = 0; b = r
-      CMX_HIP(hipMemcpyAsync(op.hF, op.state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, op.stream));
-      op.sync();
-    }
-    if (op.hF[F_CONV]) break;
-    if (++launched > (long)p.max_iter + 4) break;  // the device stops at MaxIter
-  }
+  run_held(
+      op, p,
+      [&] {
+        op.blas(B_BICG_P, {&pv, &r, &v}, S_OMEGA, S_BETAC, F_DONE);                // p = r + beta (p - omega v)
+        op.apply(ps, v.view(), pv.view(), isign, nullptr, F + F_DONE);             // v = A p
+        op.blas(B_CDOT, {&r0, &v}, 0, 0, F_DONE);
+        op.finalize(nb, 2, PG_RBICG_ALPHA);                                        // alpha = rho / <r0|v>
+        op.blas(B_CAXPY2, {&r, &v, &x, &pv}, S_NALPHA, S_ALPHA, F_DONE);           // s = r - alpha v; x += alpha p
+        op.apply(ps, t.view(), r.view(), isign, nullptr, F + F_DONE);              // t = A s
+        op.blas(B_TNORM_TDOT, {&t, &r}, 0, 0, F_DONE);
+        op.finalize(nb, 3, PG_BICG_OMEGA);                                         // omega = <t|s> / |t|^2
+        op.blas(B_RBICG_UPDATE, {&x, &r, &t, &r0}, S_OMEGA, 0, F_DONE);            // x += omega s; r = s - omega t
+        op.finalize(nb, 3, PG_RBICG_R);                                            // updateX / updateR
+      },
+      [&](bool updx) {  // r = b - A x in FP64 (:216-256)
+        op.blas(B_COPY, {&x_dble, &x});
+        op.apply(P64, tmp.view(), x_dble.view(), isign, nullptr);
+        op.blas(B_XMY_NORM_COPY, {&r_dble, &b, &tmp, &r});
+        op.finalize(nb, 1, PG_RBICG_UPD);
+        if (updx) op.blas(B_ADD_ZERO_COPY, {&psi, &x, &b, &r_dble}, 0, 0, F_DONE);  // psi += x; x = 0; b = r
+      },
+      [] {});
   op.blas(B_ADD, {&psi, &x});  // psi += x (:259-266)
-  res.n_count = op.hF[F_NCOUNT];
   read_state(op);
+  res.n_count = op.hF[F_NCOUNT];
   res.solve_seconds = tm.stop();
   res.n_reliable = op.hF[F_NUPD];
   res.gflops = (res.n_count + 1) * (2 * flops_per_apply(op) + 80 * 12.0 * n) / std::max(res.solve_seconds, 1e-12) * 1e-9;
@@ -517,17 +551,20 @@ void true_residual(Op& op, const Vec& psi, const Vec& chi, bool mdagm, cmx_solve
 // each later kernel.
 namespace {
 
-// candidate launch shapes for a batch: the plane-grid kernel needs it admitted on every lattice
+// candidate launch shapes for a batch: the plane-grid and direction-split kernels need to be admitted on
+// every lattice
 std::vector<HopConfig> batch_candidates(const std::vector<Op*>& ops, int ps) {
-  bool fast_ok = ps != P64;
+  bool fast_ok = true, split_ok = true;
   for (Op* o : ops) {
     HopLaunch h = o->hop_base(ps);
     HopConfig c;
-    c.fast = 1;
+    c.fast = 1 | HOP_SPLIT;
     hop_apply_config(h, c);
     if (!(h.fast & 1)) fast_ok = false;
+    if (!(h.fast & HOP_SPLIT)) split_ok = false;
   }
   std::vector<HopConfig> c;
+  if (split_ok) c.push_back(HopConfig{64, 0, 1, 0, 1 | HOP_SPLIT});
   for (int block : {64, 128, 256}) {
     c.push_back(HopConfig{block, 0, 1, 0, 0});
     c.push_back(HopConfig{block, 0, 1, 0, HOP_FAST_STREAM});
@@ -537,6 +574,50 @@ std::vector<HopConfig> batch_candidates(const std::vector<Op*>& ops, int ps) {
     }
   }
   return c;
+}
+
+// what the best shape of a batch depends on
+std::string batch_key(const std::vector<Op*>& ops, int ps) {
+  std::string k = "p" + std::to_string(ps);
+  for (size_t i = 0; i < ops.size(); ++i) {
+    size_t j = 0;
+    while (ops[j]->gd != ops[i]->gd) ++j;  // the first problem on the same gauge field
+    HopLaunch h = ops[i]->hop_base(ps);
+    HopConfig c;
+    c.fast = 1;
+    hop_apply_config(h, c);
+    k += "|" + std::to_string(ops[i]->par.kind) + "," + std::to_string(h.recon) + "," + std::to_string(h.fast & 1) + "," +
+         std::to_string(j);
+    for (int mu = 0; mu < 4; ++mu) k += "," + std::to_string(h.g.L[mu]);
+  }
+  return k;
+}
+
+// the tuned shapes of the last 64 batch make-ups
+class BatchShapes {
+ public:
+  bool get(const std::string& key, HopConfig& c) {
+    std::lock_guard<std::mutex> lk(m_);
+    for (const auto& e : v_)
+      if (e.first == key) {
+        c = e.second;
+        return true;
+      }
+    return false;
+  }
+  void put(const std::string& key, const HopConfig& c) {
+    std::lock_guard<std::mutex> lk(m_);
+    if (v_.size() >= 64) v_.erase(v_.begin());
+    v_.emplace_back(key, c);
+  }
+
+ private:
+  std::mutex m_;
+  std::vector<std::pair<std::string, HopConfig>> v_;
+};
+BatchShapes& batch_shapes() {
+  static BatchShapes s;
+  return s;
 }
 
 }  // namespace
@@ -893,8 +974,17 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
   }
 
   // launch shape: timed candidates (one batched operator application of every problem), or the
-  // operators' own
-  if (bp.tune) {
+  // operators' own.  A batch of the same make-up (kinds, lattices, admitted kernels and which problems share
+  // a gauge field) as an earlier one takes that one's shape: timing a dozen candidates takes some 0.2 s,
+  // ten times the twelve 16^3x32 solves themselves.
+  const std::string shape_key = bp.tune ? batch_key(ops, ps) : std::string();
+  HopConfig known;
+  if (bp.tune && batch_shapes().get(shape_key, known)) {
+    for (Op* o : ops) {
+      o->ensure_prec(ps);
+      o->hcfg[ps][0] = known;
+    }
+  } else if (bp.tune) {
     std::vector<std::unique_ptr<Vec>> va, vb, vc;
     for (Op* o : ops) {
       const int n = o->subset_sites();
@@ -943,6 +1033,7 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     (void)hipEventDestroy(e1);
     for (Op* o : ops) o->hcfg[ps][0] = bestc;
     CMX_HIP(hipStreamSynchronize(s0));
+    batch_shapes().put(shape_key, bestc);
   }
   if (!bp.tune) {
     // Shapes that depend on the volumes alone may differ (the plan batches each kernel's problems apart);
@@ -982,27 +1073,56 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
       }
     }
     for (int i : act) ops[i]->sync();
-    // one iteration per problem, recorded (the reliable update in its flag-gated form)
-    std::vector<Recorder> recs(na);
+    // one iteration per problem, recorded, and (reliable CG) its FP64 update in the flag-gated form
+    std::vector<Recorder> recs(na), upds(rel ? na : 0);
     for (int k = 0; k < na; ++k) {
-      RecordScope rs(recs[k]);
+      {
+        RecordScope rs(recs[k]);
+        if (rel)
+          rcg[k]->inner();
+        else
+          cg[k]->iter();
+      }
       if (rel) {
-        rcg[k]->inner();
-        rcg[k]->update_gated();
-      } else {
-        cg[k]->iter();
+        RecordScope rs(upds[k]);
+        rcg[k]->update(true, false);
       }
     }
-    // replay until every problem has stopped (the device stops each at its MaxIter); the problems
-    // that have stopped leave the batched grid at the next check
-    std::vector<int> live(na);
+    // replay until every problem has stopped (the device stops each at its MaxIter); problems that have
+    // stopped leave the batched grids once a quarter of them has
+    std::vector<int> live(na), in_plan;
     for (int k = 0; k < na; ++k) live[k] = k;
-    BatchPlan plan;
+    BatchPlan plan, uplan;
+    DevScratch fptr(sizeof(int*) * na), fdev(sizeof(int) * F_NFLAGS * na);
+    struct Pinned {
+      int* p = nullptr;
+      ~Pinned() {
+        if (p) (void)hipHostFree(p);
+      }
+    } fhost;
+    CMX_HIP(hipHostMalloc((void**)&fhost.p, sizeof(int) * F_NFLAGS * na * 2, 0));
+    hipGraphExec_t gx = nullptr;
+    int gx_len = 0;
+    auto drop_graph = [&]() {
+      if (gx) (void)hipGraphExecDestroy(gx);
+      gx = nullptr;
+    };
     auto rebuild = [&]() {
       std::vector<Recorder> sub;
-      sub.reserve(live.size());
-      for (int k : live) sub.push_back(recs[k]);
+      std::vector<const int*> fp;
+      for (int k : live) {
+        sub.push_back(recs[k]);
+        fp.push_back(ops[act[k]]->state_F.as<int>());
+      }
+      drop_graph();
       plan.build(sub);
+      if (rel) {
+        sub.clear();
+        for (int k : live) sub.push_back(upds[k]);
+        uplan.build(sub);
+      }
+      CMX_HIP(hipMemcpy(fptr.get(), fp.data(), sizeof(int*) * fp.size(), hipMemcpyHostToDevice));
+      in_plan = live;
     };
     rebuild();
     if (restart == 0) {
@@ -1013,49 +1133,93 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     for (int i : act) maxit = std::max(maxit, q[i].max_iter);
     Timer tm(s0);
     tm.start();
-    int batch = p.check_every > 0 ? p.check_every : 4;
     long launched = 0;
-    hipGraphExec_t gx = nullptr;
-    int gx_len = 0;
-    auto drop_graph = [&]() {
-      if (gx) (void)hipGraphExecDestroy(gx);
-      gx = nullptr;
-    };
-    try {
-      while (true) {
-        if (bp.graph && launched > 0) {
-          if (!gx || gx_len != batch) {
-            drop_graph();
-            hipGraph_t gr = nullptr;
-            CMX_HIP(hipStreamBeginCapture(s0, hipStreamCaptureModeThreadLocal));
-            for (int j = 0; j < batch; ++j) plan.run(s0);
-            CMX_HIP(hipStreamEndCapture(s0, &gr));
-            const hipError_t e = hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(gr);
-            CMX_HIP(e);
-            gx_len = batch;
-          }
-          CMX_HIP(hipGraphLaunch(gx, s0));
-        } else {
-          for (int j = 0; j < batch; ++j) plan.run(s0);
-        }
-        launched += batch;
-        for (int k : live) {
-          Op* o = ops[act[k]];
-          CMX_HIP(hipMemcpyAsync(o->hF, o->state_F.p, sizeof(int) * F_NFLAGS, hipMemcpyDeviceToHost, s0));
-        }
-        CMX_HIP(hipStreamSynchronize(s0));
-        std::vector<int> still;
-        for (int k : live)
-          if (!ops[act[k]]->hF[F_CONV]) still.push_back(k);
-        if (still.empty() || launched > (long)maxit + 8) break;
-        if (still.size() < live.size()) {
-          live = still;
+    // `count` iterations of the problems in the plan
+    auto iterate = [&](int count) {
+      if (bp.graph && launched > 0) {
+        if (!gx || gx_len != count) {
           drop_graph();
-          rebuild();
+          hipGraph_t gr = nullptr;
+          CMX_HIP(hipStreamBeginCapture(s0, hipStreamCaptureModeThreadLocal));
+          for (int j = 0; j < count; ++j) plan.run(s0);
+          CMX_HIP(hipStreamEndCapture(s0, &gr));
+          const hipError_t e = hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0);
+          (void)hipGraphDestroy(gr);
+          CMX_HIP(e);
+          gx_len = count;
         }
-        if (p.check_every <= 0 && batch < 32) batch *= 2;
+        CMX_HIP(hipGraphLaunch(gx, s0));
+      } else {
+        for (int j = 0; j < count; ++j) plan.run(s0);
       }
+      launched += count;
+    };
+    // snapshot q of the flags of the problems in the plan
+    auto flags = [&](int q) {
+      const int n = (int)in_plan.size();
+      launch_gather_flags(fptr.as<const int*>(), n, fdev.as<int>(), s0);
+      CMX_HIP(hipMemcpyAsync(fhost.p + (size_t)q * F_NFLAGS * na, fdev.get(), sizeof(int) * F_NFLAGS * n,
+                             hipMemcpyDeviceToHost, s0));
+    };
+    auto retire = [&](const int* f) {  // live without the stopped ones; true when all have stopped
+      std::vector<int> still;
+      for (size_t j = 0; j < in_plan.size(); ++j) {
+        const int* fj = f + j * F_NFLAGS;
+        if (!(rel ? fj[F_DONE] && !fj[F_UPDR] : fj[F_CONV])) still.push_back(in_plan[j]);
+      }
+      live = still;
+      return live.empty();
+    };
+    struct Ev {
+      hipEvent_t e[2] = {nullptr, nullptr};
+      ~Ev() {
+        for (hipEvent_t x : e)
+          if (x) (void)hipEventDestroy(x);
+      }
+    } ev;
+    try {
+      if (!rel) {
+        int batch = p.check_every > 0 ? p.check_every : 4;
+        while (true) {
+          iterate(batch);
+          flags(0);
+          CMX_HIP(hipStreamSynchronize(s0));
+          if (retire(fhost.p) || launched > (long)maxit + 8) break;
+          if (4 * live.size() <= 3 * in_plan.size()) rebuild();
+          if (p.check_every <= 0 && batch < 32) batch *= 2;
+        }
+      } else {
+        // as run_held: a problem holds at an iteration whose FP64 update is due; the flags are read one
+        // iteration behind the launches, and the gated update runs when some problem holds
+        for (hipEvent_t& e : ev.e) CMX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        bool stale = false;  // the coming snapshot precedes an update that covers all that hold in it
+        auto issue = [&](long j) {
+          iterate(1);
+          flags((int)(j & 1));
+          CMX_HIP(hipEventRecord(ev.e[j & 1], s0));
+        };
+        issue(0);
+        for (long j = 0;; ++j) {
+          issue(j + 1);
+          CMX_HIP(hipEventSynchronize(ev.e[j & 1]));
+          const int* f = fhost.p + (size_t)(j & 1) * F_NFLAGS * na;
+          bool due = false;
+          for (size_t x = 0; x < in_plan.size(); ++x) due = due || (f[x * F_NFLAGS + F_DONE] && f[x * F_NFLAGS + F_UPDR]);
+          due = due && !stale;
+          if (due) uplan.run(s0);
+          stale = due;
+          if (retire(f) || launched > 2L * maxit + 8) break;
+          if (4 * live.size() <= 3 * in_plan.size()) {
+            // the iteration in flight belongs to the old plan: its flags are not read
+            CMX_HIP(hipStreamSynchronize(s0));
+            rebuild();
+            stale = false;
+            issue(j + 2);
+            ++j;
+          }
+        }
+      }
+      CMX_HIP(hipGetLastError());
     } catch (...) {
       drop_graph();
       throw;

@@ -221,7 +221,8 @@ struct Cached {
   size_t cap;
   int dev;
 };
-constexpr size_t CACHE_MAX = (size_t)1 << 30;  // device bytes the scratch cache keeps at most
+// device bytes and buffers the scratch cache keeps at most
+constexpr size_t CACHE_MAX = (size_t)4 << 30, CACHE_ENTRIES = 1024;
 
 struct Pool {
   std::mutex m;
@@ -230,6 +231,7 @@ struct Pool {
   std::vector<int> made;  // lanes per device
   std::vector<Cached> cache;
   size_t cached = 0;
+  std::vector<void*> pinned;
 };
 // never destroyed: its threads may outlive static destruction
 Pool& pool() {
@@ -311,51 +313,97 @@ void device_to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
   CMX_HIP(hipStreamSynchronize(s));
 }
 
-DevScratch::DevScratch(size_t bytes) : bytes_(bytes), throwing_(std::uncaught_exceptions()) {
-  CMX_HIP(hipGetDevice(&dev_));
-  if (!bytes) return;
+void* scratch_take(size_t bytes, size_t& cap, int& dev) {
+  CMX_HIP(hipGetDevice(&dev));
+  cap = 0;
+  if (!bytes) return nullptr;
   Pool& P = pool();
   {
     std::lock_guard<std::mutex> lk(P.m);
     size_t best = P.cache.size();
     for (size_t k = 0; k < P.cache.size(); ++k) {
       const Cached& c = P.cache[k];
-      if (c.dev == dev_ && c.cap >= bytes && c.cap <= 2 * bytes + (1 << 20) &&
+      if (c.dev == dev && c.cap >= bytes && c.cap <= bytes + bytes / 4 + 65536 &&
           (best == P.cache.size() || c.cap < P.cache[best].cap))
         best = k;
     }
     if (best < P.cache.size()) {
-      p_ = P.cache[best].p, cap_ = P.cache[best].cap;
-      P.cached -= cap_;
-      P.cache.erase(P.cache.begin() + (long)best);
+      const Cached c = P.cache[best];
+      cap = c.cap;
+      P.cached -= cap;
+      P.cache[best] = P.cache.back();
+      P.cache.pop_back();
+      return c.p;
+    }
+  }
+  cap = bytes;
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  xfer_release();  // the cached buffers may be what is missing
+  CMX_HIP(hipMalloc(&p, bytes));
+  return p;
+}
+
+void scratch_give(void* p, size_t cap, int dev) {
+  if (!p) return;
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lk(P.m);
+    if (P.cached + cap <= CACHE_MAX && P.cache.size() < CACHE_ENTRIES) {
+      P.cache.push_back(Cached{p, cap, dev});
+      P.cached += cap;
       return;
     }
   }
-  cap_ = bytes;
-  if (hipMalloc(&p_, bytes) == hipSuccess) return;
-  (void)hipGetLastError();
-  xfer_release();  // the cached buffers may be what is missing
-  CMX_HIP(hipMalloc(&p_, bytes));
+  (void)hipFree(p);
+}
+
+void* pinned_take() {
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lk(P.m);
+    if (!P.pinned.empty()) {
+      void* p = P.pinned.back();
+      P.pinned.pop_back();
+      return p;
+    }
+  }
+  void* p = nullptr;
+  CMX_HIP(hipHostMalloc(&p, PINNED_BLOCK, 0));
+  return p;
+}
+
+void pinned_give(void* p) {
+  if (!p) return;
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lk(P.m);
+    if (P.pinned.size() < 128) {
+      P.pinned.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
+}
+
+DevScratch::DevScratch(size_t bytes) : bytes_(bytes), throwing_(std::uncaught_exceptions()) {
+  p_ = scratch_take(bytes, cap_, dev_);
 }
 
 DevScratch::~DevScratch() {
   if (!p_) return;
-  Pool& P = pool();
-  if (std::uncaught_exceptions() == throwing_) {  // an error may leave work queued: hipFree waits for it
-    std::lock_guard<std::mutex> lk(P.m);
-    if (P.cached + cap_ <= CACHE_MAX) {
-      P.cache.push_back(Cached{p_, cap_, dev_});
-      P.cached += cap_;
-      return;
-    }
-  }
-  (void)hipFree(p_);
+  if (std::uncaught_exceptions() == throwing_)
+    scratch_give(p_, cap_, dev_);
+  else
+    (void)hipFree(p_);  // an error may leave work queued: hipFree waits for it
 }
 
 void xfer_release() {
   Pool& P = pool();
   std::vector<Lane*> lanes;
   std::vector<Cached> cache;
+  std::vector<void*> pinned;
   {
     std::lock_guard<std::mutex> lk(P.m);
     if (P.pid == getpid()) {
@@ -364,9 +412,11 @@ void xfer_release() {
     }
     cache.swap(P.cache);
     P.cached = 0;
+    pinned.swap(P.pinned);
   }
   for (Lane* l : lanes) delete l;
   for (const Cached& c : cache) (void)hipFree(c.p);
+  for (void* p : pinned) (void)hipHostFree(p);
 }
 
 }  // namespace cmx

@@ -15,6 +15,15 @@ void device_to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
 // Gives back the pinned staging buffers, the copy threads and the cached scratch that no call is using
 void xfer_release();
 
+// Device memory from the bounded cache of earlier calls' buffers (cap: its size, dev: its device), and back
+// to it; work on a buffer that is given back must have completed
+void* scratch_take(size_t bytes, size_t& cap, int& dev);
+void scratch_give(void* p, size_t cap, int dev);
+// Small pinned host blocks (PINNED_BLOCK bytes), cached likewise
+constexpr size_t PINNED_BLOCK = 8192;
+void* pinned_take();
+void pinned_give(void* p);
+
 // Device memory of one call, from a bounded cache of earlier calls' buffers.  The caller's work on it must
 // have completed (stream synchronised) when the object goes out of scope.
 class DevScratch {
