@@ -38,6 +38,12 @@ void record_blas(Recorder& r, int op, const BlasLaunch& b, const int prec[4]) {
   r.recs.push_back(std::move(x));
 }
 
+static int fin_partials(const LaunchRec& r) {
+  FinLaunch f;
+  std::memcpy(&f, r.bytes.data(), sizeof(f));
+  return f.nb;
+}
+
 void record_fin(Recorder& r, const FinLaunch& f) { r.recs.push_back(make_rec(REC_FIN, f, 1)); }
 
 void BatchPlan::build(const std::vector<Recorder>& recs) {
@@ -135,6 +141,7 @@ void BatchPlan::add_group(const std::vector<Recorder>& recs) {
     tab_at[j] = place(tab.data(), tab.size());
     if (s.kind == REC_FIN) {
       s.nblocks = np;
+      for (int p = 0; p < np; ++p) s.fin_nb = std::max(s.fin_nb, fin_partials(recs[p].recs[j]));
     } else if (known) {
       s.nblocks = known->n;
       map_at[j] = known->at;
@@ -183,6 +190,10 @@ void BatchPlan::refresh(const std::vector<Recorder>& recs, hipStream_t strm) {
     unsigned char* h = static_cast<unsigned char*>(s.htab.get());
     for (int p = 0; p < np; ++p) std::memcpy(h + rb * p, recs[p].recs[j].bytes.data(), rb);
     s.rec0 = recs[0].recs[j].bytes;
+    if (s.kind == REC_FIN) {
+      s.fin_nb = 0;
+      for (int p = 0; p < np; ++p) s.fin_nb = std::max(s.fin_nb, fin_partials(recs[p].recs[j]));
+    }
     CMX_HIP(hipMemcpyAsync(s.tab, h, bytes, hipMemcpyHostToDevice, strm));
   }
 }
@@ -211,7 +222,7 @@ void BatchPlan::run(hipStream_t strm) const {
         break;
       }
       default:
-        launch_finalize_batch(static_cast<const FinLaunch*>(s.tab), s.nprob, strm);
+        launch_finalize_batch(static_cast<const FinLaunch*>(s.tab), s.nprob, s.fin_nb, strm);
         break;
     }
   }

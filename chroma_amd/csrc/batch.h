@@ -61,6 +61,7 @@ class BatchPlan {
     int kind = 0, opc = 0;
     int prec[4] = {0, 0, 0, 0};
     int nprob = 0, nblocks = 0;
+    int fin_nb = 0;                   // most partials of a problem (finalize stages)
     std::vector<unsigned char> rec0;  // the first problem's record: selects the kernel
     void* tab = nullptr;              // in the group's memory
     const int4* map = nullptr;

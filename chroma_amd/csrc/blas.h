@@ -63,6 +63,7 @@ enum Prog {
   PG_RBICG_UPD,      // after the FP64 update of r: r_sq, norms; ends the hold; k++, convergence, beta
   // MR (invmr.cc:100-160), run with the F_MRDONE skip flag
   PG_MR_INIT,        // cp = |r|^2; rsd_sq = RsdMR^2 |v|^2; F_MRDONE = cp <= rsd_sq
+  PG_MR_START,       // without a stopping test: F_MRDONE = 0
   PG_MR_A,           // d = |Mr|^2, c = <Mr, r>: a = omega c / d
   PG_MR_R,           // cp = |r|^2; F_MRDONE = cp <= rsd_sq
 };
@@ -111,6 +112,8 @@ enum BlasOp {
   B_AXPY_CNORM,     // v0 += S[ia] v1 (complex) ; red0 = |v0|^2
   B_AXPBY,          // v0 = S[ia] v1 + S[ib] v0 (real)
   B_MR_UPDATE,      // v0 += S[ia] v1 ; v1 += S[ib] v2 (complex) ; red0 = |v1|^2  (psi += a r ; r -= a M r)
+  B_MR_STEP,        // B_MR_UPDATE without the norm
+  B_XMY,            // v0 = v1 - v2
   B_NOPS
 };
 
@@ -155,6 +158,6 @@ void launch_finalize(const FinLaunch& L, hipStream_t s);
 // out[F_NFLAGS * i ..] = the flags of problem i, i < n: one read-back for a batch
 void launch_gather_flags(const int* const* flags, int n, int* out, hipStream_t s);
 // one finalize per problem: tab is a device array of nproblems records
-void launch_finalize_batch(const FinLaunch* tab, int nproblems, hipStream_t s);
+void launch_finalize_batch(const FinLaunch* tab, int nproblems, int nb_max, hipStream_t s);
 
 }  // namespace cmx

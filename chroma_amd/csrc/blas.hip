@@ -2,6 +2,7 @@
 // The reductions follow the fused kernels of bicgstab_kernels_scalarsite.h:29-742 (one pass that
 // updates a vector and returns its norm) with FP64 accumulation and a deterministic two-stage sum.
 #include <cmath>
+#include <type_traits>
 
 #include "blas.h"
 
@@ -222,7 +223,7 @@ CMX_F(FAxpyCNorm, 1, 3, 1) {
   red[0] += nrm2(v0);
 }
 };
-// the two updates of an MR step in one pass: the same arithmetic as FCaxpy then FAxpyCNorm (v0 is
+// the two updates of an MR step and the norm in one pass (v0 is
 // updated from v1 before v1 changes)
 CMX_F(FMrUpdate, 1, 7, 3) {
   const R ar = (R)S[ia], ai = (R)S[ia + 1], br = (R)S[ib], bi = (R)S[ib + 1];
@@ -235,6 +236,24 @@ CMX_F(FMrUpdate, 1, 7, 3) {
     v1[2 * k + 1] += br * yi + bi * yr;
   }
   red[0] += nrm2(v1);
+}
+};
+// FMrUpdate where nothing reads the norm
+CMX_F(FMrStep, 0, 7, 3) {
+  const R ar = (R)S[ia], ai = (R)S[ia + 1], br = (R)S[ib], bi = (R)S[ib + 1];
+#pragma unroll
+  for (int k = 0; k < 12; ++k) {
+    const R xr = v1[2 * k], xi = v1[2 * k + 1], yr = v2[2 * k], yi = v2[2 * k + 1];
+    v0[2 * k] += ar * xr - ai * xi;
+    v0[2 * k + 1] += ar * xi + ai * xr;
+    v1[2 * k] += br * yr - bi * yi;
+    v1[2 * k + 1] += br * yi + bi * yr;
+  }
+}
+};
+CMX_F(FXmy, 0, 6, 1) {
+#pragma unroll
+  for (int k = 0; k < 24; ++k) v0[k] = v1[k] - v2[k];
 }
 };
 #undef CMX_F
@@ -320,6 +339,8 @@ void dispatch(const BlasLaunch& b, const int p[4], hipStream_t s, const BatchGri
 }
 
 // ------------------------------------------------------------------------------------------------
+constexpr int FIN_THREADS = 1024;
+
 // the end of a reliable CG iteration (reliable_cg.cc:150-170)
 __device__ __forceinline__ void rcg_end(double* S, int* F) {
   const int k = F[F_K];
@@ -340,23 +361,33 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
   const int nb = L.nb, nred = L.nred, prog = L.prog, slot = L.slot;
   double* S = L.S;
   int* F = L.F;
+  // each thread sums partials threadIdx.x, + FIN_THREADS, ... in that order, the sums of an entry side by
+  // side; the loads of four entries are issued before their additions, so that the 5000 to 20000 partials
+  // of a large reduction cost one or two load latencies per sum (with 256 threads and one sum after another
+  // three sums over 5760 partials took 6.6 us)
   double red[3] = {0, 0, 0};
-  for (int r = 0; r < nred; ++r) {
-    // each thread sums partials threadIdx.x, + blockDim.x, ... in that order; the loads of eight terms
-    // are issued before their additions, so the sum waits for one load latency per eight terms (the
-    // partials of a 48^3x96 reduction are 20736 per entry) and the order, hence the result, is unchanged
-    double acc = 0;
-    const int step = blockDim.x;
+  auto sums = [&](auto nr) {
+    constexpr int NR = decltype(nr)::value;
     int k = threadIdx.x;
-    for (; k + 7 * step < nb; k += 8 * step) {
-      double t[8];
+    for (; k + 3 * FIN_THREADS < nb; k += 4 * FIN_THREADS) {
+      double t[4][NR];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) t[j] = partials[(size_t)(k + j * step) * nred + r];
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc += t[j];
+        for (int r = 0; r < NR; ++r) t[j][r] = partials[(size_t)(k + j * FIN_THREADS) * NR + r];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < NR; ++r) red[r] += t[j][r];
     }
-    for (; k < nb; k += step) acc += partials[(size_t)k * nred + r];
-    red[r] = acc;
+    for (; k < nb; k += FIN_THREADS)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) red[r] += partials[(size_t)k * NR + r];
+  };
+  switch (nred) {
+    case 1: sums(std::integral_constant<int, 1>()); break;
+    case 2: sums(std::integral_constant<int, 2>()); break;
+    case 3: sums(std::integral_constant<int, 3>()); break;
   }
   block_sum<3>(red);
   if (threadIdx.x != 0) return;
@@ -634,6 +665,9 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       F[F_MRDONE] = red[0] <= S[S_MR + 11] ? 1 : 0;
       break;
     }
+    case PG_MR_START:
+      F[F_MRDONE] = 0;
+      break;
     case PG_MR_A: {
       if (F[F_MRDONE]) break;
       const double d = red[0], cr = red[1], ci = red[2], w = S[S_MR + 9];
@@ -658,12 +692,12 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
   }
 }
 
-__global__ void __launch_bounds__(256) k_finalize(FinLaunch L) { finalize_body(L); }
+__global__ void __launch_bounds__(FIN_THREADS) k_finalize(FinLaunch L) { finalize_body(L); }
 __global__ void __launch_bounds__(256) k_gather_flags(const int* const* __restrict__ flags, int n, int* out) {
   for (int t = threadIdx.x; t < n * F_NFLAGS; t += 256) out[t] = flags[t / F_NFLAGS][t % F_NFLAGS];
 }
 // one work-group per problem
-__global__ void __launch_bounds__(256) k_finalize_b(const FinLaunch* __restrict__ tab) { finalize_body(tab[blockIdx.x]); }
+__global__ void __launch_bounds__(FIN_THREADS) k_finalize_b(const FinLaunch* __restrict__ tab) { finalize_body(tab[blockIdx.x]); }
 
 }  // namespace
 
@@ -693,7 +727,6 @@ void launch_blas(int op, const BlasLaunch& b, const int prec[4], hipStream_t s, 
     case B_AXPY_NORM: dispatch<FAxpyNorm>(b, prec, s, bg); break;
     case B_AXPY: dispatch<FAxpy>(b, prec, s, bg); break;
     case B_XPAY: dispatch<FXpay>(b, prec, s, bg); break;
-    case B_AXPBY: dispatch<FAxpby>(b, prec, s, bg); break;
     case B_CG_UPDATE: dispatch<FCgUpdate>(b, prec, s, bg); break;
     case B_AXPY2_NORM: dispatch<FAxpy2Norm>(b, prec, s, bg); break;
     case B_ADD_ZERO_COPY: dispatch<FAddZeroCopy>(b, prec, s, bg); break;
@@ -708,16 +741,22 @@ void launch_blas(int op, const BlasLaunch& b, const int prec[4], hipStream_t s, 
     case B_SCALE: dispatch<FScale>(b, prec, s, bg); break;
     case B_AXPY_CNORM: dispatch<FAxpyCNorm>(b, prec, s, bg); break;
     case B_MR_UPDATE: dispatch<FMrUpdate>(b, prec, s, bg); break;
+    case B_AXPBY: dispatch<FAxpby>(b, prec, s, bg); break;
+    case B_MR_STEP: dispatch<FMrStep>(b, prec, s, bg); break;
+    case B_XMY: dispatch<FXmy>(b, prec, s, bg); break;
     default: throw Error(CMX_ERR_ARG, "blas: unknown op");
   }
 }
 
-void launch_finalize(const FinLaunch& L, hipStream_t s) { hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, L); }
+// Up to 256 partials a thread holds one at most, whatever the size of the group, and block_sum adds the
+// waves in order, so that both sizes of group give the same bits and a batch may take its largest problem's.
+static int fin_threads(int nb) { return nb <= 256 ? 256 : FIN_THREADS; }
+void launch_finalize(const FinLaunch& L, hipStream_t s) { hipLaunchKernelGGL(k_finalize, dim3(1), dim3(fin_threads(L.nb)), 0, s, L); }
 void launch_gather_flags(const int* const* flags, int n, int* out, hipStream_t s) {
   hipLaunchKernelGGL(k_gather_flags, dim3(1), dim3(256), 0, s, flags, n, out);
 }
-void launch_finalize_batch(const FinLaunch* tab, int nproblems, hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize_b, dim3(nproblems), dim3(256), 0, s, tab);
+void launch_finalize_batch(const FinLaunch* tab, int nproblems, int nb_max, hipStream_t s) {
+  hipLaunchKernelGGL(k_finalize_b, dim3(nproblems), dim3(fin_threads(nb_max)), 0, s, tab);
 }
 
 }  // namespace cmx

@@ -24,11 +24,21 @@ struct MRPrecond {
     op.hS[S_MR + 10] = rsd;
     CMX_HIP(hipMemcpyAsync(static_cast<double*>(op.state_S.p) + S_MR + 9, op.hS + S_MR + 9, 2 * sizeof(double),
                            hipMemcpyHostToDevice, op.stream));
-    op.blas(B_NORM2, {&v});
-    op.finalize(nb, 1, PG_STORE, S_MR + 7);  // |chi|^2
+    // RsdMR = 0 (the multigrid smoother): the stopping test holds for r = 0 alone, which the next step's
+    // |M r|^2 = 0 detects as well, so the norms of chi and r are left out
+    const bool test = rsd != 0;
+    if (test) {
+      op.blas(B_NORM2, {&v});
+      op.finalize(nb, 1, PG_STORE, S_MR + 7);  // |chi|^2
+    }
     op.apply(ps, mr.view(), z.view(), +1, nullptr);
-    op.blas(B_XMY_NORM, {&r, &v, &mr});      // r = chi - M psi
-    op.finalize(nb, 1, PG_MR_INIT);
+    if (test) {
+      op.blas(B_XMY_NORM, {&r, &v, &mr});      // r = chi - M psi
+      op.finalize(nb, 1, PG_MR_INIT);
+    } else {
+      op.blas(B_XMY, {&r, &v, &mr});
+      op.finalize(0, 0, PG_MR_START);
+    }
     for (int k = 0; k < maxit; ++k) {
       if (op.eo()) {  // M r with |Mr|^2 and <Mr, r> from the operator's second kernel
         const int nh = op.apply(ps, mr.view(), r.view(), +1, op.partials.as<double>(), F + F_MRDONE, nullptr, true);
@@ -38,8 +48,14 @@ struct MRPrecond {
         op.blas(B_TNORM_TDOT, {&mr, &r}, 0, 0, F_MRDONE);               // |Mr|^2, <Mr, r>
         op.finalize(nb, 3, PG_MR_A);                                     // a = omega c / d
       }
-      op.blas(B_MR_UPDATE, {&z, &r, &mr}, S_MR + 3, S_MR + 5, F_MRDONE);  // psi += a r ; r -= a M r
-      op.finalize(nb, 1, PG_MR_R);
+      if (test) {
+        op.blas(B_MR_UPDATE, {&z, &r, &mr}, S_MR + 3, S_MR + 5, F_MRDONE);  // psi += a r ; r -= a M r
+        op.finalize(nb, 1, PG_MR_R);
+      } else if (k + 1 < maxit) {
+        op.blas(B_MR_STEP, {&z, &r, &mr}, S_MR + 3, S_MR + 5, F_MRDONE);
+      } else {
+        op.blas(B_CAXPY, {&z, &r}, S_MR + 3, 0, F_MRDONE);  // nothing reads the last r
+      }
     }
   }
 };
