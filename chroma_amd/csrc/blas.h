@@ -97,20 +97,16 @@ enum BlasOp {
   B_AXPY,           // v0 += S[ia] v1
   B_XPAY,           // v0 = v1 + S[ia] v0
   B_CG_UPDATE,      // v0 += S[ia] v1 ; v1 = v2 + S[ib] v1             (psi, p, r)
-  B_AXPY2_NORM,     // v0 += S[ia] v2 ; v1 -= S[ia] v3 ; red0 = |v1|^2 (x, r, p, Ap)
   B_ADD_ZERO_COPY,  // v0 += v1 ; v1 = 0 ; v2 = v3                   (psi += x_dble; x = 0; b = r_dble)
   B_ADD,            // v0 += v1
   B_CDOT,           // red0,1 = <v0, v1>
   B_BICG_P,         // v0 = v1 + S[ib](v0 - S[ia] v2)                (p = r + beta (p - omega v))
   B_CAXPY,          // v0 += S[ia] v1 (complex)
-  B_TNORM_TDOT,     // red0 = |v0|^2, red1,2 = <v0, v1>
   B_BICG_UPDATE,    // v0 += S[ia] v1 + S[ib] v2 ; v1 -= S[ia] v3 ; red0 = |v1|^2  (psi, r, p, t)
   B_CAXPY2,         // v0 += S[ia] v1 ; v2 += S[ib] v3 (complex)    (r -= alpha v ; x += alpha p)
   B_RBICG_UPDATE,   // v0 += S[ia] v1 ; v1 -= S[ia] v2 ; red0 = |v1|^2, red1,2 = <v3, v1>
                     //                                     (x += omega s ; r = s - omega t ; |r|^2, <r0|r>)
   B_SCALE,          // v0 = S[ia] v1 (real)
-  B_AXPY_CNORM,     // v0 += S[ia] v1 (complex) ; red0 = |v0|^2
-  B_AXPBY,          // v0 = S[ia] v1 + S[ib] v0 (real)
   B_MR_UPDATE,      // v0 += S[ia] v1 ; v1 += S[ib] v2 (complex) ; red0 = |v1|^2  (psi += a r ; r -= a M r)
   B_MR_STEP,        // B_MR_UPDATE without the norm
   B_XMY,            // v0 = v1 - v2

@@ -85,12 +85,6 @@ CMX_F(FXpay, 0, 3, 1) {
   for (int k = 0; k < 24; ++k) v0[k] = v1[k] + a * v0[k];
 }
 };
-CMX_F(FAxpby, 0, 3, 1) {
-  const R a = (R)S[ia], b = (R)S[ib];
-#pragma unroll
-  for (int k = 0; k < 24; ++k) v0[k] = a * v1[k] + b * v0[k];
-}
-};
 CMX_F(FCgUpdate, 0, 7, 3) {
   const R a = (R)S[ia], b = (R)S[ib];
 #pragma unroll
@@ -98,16 +92,6 @@ CMX_F(FCgUpdate, 0, 7, 3) {
     v0[k] += a * v1[k];
     v1[k] = v2[k] + b * v1[k];
   }
-}
-};
-CMX_F(FAxpy2Norm, 1, 15, 3) {
-  const R a = (R)S[ia];
-#pragma unroll
-  for (int k = 0; k < 24; ++k) {
-    v0[k] += a * v2[k];
-    v1[k] -= a * v3[k];
-  }
-  red[0] += nrm2(v1);
 }
 };
 CMX_F(FAddZeroCopy, 0, 11, 7) {
@@ -151,16 +135,6 @@ CMX_F(FCaxpy, 0, 3, 1) {
     const R xr = v1[2 * k], xi = v1[2 * k + 1];
     v0[2 * k] += ar * xr - ai * xi;
     v0[2 * k + 1] += ar * xi + ai * xr;
-  }
-}
-};
-CMX_F(FTnormTdot, 3, 3, 0) {
-#pragma unroll
-  for (int k = 0; k < 12; ++k) {
-    const double ar = v0[2 * k], ai = v0[2 * k + 1], br = v1[2 * k], bi = v1[2 * k + 1];
-    red[0] += ar * ar + ai * ai;
-    red[1] += ar * br + ai * bi;
-    red[2] += ar * bi - ai * br;
   }
 }
 };
@@ -210,17 +184,6 @@ CMX_F(FScale, 0, 2, 1) {
   const R a = (R)S[ia];
 #pragma unroll
   for (int k = 0; k < 24; ++k) v0[k] = a * v1[k];
-}
-};
-CMX_F(FAxpyCNorm, 1, 3, 1) {
-  const R ar = (R)S[ia], ai = (R)S[ia + 1];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) {
-    const R xr = v1[2 * k], xi = v1[2 * k + 1];
-    v0[2 * k] += ar * xr - ai * xi;
-    v0[2 * k + 1] += ar * xi + ai * xr;
-  }
-  red[0] += nrm2(v0);
 }
 };
 // the two updates of an MR step and the norm in one pass (v0 is
@@ -444,6 +407,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       S[S_MAXRX] = S[S_RNORM];
       S[S_MAXRR] = S[S_RNORM];
       S[S_BETA] = 0.0;
+      S[S_A] = 0.0;
       F[F_K] = 0;
       F[F_NUPD] = 0;
       break;
@@ -453,6 +417,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
       S[S_C] = S[S_RSQ];
       S[S_D] = red[0];
       if (!(S[S_D] > 0.0) || !isfinite(S[S_D])) {
+        S[S_A] = 0.0;  // x holds everything
         F[F_ERR] = CMX_ERR_BREAKDOWN;
         F[F_CONV] = 1;
         F[F_DONE] = 1;
@@ -484,6 +449,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
     }
     case PG_RCG_UPD: {  // reliable_cg.cc:120-170 (update part, then the convergence test)
       if (!F[F_UPDR]) break;
+      S[S_A] = 0.0;  // the update added a p to x
       S[S_RSQ] = red[0];
       S[S_RNORM] = sqrt(red[0]);
       S[S_MAXRR] = S[S_RNORM];
@@ -523,7 +489,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
     }
     case PG_BICG_ALPHA: {  // invbicgstab.cc:100-118
       if (F[F_DONE]) break;
-      const double cr = red[0], ci = red[1];
+      const double cr = red[1], ci = red[2];  // red[0] = |v|^2
       if (cr == 0.0 && ci == 0.0) {
         F[F_ERR] = CMX_ERR_BREAKDOWN;
         F[F_CONV] = F[F_DONE] = 1;
@@ -585,7 +551,7 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
     }
     case PG_RBICG_ALPHA: {  // reliable_bicgstab.cc:135-150
       if (F[F_DONE]) break;
-      const double cr = red[0], ci = red[1];
+      const double cr = red[1], ci = red[2];  // red[0] = |v|^2
       if (cr == 0.0 && ci == 0.0) {
         F[F_ERR] = CMX_ERR_BREAKDOWN;
         F[F_CONV] = F[F_DONE] = 1;
@@ -703,12 +669,12 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finalize_b(const FinLaunch* __r
 
 int blas_nred(int op) {
   switch (op) {
-    case B_NORM2: case B_XMY_NORM: case B_XMY_NORM_COPY: case B_AXPY_NORM: case B_AXPY2_NORM: case B_BICG_UPDATE:
-    case B_AXPY_CNORM: case B_MR_UPDATE:
+    case B_NORM2: case B_XMY_NORM: case B_XMY_NORM_COPY: case B_AXPY_NORM: case B_BICG_UPDATE:
+    case B_MR_UPDATE:
       return 1;
     case B_CDOT:
       return 2;
-    case B_TNORM_TDOT: case B_RBICG_UPDATE:
+    case B_RBICG_UPDATE:
       return 3;
     default:
       return 0;
@@ -728,20 +694,16 @@ void launch_blas(int op, const BlasLaunch& b, const int prec[4], hipStream_t s, 
     case B_AXPY: dispatch<FAxpy>(b, prec, s, bg); break;
     case B_XPAY: dispatch<FXpay>(b, prec, s, bg); break;
     case B_CG_UPDATE: dispatch<FCgUpdate>(b, prec, s, bg); break;
-    case B_AXPY2_NORM: dispatch<FAxpy2Norm>(b, prec, s, bg); break;
     case B_ADD_ZERO_COPY: dispatch<FAddZeroCopy>(b, prec, s, bg); break;
     case B_ADD: dispatch<FAdd>(b, prec, s, bg); break;
     case B_CDOT: dispatch<FCdot>(b, prec, s, bg); break;
     case B_BICG_P: dispatch<FBicgP>(b, prec, s, bg); break;
     case B_CAXPY: dispatch<FCaxpy>(b, prec, s, bg); break;
-    case B_TNORM_TDOT: dispatch<FTnormTdot>(b, prec, s, bg); break;
     case B_BICG_UPDATE: dispatch<FBicgUpdate>(b, prec, s, bg); break;
     case B_CAXPY2: dispatch<FCaxpy2>(b, prec, s, bg); break;
     case B_RBICG_UPDATE: dispatch<FRbicgUpdate>(b, prec, s, bg); break;
     case B_SCALE: dispatch<FScale>(b, prec, s, bg); break;
-    case B_AXPY_CNORM: dispatch<FAxpyCNorm>(b, prec, s, bg); break;
     case B_MR_UPDATE: dispatch<FMrUpdate>(b, prec, s, bg); break;
-    case B_AXPBY: dispatch<FAxpby>(b, prec, s, bg); break;
     case B_MR_STEP: dispatch<FMrStep>(b, prec, s, bg); break;
     case B_XMY: dispatch<FXmy>(b, prec, s, bg); break;
     default: throw Error(CMX_ERR_ARG, "blas: unknown op");

@@ -379,7 +379,11 @@ struct HopLaunch {
   int x_stride;
   double a, b;
   double* partials;  // |out|^2 per work-group (nullable)
-  int ndot;          // with partials and an xpay epilogue: |out|^2, Re <out, x>, Im <out, x> per work-group
+  int tail;          // with partials: what the epilogue does with out beyond |out|^2 (HopTail)
+  void* y;           // the vector of TAIL_DOT_Y and TAIL_UPDATE
+  float* y_nrm;
+  int y_stride;
+  const double* coef;  // TAIL_UPDATE
   const int* skip;   // device flag: return immediately when *skip != 0 (nullable)
   const int* run;    // device flag: run only when *run != 0 (nullable)
   // launch shape (chosen by the operator's tuner, see hop_config)
@@ -396,6 +400,19 @@ struct HopLaunch {
   float inv_lxh;     // 1 / (Lx/2), for the fast kernel's plane decomposition
   float inv_ly, inv_lz;  // 1 / Ly, 1 / Lz (direction-split kernel)
   float sgn[4][2];   // real det(U) phase per direction: [bulk | last slice]
+};
+
+// The solver's next vector operation, done on the values that a hopping kernel's epilogue holds: the operator's
+// result then needs no pass of its own, and with TAIL_UPDATE it is never stored.  Small lattices save a launch of
+// 3.6 to 5 us per operation, large ones the bytes: CG on 8^3x16 4.79 -> 4.46 ms (124 iterations), reliable CG in
+// FP16 on 32^3x64 71.3 -> 69.2 ms, twelve batched reliable CG solves on 16^3x32 36.7 -> 33.4 ms.  Each
+// tail is a kernel of its own (67 to 110 VGPRs on the plane grid in FP16; as a branch on the launch record the
+// tails took 126 to 147 and one or two of the four to seven waves per SIMD).
+enum HopTail {
+  TAIL_NONE = 0,    // |out|^2 per work-group
+  TAIL_DOT_X = 1,   // |out|^2, Re <out, x>, Im <out, x> (x: the xpay input)
+  TAIL_DOT_Y = 2,   // |out|^2, Re <y, out>, Im <y, out>; y in the kernel's precision
+  TAIL_UPDATE = 3,  // y += *coef out in place of the store, |y|^2; y in FP64 (FP64 kernel) or FP32 (FP32, FP16)
 };
 
 constexpr int HOP_FAST_STREAM = 2;

@@ -456,7 +456,7 @@ template <typename T> __device__ __forceinline__ void pin_acc(T (&acc)[24]) {
 }
 
 // work-group blk of the launch h
-template <int P, int ISIGN, int EPI, bool NORM, int LCP>
+template <int P, int ISIGN, int EPI, int NORM, int LCP>
 __device__ __forceinline__ void hop_fast_body(const HopLaunch& h, int blk) {
   if (h.skip && *h.skip) return;
   if (h.run && !*h.run) return;
@@ -572,31 +572,25 @@ __device__ __forceinline__ void hop_fast_body(const HopLaunch& h, int blk) {
       const R a = (R)h.a;
 #pragma unroll
       for (int k = 0; k < 24; ++k) out[k] = fmar(a, xs[k], b * acc[k]);
-      if constexpr (NORM)
-        if (h.ndot) out_dot_x(out, xs, dre, dim);
+      if constexpr (NORM == NORM_DOT_X) out_dot_x(out, xs, dre, dim);
     } else {
       R xs[24];
       SpinorIO<P>::template load<LCP>(h.x, h.x_nrm, h.x_stride, i, xs);
       clover_apply_site<P, LCP>(h.clov, Vh, i, xs, out);
 #pragma unroll
       for (int k = 0; k < 24; ++k) out[k] = fmar(b, acc[k], out[k]);
-      if constexpr (NORM)
-        if (h.ndot) out_dot_x(out, xs, dre, dim);
+      if constexpr (NORM == NORM_DOT_X) out_dot_x(out, xs, dre, dim);
     }
-    SpinorIO<P>::store(h.out, h.out_nrm, h.out_stride, i, out);
-    if constexpr (NORM) {
-#pragma unroll
-      for (int k = 0; k < 24; ++k) nsq += (double)out[k] * (double)out[k];
-    }
+    hop_finish<P, NORM>(h, i, out, nsq, dre, dim);
   }
-  if constexpr (NORM) write_norm_partials(h, blk, nsq, dre, dim);
+  if constexpr (NORM) write_norm_partials<NORM>(h, blk, nsq, dre, dim);
 }
 
-template <int P, int ISIGN, int EPI, bool NORM, int LCP>
+template <int P, int ISIGN, int EPI, int NORM, int LCP>
 __global__ void __launch_bounds__(256) k_hop_fast(HopLaunch h) {
   hop_fast_body<P, ISIGN, EPI, NORM, LCP>(h, blockIdx.x);
 }
-template <int P, int ISIGN, int EPI, bool NORM, int LCP>
+template <int P, int ISIGN, int EPI, int NORM, int LCP>
 __global__ void __launch_bounds__(256) k_hop_fast_b(const HopLaunch* __restrict__ tab, const int4* __restrict__ map) {
   const int4 m = map[blockIdx.x];
   if (m.x < 0) return;  // alignment padding of the batched grid
@@ -609,7 +603,7 @@ template <int P> void launch_hop_fast_t(const HopLaunch& h, hipStream_t s, const
     throw Error(CMX_ERR_UNSUPPORTED, "plane-grid hopping kernel: field above 2 GiB (32-bit buffer offsets)");
   const int Pl = h.g.Lxh * h.g.L[1];
   const dim3 grid(((Pl + h.block - 1) / h.block) * h.g.L[2] * h.g.L[3]);
-  const bool norm = h.partials != nullptr;
+  const int norm = hop_norm(h);
   const bool lnt = (h.fast & HOP_FAST_STREAM) != 0;
 #define CMX_HOPF_GO(IS, EP, NM, CP)                                                             \
   if (bg)                                                                                       \
@@ -625,13 +619,30 @@ template <int P> void launch_hop_fast_t(const HopLaunch& h, hipStream_t s, const
   }
 #define CMX_HOPF_CASE(IS, EP)                                                                   \
   if (h.isign == IS && h.epi == EP) {                                                           \
-    if (norm) {                                                                                 \
-      CMX_HOPF_NT(IS, EP, true)                                                                 \
+    if (norm == NORM_ONLY) {                                                                    \
+      CMX_HOPF_NT(IS, EP, NORM_ONLY)                                                            \
     } else {                                                                                    \
-      CMX_HOPF_NT(IS, EP, false)                                                                \
+      CMX_HOPF_NT(IS, EP, NORM_NONE)                                                            \
     }                                                                                           \
     return;                                                                                     \
   }
+#define CMX_HOPF_TAIL(IS, EP, NM)                                                               \
+  if (h.isign == IS && h.epi == EP && norm == NM) {                                             \
+    CMX_HOPF_NT(IS, EP, NM)                                                                     \
+    return;                                                                                     \
+  }
+  CMX_HOPF_TAIL(-1, EPI_XPAY, NORM_UPDATE)
+  CMX_HOPF_TAIL(-1, EPI_CLOV_XPAY, NORM_UPDATE)
+  CMX_HOPF_TAIL(1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOPF_TAIL(1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOPF_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOPF_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_Y)
+  CMX_HOPF_TAIL(-1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOPF_TAIL(-1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOPF_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOPF_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_Y)
+#undef CMX_HOPF_TAIL
+  if (norm > NORM_ONLY) throw Error(CMX_ERR_ARG, "launch_hop_fast: tail not instantiated");
   CMX_HOPF_CASE(1, EPI_NONE)
   CMX_HOPF_CASE(1, EPI_CLOV)
   CMX_HOPF_CASE(1, EPI_XPAY)

@@ -433,10 +433,45 @@ __device__ __forceinline__ void out_dot_x(const R (&out)[24], const R (&xs)[24],
     dim += orr * xi - oi * xr;
   }
 }
-// the work-group's reductions: |out|^2 (h.partials[blk]), or with h.ndot |out|^2, Re <out, x>, Im <out, x>
+// what a kernel computes beside its result: the HopTail that the launch asks for, as the template argument NORM
+enum HopNorm { NORM_NONE = 0, NORM_ONLY, NORM_DOT_X, NORM_DOT_Y, NORM_UPDATE };
+inline int hop_norm(const HopLaunch& h) {
+  if (!h.partials) return NORM_NONE;
+  static_assert(NORM_DOT_X == NORM_ONLY + TAIL_DOT_X && NORM_UPDATE == NORM_ONLY + TAIL_UPDATE, "HopTail order");
+  return NORM_ONLY + h.tail;
+}
+// The store of one site and its contribution to the reductions.  Norms are of the values computed (below
+// the storage rounding; FP64 accumulation).
+template <int P, int NORM, typename R>
+__device__ __forceinline__ void hop_finish(const HopLaunch& h, int i, R (&out)[24], double& nsq, double& dre, double& dim) {
+  if constexpr (NORM == NORM_UPDATE) {
+    constexpr int PY = P == P64 ? P64 : P32;
+    R y[24];
+    const R c = (R)*h.coef;
+    SpinorIO<PY>::load(h.y, nullptr, h.y_stride, i, y);
+#pragma unroll
+    for (int k = 0; k < 24; ++k) y[k] += c * out[k];
+    SpinorIO<PY>::store(h.y, nullptr, h.y_stride, i, y);
+#pragma unroll
+    for (int k = 0; k < 24; ++k) nsq += (double)y[k] * (double)y[k];
+  } else {
+    if constexpr (NORM == NORM_DOT_Y) {
+      R y[24];
+      SpinorIO<P>::load(h.y, h.y_nrm, h.y_stride, i, y);
+      out_dot_x(y, out, dre, dim);
+    }
+    SpinorIO<P>::store(h.out, h.out_nrm, h.out_stride, i, out);
+    if constexpr (NORM) {
+#pragma unroll
+      for (int k = 0; k < 24; ++k) nsq += (double)out[k] * (double)out[k];
+    }
+  }
+}
+// the work-group's reductions: |out|^2 or |y|^2 (h.partials[blk]), or with a dot product the three sums
 // (h.partials[3 blk + 0..2], the layout the finalize kernel reads for three reductions)
+template <int NORM>
 __device__ __forceinline__ void write_norm_partials(const HopLaunch& h, int blk, double nsq, double dre, double dim) {
-  if (h.ndot) {
+  if constexpr (NORM == NORM_DOT_X || NORM == NORM_DOT_Y) {
     double v[3] = {nsq, dre, dim};
     block_sum<3>(v);
     if (threadIdx.x == 0) {
@@ -451,7 +486,7 @@ __device__ __forceinline__ void write_norm_partials(const HopLaunch& h, int blk,
   }
 }
 
-template <int P, int RECON, int ISIGN, int EPI, bool NORM, bool PF, int LCP>
+template <int P, int RECON, int ISIGN, int EPI, int NORM, bool PF, int LCP>
 __device__ __forceinline__ void hop_body(const HopLaunch& h, int blk, int nblk) {
   using R = typename SpinorIO<P>::R;
   if (h.skip && *h.skip) return;
@@ -510,32 +545,25 @@ __device__ __forceinline__ void hop_body(const HopLaunch& h, int blk, int nblk) 
       const R a = R(h.a);
 #pragma unroll
       for (int k = 0; k < 24; ++k) out[k] = a * xs[k] + b * acc[k];
-      if constexpr (NORM)
-        if (h.ndot) out_dot_x(out, xs, dre, dim);
+      if constexpr (NORM == NORM_DOT_X) out_dot_x(out, xs, dre, dim);
     } else {
       R xs[24];
       SpinorIO<P>::template load<LCP>(h.x, h.x_nrm, h.x_stride, i, xs);
       clover_apply_site<P, LCP>(h.clov, h.g.Vh, i, xs, out);
 #pragma unroll
       for (int k = 0; k < 24; ++k) out[k] += b * acc[k];
-      if constexpr (NORM)
-        if (h.ndot) out_dot_x(out, xs, dre, dim);
+      if constexpr (NORM == NORM_DOT_X) out_dot_x(out, xs, dre, dim);
     }
-    SpinorIO<P>::store(h.out, h.out_nrm, h.out_stride, i, out);
-    if constexpr (NORM) {
-      // |out|^2 of the values computed (below the FP16 storage rounding; FP64 accumulation)
-#pragma unroll
-      for (int k = 0; k < 24; ++k) nsq += (double)out[k] * (double)out[k];
-    }
+    hop_finish<P, NORM>(h, i, out, nsq, dre, dim);
   }
-  if constexpr (NORM) write_norm_partials(h, blk, nsq, dre, dim);
+  if constexpr (NORM) write_norm_partials<NORM>(h, blk, nsq, dre, dim);
 }
 
-template <int P, int RECON, int ISIGN, int EPI, bool NORM, bool PF, int LCP>
+template <int P, int RECON, int ISIGN, int EPI, int NORM, bool PF, int LCP>
 __global__ void __launch_bounds__(256) k_hop(HopLaunch h) {
   hop_body<P, RECON, ISIGN, EPI, NORM, PF, LCP>(h, blockIdx.x, gridDim.x);
 }
-template <int P, int RECON, int ISIGN, int EPI, bool NORM, bool PF, int LCP>
+template <int P, int RECON, int ISIGN, int EPI, int NORM, bool PF, int LCP>
 __global__ void __launch_bounds__(256) k_hop_b(const HopLaunch* __restrict__ tab, const int4* __restrict__ map) {
   const int4 m = map[blockIdx.x];
   if (m.x < 0) return;  // alignment padding of the batched grid
@@ -544,7 +572,7 @@ __global__ void __launch_bounds__(256) k_hop_b(const HopLaunch* __restrict__ tab
 
 template <int P, int RECON, bool PF> void launch_hop_t(const HopLaunch& h, hipStream_t s, const BatchGrid* bg) {
   const int nb = (h.g.Vh + h.block - 1) / h.block;
-  const bool norm = h.partials != nullptr;
+  const int norm = hop_norm(h);
   const bool lnt = (h.fast & HOP_FAST_STREAM) != 0 && !PF;
 #define CMX_HOP_GO2(IS, EP, NM, CP)                                                                       \
   if (bg)                                                                                                 \
@@ -560,13 +588,30 @@ template <int P, int RECON, bool PF> void launch_hop_t(const HopLaunch& h, hipSt
   }
 #define CMX_HOP_CASE(IS, EP)                                                                              \
   if (h.isign == IS && h.epi == EP) {                                                                     \
-    if (norm) {                                                                                           \
-      CMX_HOP_GO(IS, EP, true)                                                                            \
+    if (norm == NORM_ONLY) {                                                                              \
+      CMX_HOP_GO(IS, EP, NORM_ONLY)                                                                       \
     } else {                                                                                              \
-      CMX_HOP_GO(IS, EP, false)                                                                           \
+      CMX_HOP_GO(IS, EP, NORM_NONE)                                                                       \
     }                                                                                                     \
     return;                                                                                               \
   }
+#define CMX_HOP_TAIL(IS, EP, NM)                                                                          \
+  if (h.isign == IS && h.epi == EP && norm == NM) {                                                       \
+    CMX_HOP_GO(IS, EP, NM)                                                                                \
+    return;                                                                                               \
+  }
+  CMX_HOP_TAIL(-1, EPI_XPAY, NORM_UPDATE)
+  CMX_HOP_TAIL(-1, EPI_CLOV_XPAY, NORM_UPDATE)
+  CMX_HOP_TAIL(1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOP_TAIL(1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOP_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOP_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_Y)
+  CMX_HOP_TAIL(-1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOP_TAIL(-1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOP_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOP_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_Y)
+#undef CMX_HOP_TAIL
+  if (norm > NORM_ONLY) throw Error(CMX_ERR_ARG, "launch_hop: tail not instantiated");
   CMX_HOP_CASE(1, EPI_NONE)
   CMX_HOP_CASE(1, EPI_CLOV)
   CMX_HOP_CASE(1, EPI_XPAY)

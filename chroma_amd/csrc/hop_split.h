@@ -124,7 +124,7 @@ template <typename R> __device__ __forceinline__ void half_clover(const R (&c)[3
   }
 }
 
-template <int P, int ISIGN, int EPI, bool NORM>
+template <int P, int ISIGN, int EPI, int NORM>
 __device__ __forceinline__ void hop_split_body(const HopLaunch& h, int blk, int nblk) {
   using R = typename FastReal<P>::T;
   __shared__ R part[4][24][64];
@@ -200,21 +200,35 @@ __device__ __forceinline__ void hop_split_body(const HopLaunch& h, int blk, int 
       for (int k = 0; k < 12; ++k) out[k] += s[k];
     }
     if constexpr (NORM) {
+      auto dot = [&](const R(&u)[12], const R(&v)[12]) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          const double ur = u[2 * k], ui = u[2 * k + 1], vr = v[2 * k], vi = v[2 * k + 1];
+          dre += ur * vr + ui * vi;
+          dim += ur * vi - ui * vr;
+        }
+      };
+      if constexpr (NORM == NORM_UPDATE) {  // as hop_finish, on half a site
+        constexpr int PY = P == P64 ? P64 : P32;
+        R y[12];
+        const R cf = (R)*h.coef;
+        half_load<PY>(h.y, nullptr, h.y_stride, i, w, y);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) out[k] = y[k] + cf * out[k];
+        half_store<PY>(h.y, nullptr, h.y_stride, i, w, out, 0.f);
+      } else if constexpr (NORM == NORM_DOT_Y) {
+        R y[12];
+        half_load<P>(h.y, h.y_nrm, h.y_stride, i, w, y);
+        dot(y, out);
+      } else if constexpr (NORM == NORM_DOT_X) {
+        dot(out, xs);
+      }
 #pragma unroll
       for (int k = 0; k < 12; ++k) nsq += (double)out[k] * (double)out[k];
-      if constexpr (EPI == EPI_XPAY || EPI == EPI_CLOV_XPAY)
-        if (h.ndot) {
-#pragma unroll
-          for (int k = 0; k < 6; ++k) {
-            const double orr = out[2 * k], oi = out[2 * k + 1], xr = xs[2 * k], xi = xs[2 * k + 1];
-            dre += orr * xr + oi * xi;
-            dim += orr * xi - oi * xr;
-          }
-        }
     }
   }
   float m = 0;
-  if constexpr (P == P16) {
+  if constexpr (P == P16 && NORM != NORM_UPDATE) {
     if (fin) {
 #pragma unroll
       for (int k = 0; k < 12; ++k) m = fmaxf(m, fabsf(out[k]));
@@ -223,15 +237,16 @@ __device__ __forceinline__ void hop_split_body(const HopLaunch& h, int blk, int 
     __syncthreads();
     if (fin) m = fmaxf(m, mx[1 - w][lane]);
   }
-  if (fin) half_store<P>(h.out, h.out_nrm, h.out_stride, i, w, out, m);
-  if constexpr (NORM) write_norm_partials(h, blk, nsq, dre, dim);
+  if constexpr (NORM != NORM_UPDATE)
+    if (fin) half_store<P>(h.out, h.out_nrm, h.out_stride, i, w, out, m);
+  if constexpr (NORM) write_norm_partials<NORM>(h, blk, nsq, dre, dim);
 }
 
-template <int P, int ISIGN, int EPI, bool NORM>
+template <int P, int ISIGN, int EPI, int NORM>
 __global__ void __launch_bounds__(256) k_hop_split(HopLaunch h) {
   hop_split_body<P, ISIGN, EPI, NORM>(h, blockIdx.x, gridDim.x);
 }
-template <int P, int ISIGN, int EPI, bool NORM>
+template <int P, int ISIGN, int EPI, int NORM>
 __global__ void __launch_bounds__(256) k_hop_split_b(const HopLaunch* __restrict__ tab, const int4* __restrict__ map) {
   const int4 m = map[blockIdx.x];
   if (m.x < 0) return;  // alignment padding of the batched grid
@@ -240,6 +255,7 @@ __global__ void __launch_bounds__(256) k_hop_split_b(const HopLaunch* __restrict
 
 template <int P> void launch_hop_split_t(const HopLaunch& h, hipStream_t s, const BatchGrid* bg) {
   const dim3 grid((h.g.Vh + 63) / 64);
+  const int norm = hop_norm(h);
 #define CMX_HOPS_GO(IS, EP, NM)                                                                     \
   if (bg)                                                                                           \
     hipLaunchKernelGGL((k_hop_split_b<P, IS, EP, NM>), dim3(bg->nblocks), dim3(256), 0, s,          \
@@ -248,13 +264,30 @@ template <int P> void launch_hop_split_t(const HopLaunch& h, hipStream_t s, cons
     hipLaunchKernelGGL((k_hop_split<P, IS, EP, NM>), grid, dim3(256), 0, s, h);
 #define CMX_HOPS_CASE(IS, EP)                                                                       \
   if (h.isign == IS && h.epi == EP) {                                                               \
-    if (h.partials) {                                                                               \
-      CMX_HOPS_GO(IS, EP, true)                                                                     \
+    if (norm == NORM_ONLY) {                                                                        \
+      CMX_HOPS_GO(IS, EP, NORM_ONLY)                                                                \
     } else {                                                                                        \
-      CMX_HOPS_GO(IS, EP, false)                                                                    \
+      CMX_HOPS_GO(IS, EP, NORM_NONE)                                                                \
     }                                                                                               \
     return;                                                                                         \
   }
+#define CMX_HOPS_TAIL(IS, EP, NM)                                                                   \
+  if (h.isign == IS && h.epi == EP && norm == NM) {                                                 \
+    CMX_HOPS_GO(IS, EP, NM)                                                                         \
+    return;                                                                                         \
+  }
+  CMX_HOPS_TAIL(-1, EPI_XPAY, NORM_UPDATE)
+  CMX_HOPS_TAIL(-1, EPI_CLOV_XPAY, NORM_UPDATE)
+  CMX_HOPS_TAIL(1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOPS_TAIL(1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOPS_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOPS_TAIL(1, EPI_CLOV_XPAY, NORM_DOT_Y)
+  CMX_HOPS_TAIL(-1, EPI_XPAY, NORM_DOT_X)
+  CMX_HOPS_TAIL(-1, EPI_XPAY, NORM_DOT_Y)
+  CMX_HOPS_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_X)
+  CMX_HOPS_TAIL(-1, EPI_CLOV_XPAY, NORM_DOT_Y)
+#undef CMX_HOPS_TAIL
+  if (norm > NORM_ONLY) throw Error(CMX_ERR_ARG, "launch_hop_split: tail not instantiated");
   CMX_HOPS_CASE(1, EPI_NONE)
   CMX_HOPS_CASE(1, EPI_CLOV)
   CMX_HOPS_CASE(1, EPI_XPAY)

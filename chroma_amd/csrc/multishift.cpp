@@ -105,9 +105,8 @@ void solve_multishift(Op& op, const cmx_solver_params& p, int ns, const double* 
     auto step = [&](int phase) {
       L.nb = op.apply(P64, mp.view(), p0.view(), +1, op.partials.as<double>(), F + F_DONE);
       ms_scalars(L, 1, op.stream);
-      op.apply(P64, mmp.view(), mp.view(), -1, nullptr, F + F_DONE);
-      op.blas(B_AXPY_NORM, {&r, &mmp}, MS_B, 0, F_DONE);
-      L.nb = nb;
+      L.nb = op.apply(P64, r.view(), mp.view(), -1, op.partials.as<double>(), F + F_DONE, nullptr,
+                      {TAIL_UPDATE, &r, op.state_S.as<double>() + MS_B});
       ms_scalars(L, phase, op.stream);
     };
     auto poll = [&]() {

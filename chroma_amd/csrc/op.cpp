@@ -382,12 +382,27 @@ static void set_in(HopLaunch& h, VRef r) {
 static void set_out(HopLaunch& h, VRef r) {
   h.out = r.v, h.out_nrm = r.nrm, h.out_stride = r.stride;
 }
+static void set_tail(HopLaunch& h, const ApplyTail& t, int off) {
+  h.tail = t.kind;
+  if (!t.y) return;
+  const VRef r = t.y->view(off);
+  h.y = r.v;
+  h.y_nrm = r.nrm;
+  h.y_stride = r.stride;
+  h.coef = t.coef;
+}
 static void set_x(HopLaunch& h, VRef r) {
   h.x = r.v, h.x_nrm = r.nrm, h.x_stride = r.stride;
 }
 
-int Op::apply(int prec, VRef out, VRef in, int isign, double* parts, const int* skip, const int* run, bool ndot) {
-  CMX_REQUIRE(!ndot || (parts && eo()), CMX_ERR_ARG, "apply: <chi, psi> partials need an even-odd operator");
+int Op::apply(int prec, VRef out, VRef in, int isign, double* parts, const int* skip, const int* run,
+              const ApplyTail& tail) {
+  CMX_REQUIRE(tail.kind == TAIL_NONE || parts, CMX_ERR_ARG, "apply: a tail needs partials");
+  if (tail.kind >= TAIL_DOT_Y)
+    CMX_REQUIRE(tail.y && tail.y->n == subset_sites() &&
+                    tail.y->prec == (tail.kind == TAIL_UPDATE && prec == P16 ? (int)P32 : prec) &&
+                    (tail.kind != TAIL_UPDATE || tail.coef),
+                CMX_ERR_ARG, "apply: the tail's vector does not fit the operator");
   ensure_prec(prec);
   HopLaunch h = hop_base(prec);
   const int nb = hop_num_blocks(h);
@@ -416,7 +431,7 @@ int Op::apply(int prec, VRef out, VRef in, int isign, double* parts, const int* 
     h.a = fact;
     h.b = clover() ? -0.25 : -0.25 / fact;
     h.partials = parts;
-    h.ndot = ndot ? 1 : 0;  // x = psi_o: <chi_o, psi_o> from the values the epilogue holds
+    set_tail(h, tail, 0);
     launch_hop(h, stream);
     return parts ? nb : 0;
   }
@@ -434,12 +449,14 @@ int Op::apply(int prec, VRef out, VRef in, int isign, double* parts, const int* 
   set_x(h, in_e);
   set_out(h, out_e);
   h.partials = parts;
+  set_tail(h, tail, 0);
   launch_hop(h, stream);
   h.cb = 1;
   set_in(h, in_e);
   set_x(h, in_o);
   set_out(h, out_o);
-  h.partials = parts ? parts + nb : nullptr;
+  h.partials = parts ? parts + nb * (tail.kind == TAIL_DOT_X || tail.kind == TAIL_DOT_Y ? 3 : 1) : nullptr;
+  set_tail(h, tail, (int)Vh);
   launch_hop(h, stream);
   return parts ? 2 * nb : 0;
 }

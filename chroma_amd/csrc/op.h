@@ -120,6 +120,13 @@ struct GaugeData {
   double su3_dev = 0;      // max deviation from (phase x SU(3)) over all links
 };
 
+// what the operator's last kernel does with its result (HopTail); y spans the operator's subset
+struct ApplyTail {
+  int kind = TAIL_NONE;
+  const Vec* y = nullptr;
+  const double* coef = nullptr;
+};
+
 struct Op {
   std::shared_ptr<GaugeData> gd;
   cmx_op_params par{};
@@ -176,11 +183,11 @@ struct Op {
   Vec& tmp(int prec, int k);
   HopLaunch hop_base(int prec, int which = 0) const;
 
-  // chi = M(isign) psi on the subset; partials (optional) receives |chi|^2 per work-group, or with ndot
-  // (even-odd operators) |chi|^2, Re <chi, psi>, Im <chi, psi> per work-group (three partials each);
-  // returns the number of work-groups whose partials were written.
+  // chi = M(isign) psi on the subset; partials (optional) receives |chi|^2 per work-group, or what tail says
+  // (a tail needs partials; TAIL_UPDATE does not write chi); returns the number of work-groups whose partials
+  // were written.
   int apply(int prec, VRef out, VRef in, int isign, double* partials, const int* skip = nullptr,
-            const int* run = nullptr, bool ndot = false);
+            const int* run = nullptr, const ApplyTail& tail = ApplyTail());
   // raw hopping term on output checkerboard cb (views of one checkerboard each), scaled by b
   void dslash(int prec, VRef out, VRef in, int isign, int cb, double b = 1.0);
   // the same on n sources at once (FP16 storage: links loaded once per group of sources); false when

@@ -231,11 +231,10 @@ struct CGState {
   const Vec& chi;
   bool mdagm;
   int n, nb;
-  Vec &chi_tmp, &r, &pv, &mp, &mmp;
+  Vec &chi_tmp, &r, &pv, &mp;
   CGState(Op& o, const cmx_solver_params& p_, Vec& psi_, const Vec& chi_, bool mdagm_)
       : op(o), p(p_), psi(psi_), chi(chi_), mdagm(mdagm_), n(o.subset_sites()), nb(blas_blocks(n)),
-        chi_tmp(o.work(10, P64, n)), r(o.work(11, P64, n)), pv(o.work(12, P64, n)), mp(o.work(13, P64, n)),
-        mmp(o.work(14, P64, n)) {}
+        chi_tmp(o.work(10, P64, n)), r(o.work(11, P64, n)), pv(o.work(12, P64, n)), mp(o.work(13, P64, n)) {}
   // chi_tmp = M^dag chi, the tolerance, and the start r = chi_tmp - M^dag M psi ; p = r
   void setup(Timer* tm) {
     if (mdagm)  // syssolver_linop_cg.h:65-66
@@ -247,18 +246,17 @@ struct CGState {
     if (tm) tm->start();
     // invcg2.cc:109-131
     op.apply(P64, mp.view(), psi.view(), +1, nullptr);
-    op.apply(P64, mmp.view(), mp.view(), -1, nullptr);
-    op.blas(B_XMY_NORM, {&r, &chi_tmp, &mmp});
+    op.apply(P64, pv.view(), mp.view(), -1, nullptr);
+    op.blas(B_XMY_NORM_COPY, {&r, &chi_tmp, &pv, &pv});
     op.finalize(nb, 1, PG_CG_INIT);
-    op.blas(B_COPY, {&pv, &r});
   }
   void iter() {
     int* F = op.state_F.as<int>();
     const int np = op.apply(P64, mp.view(), pv.view(), +1, op.partials.as<double>(), F + F_DONE);  // Mp, |Mp|^2
     op.finalize(np, 1, PG_CG_D);                                                                 // a = c/d
-    op.apply(P64, mmp.view(), mp.view(), -1, nullptr, F + F_DONE);                               // M^dag M p
-    op.blas(B_AXPY_NORM, {&r, &mmp}, S_NEGA, 0, F_DONE);                                         // r -= a M^dag M p
-    op.finalize(nb, 1, PG_CG_R);                                                                 // cp, b, test
+    const int nr = op.apply(P64, r.view(), mp.view(), -1, op.partials.as<double>(), F + F_DONE, nullptr,
+                            {TAIL_UPDATE, &r, op.state_S.as<double>() + S_NEGA});                // r -= a M^dag M p
+    op.finalize(nr, 1, PG_CG_R);                                                                 // cp, b, test
     op.blas(B_CG_UPDATE, {&psi, &pv, &r}, S_A, S_B, F_DONE);                                     // psi += a p; p = r + b p
   }
   // results once the device has stopped (state read back)
@@ -303,13 +301,13 @@ void solve_bicgstab(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& chi
     op.blas(B_CDOT, {&r0, &r}, 0, 0, F_DONE);  // rho = <r0|r>
     op.finalize(nb, 2, PG_BICG_RHO);           // beta = (rho/rho_prev)(alpha/omega)
     op.blas(B_BICG_P, {&pv, &r, &v}, S_OMEGA, S_BETAC, F_DONE);  // p = r + beta (p - omega v)
-    op.apply(P64, v.view(), pv.view(), isign, nullptr, F + F_DONE);  // v = A p
-    op.blas(B_CDOT, {&r0, &v}, 0, 0, F_DONE);
-    op.finalize(nb, 2, PG_BICG_ALPHA);                            // alpha = rho / <r0|v>
+    const int nv = op.apply(P64, v.view(), pv.view(), isign, op.partials.as<double>(), F + F_DONE, nullptr,
+                            {TAIL_DOT_Y, &r0});                   // v = A p, <r0|v>
+    op.finalize(nv, 3, PG_BICG_ALPHA);                            // alpha = rho / <r0|v>
     op.blas(B_CAXPY, {&r, &v}, S_NALPHA, 0, F_DONE);              // s = r - alpha v
-    op.apply(P64, t.view(), r.view(), isign, nullptr, F + F_DONE);   // t = A s
-    op.blas(B_TNORM_TDOT, {&t, &r}, 0, 0, F_DONE);
-    op.finalize(nb, 3, PG_BICG_OMEGA);                            // omega = <t|s>/|t|^2
+    const int nt = op.apply(P64, t.view(), r.view(), isign, op.partials.as<double>(), F + F_DONE, nullptr,
+                            {TAIL_DOT_X});                        // t = A s, |t|^2, <t|s>
+    op.finalize(nt, 3, PG_BICG_OMEGA);                            // omega = <t|s>/|t|^2
     op.blas(B_BICG_UPDATE, {&psi, &r, &pv, &t}, S_OMEGA, S_ALPHA, F_DONE);  // psi += omega s + alpha p; r = s - omega t
     op.finalize(nb, 1, PG_BICG_R);
   };
@@ -330,7 +328,7 @@ struct RelCGState {
   bool mdagm;
   int n, ps, nb;
   Vec &chi_tmp, &b, &r_dble, &x_dble, &tmp1, &tmp2;
-  Vec &r, &x, &pv, &mp, &mmp;
+  Vec &r, &x, &pv, &mp;
   static int check_prec(int ps) {
     CMX_REQUIRE(ps == P32 || ps == P16, CMX_ERR_ARG, "reliable CG: sloppy precision must be single or half");
     return ps;
@@ -339,7 +337,7 @@ struct RelCGState {
       : op(o), p(p_), psi(psi_), chi(chi_), mdagm(mdagm_), n(o.subset_sites()), ps(check_prec(p_.sloppy_prec)),
         nb(blas_blocks(n)), chi_tmp(o.work(30, P64, n)), b(o.work(31, P64, n)), r_dble(o.work(32, P64, n)),
         x_dble(o.work(33, P64, n)), tmp1(o.work(34, P64, n)), tmp2(o.work(35, P64, n)), r(o.work(36, P32, n)),
-        x(o.work(37, P32, n)), pv(o.work(38, ps, n)), mp(o.work(39, ps, n)), mmp(o.work(40, ps, n)) {}
+        x(o.work(37, P32, n)), pv(o.work(38, ps, n)), mp(o.work(39, ps, n)) {}
   void setup(Timer* tm) {
     // chi_tmp = M^dag chi (syssolver_linop_rel_cg_clover.h:121-125); the MdagM solver takes chi as is
     // (syssolver_mdagm_rel_cg_clover.h:126-133)
@@ -361,12 +359,18 @@ struct RelCGState {
   }
   void inner() {
     int* F = op.state_F.as<int>();
-    op.blas(B_XPAY, {&pv, &r}, S_BETA, 0, F_DONE);                                          // p = r + beta p
+    // x += a p of the iteration before (a = 0 at the start and after an FP64 update); p = r + beta p
+    op.blas(B_CG_UPDATE, {&x, &pv, &r}, S_A, S_BETA, F_DONE);
     const int np = op.apply(ps, mp.view(), pv.view(), +1, op.partials.as<double>(), F + F_DONE);
     op.finalize(np, 1, PG_RCG_D);                                                           // c = r_sq; a = c/d
-    op.apply(ps, mmp.view(), mp.view(), -1, nullptr, F + F_DONE);
-    op.blas(B_AXPY2_NORM, {&x, &r, &pv, &mmp}, S_A, 0, F_DONE);                             // x += a p; r -= a mmp
-    op.finalize(nb, 1, PG_RCG_R);                                                           // updateX / updateR
+    const int nr = op.apply(ps, r.view(), mp.view(), -1, op.partials.as<double>(), F + F_DONE, nullptr,
+                            {TAIL_UPDATE, &r, op.state_S.as<double>() + S_NEGA});           // r -= a M^dag M p
+    op.finalize(nr, 1, PG_RCG_R);                                                           // updateX / updateR
+  }
+  // once the iterations have stopped: the x += a p of the last one, psi += x (reliable_cg.cc:158-163)
+  void add_x() {
+    op.blas(B_AXPY, {&x, &pv}, S_A);
+    op.blas(B_ADD, {&psi, &x});
   }
   // The FP64 update of an iteration that holds for it: r = b - A^dag A x (reliable_cg.cc:120-136), the norms
   // and the convergence test, and (F_UPDX) psi += x; x = 0; b = r.  gated: every launch asks the flags (a
@@ -375,6 +379,7 @@ struct RelCGState {
     int* F = op.state_F.as<int>();
     const int run = gated ? F_UPDR : -1;
     const int* runp = gated ? F + F_UPDR : nullptr;
+    op.blas(B_AXPY, {&x, &pv}, S_A, 0, -1, run);
     op.blas(B_COPY, {&x_dble, &x}, 0, 0, -1, run);
     op.apply(P64, tmp1.view(), x_dble.view(), +1, nullptr, nullptr, runp);
     op.apply(P64, tmp2.view(), tmp1.view(), -1, nullptr, nullptr, runp);
@@ -413,7 +418,7 @@ void solve_relcg(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& chi, b
         std::printf("RelCG: k = %d  r_sq = %.6e  d = %.6e  a = %.6e  updateR %d updateX %d err %d\n", op.hF[F_K],
                     op.hS[S_RSQ], op.hS[S_D], op.hS[S_A], op.hF[F_UPDR], op.hF[F_UPDX], op.hF[F_ERR]);
       });
-  op.blas(B_ADD, {&psi, &st.x});                                                            // psi += x (reliable_cg.cc:158-163)
+  st.add_x();
   read_state(op);
   st.finish(tm.stop(), res);
 }
@@ -451,13 +456,13 @@ void solve_relbicgstab(Op& op, const cmx_solver_params& p, Vec& psi, const Vec& 
       op, p,
       [&] {
         op.blas(B_BICG_P, {&pv, &r, &v}, S_OMEGA, S_BETAC, F_DONE);                // p = r + beta (p - omega v)
-        op.apply(ps, v.view(), pv.view(), isign, nullptr, F + F_DONE);             // v = A p
-        op.blas(B_CDOT, {&r0, &v}, 0, 0, F_DONE);
-        op.finalize(nb, 2, PG_RBICG_ALPHA);                                        // alpha = rho / <r0|v>
+        const int nv = op.apply(ps, v.view(), pv.view(), isign, op.partials.as<double>(), F + F_DONE, nullptr,
+                                {TAIL_DOT_Y, &r0});                                // v = A p, <r0|v>
+        op.finalize(nv, 3, PG_RBICG_ALPHA);                                        // alpha = rho / <r0|v>
         op.blas(B_CAXPY2, {&r, &v, &x, &pv}, S_NALPHA, S_ALPHA, F_DONE);           // s = r - alpha v; x += alpha p
-        op.apply(ps, t.view(), r.view(), isign, nullptr, F + F_DONE);              // t = A s
-        op.blas(B_TNORM_TDOT, {&t, &r}, 0, 0, F_DONE);
-        op.finalize(nb, 3, PG_BICG_OMEGA);                                         // omega = <t|s> / |t|^2
+        const int nt = op.apply(ps, t.view(), r.view(), isign, op.partials.as<double>(), F + F_DONE, nullptr,
+                                {TAIL_DOT_X});                                     // t = A s, |t|^2, <t|s>
+        op.finalize(nt, 3, PG_BICG_OMEGA);                                         // omega = <t|s> / |t|^2
         op.blas(B_RBICG_UPDATE, {&x, &r, &t, &r0}, S_OMEGA, 0, F_DONE);            // x += omega s; r = s - omega t
         op.finalize(nb, 3, PG_RBICG_R);                                            // updateX / updateR
       },
@@ -1233,7 +1238,7 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
     for (int k = 0; k < na; ++k) {
       const int i = act[k];
       Op& op = *ops[i];
-      if (rel) op.blas(B_ADD, {psi[i], &rcg[k]->x});  // psi += x (reliable_cg.cc:158-163)
+      if (rel) rcg[k]->add_x();
       read_state(op);
       cmx_solver_result part;
       std::memset(&part, 0, sizeof(part));

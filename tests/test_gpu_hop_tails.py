@@ -1,0 +1,44 @@
+"""GPU: the vector operations that the hopping kernels' epilogues do for the solvers (the dot products of BiCGStab
+and the residual update of CG), in each of the three kernels, for each storage precision and on the full lattice
+as well as on a checkerboard, with a last work-group that is partly empty.  A wrong sum or update shows in the
+iteration count against the oracle's solver."""
+import numpy as np
+import pytest
+
+import oracle
+from chroma_amd import lib as cmx
+from tests.util import random_fermion, rel
+
+pytestmark = pytest.mark.gpu
+
+SOLVERS = [(cmx.CG, cmx.DOUBLE), (cmx.BICGSTAB, cmx.DOUBLE), (cmx.RELIABLE_CG, cmx.SINGLE),
+           (cmx.RELIABLE_CG, cmx.HALF), (cmx.RELIABLE_BICGSTAB, cmx.DOUBLE), (cmx.RELIABLE_BICGSTAB, cmx.SINGLE),
+           (cmx.RELIABLE_BICGSTAB, cmx.HALF)]
+ORACLE = {cmx.CG: oracle.CG, cmx.BICGSTAB: oracle.BICGSTAB, cmx.RELIABLE_CG: oracle.CG,
+          cmx.RELIABLE_BICGSTAB: oracle.BICGSTAB}
+
+
+@pytest.mark.parametrize("kernel", ["default", "plane", "linear"])
+@pytest.mark.parametrize("kind", [cmx.UNPREC_WILSON, cmx.EO_WILSON, cmx.EO_CLOVER])
+def test_solver_tails(kernel, kind):
+    L = (4, 6, 2, 10)
+    V = int(np.prod(L))
+    U = cmx.gauge_apply_bc(L, cmx.gauge_generate(L, kind=1, seed=5, eps=0.3), (1, 1, 1, -1))
+    mass = cmx.kappa_to_mass(0.11)
+    ref_op = oracle.Op(kind, L, U, mass, 1.0, 1.0)
+    lo = 0 if kind == cmx.UNPREC_WILSON else V // 2
+    chi = random_fermion(V, 6)
+    chi[:lo] = 0
+    rsd = 1e-9
+    for solver, prec in SOLVERS:
+        op = cmx.Operator(cmx.Gauge(L, U), kind, mass, 1.0, sloppy_prec=cmx.HALF if prec == cmx.HALF else cmx.SINGLE)
+        if kernel != "default":
+            op.set_hop_config(prec, block=64, fast=1 if kernel == "plane" else 0)
+        print("tails", kernel, kind, solver, prec, op.hop_config(prec), flush=True)
+        psi_ref, n_ref, _, _ = ref_op.solve(chi, solver=ORACLE[solver], rsd=rsd, maxit=500)
+        psi, res = op.solve(chi[lo:], solver=solver, rsd=rsd, maxit=500, delta=0.1, sloppy_prec=prec)
+        # the same recurrence as the oracle's up to rounding; an FP64 update may cost the directions an iteration
+        assert res["n_count"] <= n_ref + 1 + res["n_reliable"], (res["n_count"], n_ref)
+        # |psi - psi_ref| <= (|M^-1| |M|) (rsd + rsd) |psi|; the spectrum of M lies in 4 + m +- 4.2 (clover
+        # included), so the condition number is below (2 * 4.55 - 0.3) / 0.3 < 30, squared for the normal equations
+        assert rel(psi, psi_ref[lo:]) < 2 * 900 * rsd
