@@ -331,8 +331,7 @@ void* scratch_take(size_t bytes, size_t& cap, int& dev) {
       const Cached c = P.cache[best];
       cap = c.cap;
       P.cached -= cap;
-      P.cache[best] = P.cache.back();
-      P.cache.pop_back();
+      P.cache.erase(P.cache.begin() + (long)best);  // keeps the order of age
       return c.p;
     }
   }
@@ -347,16 +346,24 @@ void* scratch_take(size_t bytes, size_t& cap, int& dev) {
 
 void scratch_give(void* p, size_t cap, int dev) {
   if (!p) return;
-  Pool& P = pool();
-  {
+  // A full cache lets the buffers go that lay in it longest: they belong to sizes no longer in use, and refusing
+  // the new ones instead made every later call allocate (12 batched solves: 34 -> 63 ms).
+  std::vector<void*> out;
+  if (cap > CACHE_MAX) {
+    out.push_back(p);
+  } else {
+    Pool& P = pool();
     std::lock_guard<std::mutex> lk(P.m);
-    if (P.cached + cap <= CACHE_MAX && P.cache.size() < CACHE_ENTRIES) {
-      P.cache.push_back(Cached{p, cap, dev});
-      P.cached += cap;
-      return;
+    size_t n = 0;
+    for (; n < P.cache.size() && (P.cached + cap > CACHE_MAX || P.cache.size() - n >= CACHE_ENTRIES); ++n) {
+      out.push_back(P.cache[n].p);
+      P.cached -= P.cache[n].cap;
     }
+    P.cache.erase(P.cache.begin(), P.cache.begin() + (long)n);
+    P.cache.push_back(Cached{p, cap, dev});
+    P.cached += cap;
   }
-  (void)hipFree(p);
+  for (void* q : out) (void)hipFree(q);
 }
 
 void* pinned_take() {
