@@ -4,17 +4,23 @@
 // only smeared directions contribute staples; the staple sum C and Q of getQsandCs (:105-180):
 //   C_mu(x) = rho sum_{nu != mu} [ U_nu(x) U_mu(x+nu) U_nu^dag(x+mu) + U_nu^dag(x-nu) U_mu(x-nu) U_nu(x-nu+mu) ],
 //   Omega = C U_mu^dag(x),  Q = (i/2) [ (Omega^dag - Omega) - tr(Omega^dag - Omega)/3 ],  U'_mu(x) = exp(iQ) U_mu(x).
-// The reference evaluates exp(iQ) by Cayley-Hamilton (getFsAndBs, :383-874); here it is a degree-14
+// The reference evaluates exp(iQ) in closed form from the eigenvalues (getFsAndBs, :383-874); here it is a
 // Taylor polynomial with scaling and squaring (Moler & Van Loan, "Nineteen dubious ways to compute the
-// exponential of a matrix", method 3), exact to rounding with no small-eigenvalue special case.  The
+// exponential of a matrix", method 3), reduced by Cayley-Hamilton to a combination of 1, Q and Q^2: exact to
+// rounding with no small-eigenvalue special case.  The
 // product is re-projected onto SU(3) (rows 0 and 1 orthonormalised, row 2 = conj(row0 x row1)), which
 // moves it only at rounding level and keeps many steps from drifting off the group.
 //
 // Layout: the host gauge layout ([mu][site][3][3] complex, sites checkerboard-major, x fastest within a
 // checkerboard) is transposed on the device into [mu][element][site], so that each of a lane's loads and
 // stores is one 16 B element and a wave's 64 lanes touch 1 KiB of consecutive sites; the steps run in
-// that layout and the result is transposed back.  One lane per (mu, site); each link is read by 13 lanes
-// (its own, and as a staple leg of 12 others), mostly from L2.
+// that layout and the result is transposed back.  One lane per (mu, site).  A step is bound by link traffic:
+// each link is read by 13 lanes (its own, and as a staple leg of 12 others), 11.5 GB per step at 32^4 where the
+// field has 0.6.  A work-group is the four directions of 64 sites, the two checkerboards of a region follow each
+// other, and each XCD owns a contiguous eighth of the lattice, so that most of these reads are L1 and L2 hits.
+// Per step, 16^3x32 and 32^4: one direction after another over the whole lattice 175 and 1610 us; this order
+// 130 and 1000 us; with exp(iQ) from scalars instead of 14 matrix products 85 and 820 us.  A third wave per SIMD
+// (168 instead of 210 registers) spills and loses: 166 and 1775 us in the first order.
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -66,18 +72,38 @@ __device__ __forceinline__ M3 mul_nd(const M3& a, const M3& b) {  // a b^dag
     }
   return c;
 }
-__device__ __forceinline__ M3 mul_dn(const M3& a, const M3& b) {  // a^dag b
-  M3 c;
+// acc += a b c^dag and acc += a^dag b c, row by row: one row of the product a b is live at a time
+__device__ __forceinline__ void add_abcd(M3& acc, const M3& a, const M3& b, const M3& c) {
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+  for (int i = 0; i < 3; ++i) {
+    double2 t[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      double2 t = make_double2(0, 0);
+      t[j] = make_double2(0, 0);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) t = cfmca(a.e[3 * k + i], b.e[3 * k + j], t);
-      c.e[3 * i + j] = t;
+      for (int k = 0; k < 3; ++k) t[j] = cfma(a.e[3 * i + k], b.e[3 * k + j], t[j]);
     }
-  return c;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc.e[3 * i + j] = cfmac(t[k], c.e[3 * j + k], acc.e[3 * i + j]);
+  }
+}
+__device__ __forceinline__ void add_adbc(M3& acc, const M3& a, const M3& b, const M3& c) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    double2 t[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      t[j] = make_double2(0, 0);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) t[j] = cfmca(a.e[3 * k + i], b.e[3 * k + j], t[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc.e[3 * i + j] = cfma(t[k], c.e[3 * k + j], acc.e[3 * i + j]);
+  }
 }
 
 struct StoutGeom {
@@ -115,32 +141,63 @@ __global__ void __launch_bounds__(256) k_links_from_soa(long V, const double2* _
   for (int k = 0; k < 9; ++k) out[t * 9 + k] = in[(mu * 9 + k) * V + s];
 }
 
-// exp(X) for a 3x3 X with |X|_F = O(1): X 2^-s with |X 2^-s|_F <= 1/4, Horner form of the degree-14
-// Taylor polynomial (truncation below 1e-21 relative), then s squarings
-__device__ M3 expm(const M3& X) {
-  double nrm = 0;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) nrm += X.e[k].x * X.e[k].x + X.e[k].y * X.e[k].y;
-  nrm = sqrt(nrm);
+// exp(iQ) for a Hermitian traceless Q (diagonal q, upper triangle z01 z02 z12).  Q 2^-s with |Q 2^-s|_F <= 1,
+// the degree-18 Taylor polynomial (truncation below 1e-17), then s squarings.  By Cayley-Hamilton
+// Q^3 = c1 Q + c0 with c1 = tr Q^2 / 2 and c0 = det Q, so that Q^n = a + b Q + d Q^2 with real a, b, d that
+// follow from those of Q^(n-1), and the polynomial costs one matrix square and scalar arithmetic (as a Horner
+// scheme on matrices, degree 14 below norm 1/4, it was 14 to 16 of the 28 matrix products of a link).
+__device__ M3 exp_i(const double (&q)[3], double2 z01, double2 z02, double2 z12) {
+  auto sq = [](double2 z) { return fma(z.x, z.x, z.y * z.y); };
+  double nrm = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + 2.0 * (sq(z01) + sq(z02) + sq(z12)));
   int s = 0;
-  while (nrm > 0.25 && s < 60) {
+  while (nrm > 1.0 && s < 60) {
     nrm *= 0.5;
     ++s;
   }
   const double sc = ldexp(1.0, -s);
-  M3 Y;
+  const double q0 = q[0] * sc, q1 = q[1] * sc, q2 = q[2] * sc;
+  z01.x *= sc, z01.y *= sc, z02.x *= sc, z02.y *= sc, z12.x *= sc, z12.y *= sc;
+  const double n01 = sq(z01), n02 = sq(z02), n12 = sq(z12);
+  const double s0 = fma(q0, q0, n01 + n02), s1 = fma(q1, q1, n01 + n12), s2 = fma(q2, q2, n02 + n12);  // diag Q^2
+  const double c1 = 0.5 * (s0 + s1 + s2);
+  const double2 zz = cfma(z01, z12, make_double2(0, 0));
+  const double c0 = q0 * q1 * q2 + 2.0 * fma(zz.x, z02.x, zz.y * z02.y) - q0 * n12 - q1 * n02 - q2 * n01;
+  // f = sum i^n (a_n, b_n, d_n) / n! over n > 0; the 1 of n = 0 is added last, so that it is rounded once
+  double a = 1, b = 0, d = 0, fr[3] = {0, 0, 0}, fi[3] = {0, 0, 0};
 #pragma unroll
-  for (int k = 0; k < 9; ++k) Y.e[k] = make_double2(X.e[k].x * sc, X.e[k].y * sc);
-  // E = I + Y/1 (I + Y/2 (I + ... (I + Y/14)))
-  M3 E;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) E.e[k] = make_double2(k % 4 == 0 ? 1.0 : 0.0, 0.0);
-  for (int n = 14; n >= 1; --n) {
-    M3 T = mul(Y, E);
-    const double f = 1.0 / n;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) E.e[k] = make_double2(T.e[k].x * f + (k % 4 == 0 ? 1.0 : 0.0), T.e[k].y * f);
+  for (int n = 1; n <= 18; ++n) {
+    const double r = 1.0 / n, d0 = d * r;
+    d = b * r;
+    b = fma(c1, d0, a * r);
+    a = c0 * d0;
+    const double sg = (n >> 1) & 1 ? -1.0 : 1.0;
+    double(&f)[3] = n & 1 ? fi : fr;
+    f[0] = fma(sg, a, f[0]);
+    f[1] = fma(sg, b, f[1]);
+    f[2] = fma(sg, d, f[2]);
   }
+  // E = 1 + f0 + f1 Q + f2 Q^2; E_ji has conj(Q_ij), conj((Q^2)_ij)
+  M3 E;
+  auto diag = [&](double x, double y) {
+    return make_double2(1.0 + fma(fr[2], y, fma(fr[1], x, fr[0])), fma(fi[2], y, fma(fi[1], x, fi[0])));
+  };
+  auto off = [&](double2 x, double2 y) {  // f1 x + f2 y
+    return make_double2(fma(fr[1], x.x, fma(-fi[1], x.y, fma(fr[2], y.x, -fi[2] * y.y))),
+                        fma(fr[1], x.y, fma(fi[1], x.x, fma(fr[2], y.y, fi[2] * y.x))));
+  };
+  auto conj = [](double2 x) { return make_double2(x.x, -x.y); };
+  const double2 w01 = cfmac(z02, z12, make_double2((q0 + q1) * z01.x, (q0 + q1) * z01.y));
+  const double2 w02 = cfma(z01, z12, make_double2((q0 + q2) * z02.x, (q0 + q2) * z02.y));
+  const double2 w12 = cfmca(z01, z02, make_double2((q1 + q2) * z12.x, (q1 + q2) * z12.y));
+  E.e[0] = diag(q0, s0);
+  E.e[4] = diag(q1, s1);
+  E.e[8] = diag(q2, s2);
+  E.e[1] = off(z01, w01);
+  E.e[3] = off(conj(z01), conj(w01));
+  E.e[2] = off(z02, w02);
+  E.e[6] = off(conj(z02), conj(w02));
+  E.e[5] = off(z12, w12);
+  E.e[7] = off(conj(z12), conj(w12));
   for (int k = 0; k < s; ++k) E = mul(E, E);
   return E;
 }
@@ -178,10 +235,12 @@ __device__ void reunit(M3& U) {
 
 __global__ void __launch_bounds__(256) k_stout_step(StoutGeom g, const double2* __restrict__ cur,
                                                     double2* __restrict__ next, double rho, int dirs) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  const int mu = (int)(t / g.V);
-  const long s = t - (long)mu * g.V;
+  const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = xcd_range(blockIdx.x, gridDim.x);
+  const long r0 = (long)(l >> 1) * 64 + (threadIdx.x & 63);
+  if (r0 >= g.Vh) return;
+  const int cb = l & 1;
+  const long s = cb * g.Vh + r0;
   if (!(dirs >> mu & 1)) {  // next[mu] = current[mu]
     const double2* p = cur + (size_t)mu * 9 * g.V + s;
     double2* o = next + (size_t)mu * 9 * g.V + s;
@@ -191,8 +250,7 @@ __global__ void __launch_bounds__(256) k_stout_step(StoutGeom g, const double2* 
   }
   int x[4];
   {
-    const int cb = s >= g.Vh ? 1 : 0;
-    long r = s - cb * g.Vh;
+    long r = r0;
     const int Lxh = g.L[0] / 2;
     const int xh = (int)(r % Lxh);
     r /= Lxh;
@@ -217,27 +275,24 @@ __global__ void __launch_bounds__(256) k_stout_step(StoutGeom g, const double2* 
     y[nu] = x[nu] + 1 == g.L[nu] ? 0 : x[nu] + 1;
     const long xpn = site_of(g, y);
     // forward staple U_nu(x) U_mu(x+nu) U_nu^dag(x+mu)
-    const M3 f = mul_nd(mul(load(cur, g, nu, s), load(cur, g, mu, xpn)), load(cur, g, nu, xpm));
+    add_abcd(C, load(cur, g, nu, s), load(cur, g, mu, xpn), load(cur, g, nu, xpm));
     // backward staple U_nu^dag(x-nu) U_mu(x-nu) U_nu(x-nu+mu)
-    const M3 b = mul(mul_dn(load(cur, g, nu, xmn), load(cur, g, mu, xmn)), load(cur, g, nu, xmnpm));
-#pragma unroll
-    for (int k = 0; k < 9; ++k) C.e[k] = make_double2(C.e[k].x + f.e[k].x + b.e[k].x, C.e[k].y + f.e[k].y + b.e[k].y);
+    add_adbc(C, load(cur, g, nu, xmn), load(cur, g, mu, xmn), load(cur, g, nu, xmnpm));
   }
   const M3 U = load(cur, g, mu, s);
   const M3 Om = mul_nd(C, U);
-  // i Q = i (i/2) T = -T/2 with T = (Omega^dag - Omega) - tr/3, Omega scaled by rho
-  M3 X;
+  // Q = (i/2) T with T = (Omega^dag - Omega) - tr/3, Omega scaled by rho: Hermitian and traceless
+  double q[3];
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+  for (int i = 0; i < 3; ++i) q[i] = rho * Om.e[4 * i].y;
+  const double tr = (q[0] + q[1] + q[2]) / 3.0;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double2 a = Om.e[3 * j + i], c = Om.e[3 * i + j];
-      X.e[3 * i + j] = make_double2(-0.5 * rho * (a.x - c.x), -0.5 * rho * (-a.y - c.y));
-    }
-  const double2 tr = make_double2((X.e[0].x + X.e[4].x + X.e[8].x) / 3.0, (X.e[0].y + X.e[4].y + X.e[8].y) / 3.0);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) X.e[4 * i] = make_double2(X.e[4 * i].x - tr.x, X.e[4 * i].y - tr.y);
-  M3 N = mul(expm(X), U);
+  for (int i = 0; i < 3; ++i) q[i] -= tr;
+  auto up = [&](int i, int j) {  // (i/2) rho (conj(Omega_ji) - Omega_ij)
+    const double2 a = Om.e[3 * j + i], c = Om.e[3 * i + j];
+    return make_double2(0.5 * rho * (a.y + c.y), 0.5 * rho * (a.x - c.x));
+  };
+  M3 N = mul(exp_i(q, up(0, 1), up(0, 2), up(1, 2)), U);
   reunit(N);
   double2* o = next + (size_t)mu * 9 * g.V + s;
 #pragma unroll
@@ -273,7 +328,7 @@ void stout_smear(const int dims[4], const double* in, double* out, int nstep, do
   double2* cur = b.as<double2>();
   double2* nxt = a.as<double2>();
   for (int k = 0; k < nstep; ++k) {
-    hipLaunchKernelGGL(k_stout_step, grid, dim3(256), 0, 0, g, cur, nxt, rho, dirs);
+    hipLaunchKernelGGL(k_stout_step, dim3((unsigned)(2 * ((g.Vh + 63) / 64))), dim3(256), 0, 0, g, cur, nxt, rho, dirs);
     CMX_HIP(hipGetLastError());
     std::swap(cur, nxt);
   }
