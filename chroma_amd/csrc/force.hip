@@ -9,8 +9,7 @@
 // derivative is the sum over the four clover leaves of the plane with Lambda inserted at each corner of
 // cb (deriv_loops): per output link U_mu(x) two terms at x and two terms of the leaf below it (at
 // x - nu), and per U_nu(x) two at x and two of the leaf to its left (at x - mu).  One lane evaluates
-// all of them for its site, so each plane is one launch that writes ds_mu(x) and ds_nu(x) of its own
-// site only: no atomics, deterministic.  ds is [4][V][3][3] complex in the host site order (the layout
+// those of the three planes of its link and writes that link's derivative only: no atomics, deterministic.  ds is [4][V][3][3] complex in the host site order (the layout
 // of the C-ABI), accumulated as ds[mu] += ..., ds[nu] -= ... .
 #include <cstring>
 
@@ -35,16 +34,6 @@ struct ForcePlanes {
 
 __device__ __forceinline__ int plane_index(int mu, int nu) { return mu == 0 ? nu - 1 : mu == 1 ? nu + 1 : 5; }
 
-__device__ __forceinline__ M3 load_m3(const double2* b, size_t stride, size_t i) {
-  M3 m;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const double2 v = b[(size_t)k * stride + i];
-    m.a[2 * k] = v.x;
-    m.a[2 * k + 1] = v.y;
-  }
-  return m;
-}
 __device__ __forceinline__ M3 madd(const M3& A, const M3& B) {
   M3 C;
 #pragma unroll
@@ -116,113 +105,86 @@ __global__ void __launch_bounds__(256) k_force_lambda(Geom g, ForcePlanes P, VRe
   }
 }
 
-// The pieces of deriv_loops evaluated at site y (coordinates), Lambda on the sites of parity cb.
-// part = 0: the ds_mu terms at y; 1: the tmp_mu terms (shifted to y + nu); 2: the ds_nu terms;
-// 3: the tmp_nu terms (shifted to y + mu)
 struct LoopCtx {
   Geom g;
   const double2* g64[2];
-  const double2* Lam;  // this plane, [9][Vh]
-  int mu, nu, cb;
+  const double2* Lam;  // [6 planes][9][Vh]
+  int cb;
 };
 
-__device__ __forceinline__ M3 lam_at(const LoopCtx& C, const int (&x)[4]) {
-  if (parity(x) != C.cb) {
-    M3 z;
+// conj-transposed if dag (the same in all lanes)
+__device__ __forceinline__ M3 load_m3(const double2* b, size_t stride, bool dag) {
+  M3 m;
 #pragma unroll
-    for (int k = 0; k < 18; ++k) z.a[k] = 0;
-    return z;
+  for (int k = 0; k < 9; ++k) {
+    const double2 v = b[(size_t)(dag ? 3 * (k % 3) + k / 3 : k) * stride];
+    m.a[2 * k] = v.x;
+    m.a[2 * k + 1] = dag ? -v.y : v.y;
   }
-  return load_m3(C.Lam, C.g.Vh, cb_index(C.g, x));
+  return m;
 }
 
-__device__ M3 loop_terms(const LoopCtx& C, const int (&y)[4], int part) {
+// acc += f (one part of deriv_loops at site y (coordinates), Lambda on the sites of parity cb).
+// part = 0: the ds_mu terms at y; 1: the tmp_mu terms (shifted to y + nu); 2: the ds_nu terms;
+// 3: the tmp_nu terms (shifted to y + mu).  A part is a staple X Y Z of three links of the plaquette at y with
+// Lambda inserted at the two of its corners that have parity cb: at the two ends of Y Z, X (P W + W Q) with
+// W = Y Z, or of X Y, (P W + W Q) Z with W = X Y.  Y always enters conj-transposed.  Three links, two Lambda and
+// four products, in place of four, two and five or six with each term by itself.
+__device__ __forceinline__ void add_part(const LoopCtx& C, int mu, int nu, const int (&y)[4], int part, double f,
+                                         M3& acc) {
   const Geom& g = C.g;
-  const int mu = C.mu, nu = C.nu;
   int ym[4], yn[4], ymn[4];
   shiftc(g, y, mu, 1, ym);
   shiftc(g, y, nu, 1, yn);
   shiftc(g, ym, nu, 1, ymn);
-  const M3 unu_fmu = get_link(g, C.g64, nu, ym);  // u_nu(y + mu)
-  const M3 umu_fnu = get_link(g, C.g64, mu, yn);  // u_mu(y + nu)
-  const M3 umu = get_link(g, C.g64, mu, y);
-  const M3 unu = get_link(g, C.g64, nu, y);
-  if (parity(y) == C.cb) {
-    const M3 Lx = lam_at(C, y), Lmn = lam_at(C, ymn);
-    switch (part) {
-      case 0: {  // 1) u_nu(y+mu) L(y+mu+nu) ulc;  5) staple_for L(y)
-        const M3 ulc = mul(dag(umu_fnu), dag(unu));
-        return madd(mul(mul(unu_fmu, Lmn), ulc), mul(mul(unu_fmu, ulc), Lx));
-      }
-      case 1: {  // 4) lrc L(y) u_nu;  8) L(y+mu+nu) staple_back
-        const M3 lrc = mul(dag(unu_fmu), dag(umu));
-        const M3 llc = mul(dag(umu), unu);
-        return madd(mul(mul(lrc, Lx), unu), mul(Lmn, mul(dag(unu_fmu), llc)));
-      }
-      case 2: {  // 4') u_mu(y+nu) L(y+mu+nu) lrc;  7') staple_left L(y)
-        const M3 lrc = mul(dag(unu_fmu), dag(umu));
-        return madd(mul(mul(umu_fnu, Lmn), lrc), mul(mul(umu_fnu, lrc), Lx));
-      }
-      default: {  // 2') ulc L(y) u_mu;  6') L(y+mu+nu) staple_right
-        const M3 ulc = mul(dag(umu_fnu), dag(unu));
-        return madd(mul(mul(ulc, Lx), umu), mul(Lmn, mul(ulc, umu)));
-      }
-    }
-  } else {
-    const M3 Lm = lam_at(C, ym), Ln = lam_at(C, yn);
-    switch (part) {
-      case 0: {  // 2) urc L(y+nu) u_nu^dag;  6) L(y+mu) staple_for
-        const M3 urc = mul(unu_fmu, dag(umu_fnu));
-        const M3 ulc = mul(dag(umu_fnu), dag(unu));
-        return madd(mul(mul(urc, Ln), dag(unu)), mul(Lm, mul(unu_fmu, ulc)));
-      }
-      case 1: {  // 3) u_nu(y+mu)^dag L(y+mu) llc;  7) staple_back L(y+nu)
-        const M3 llc = mul(dag(umu), unu);
-        return madd(mul(mul(dag(unu_fmu), Lm), llc), mul(mul(dag(unu_fmu), llc), Ln));
-      }
-      case 2: {  // 3') urc^dag L(y+mu) u_mu^dag;  8') L(y+nu) staple_left
-        const M3 urc = mul(unu_fmu, dag(umu_fnu));
-        const M3 lrc = mul(dag(unu_fmu), dag(umu));
-        return madd(mul(mul(dag(urc), Lm), dag(umu)), mul(Ln, mul(umu_fnu, lrc)));
-      }
-      default: {  // 1') u_mu(y+nu)^dag L(y+nu) llc^dag;  5') staple_right L(y+mu)
-        const M3 llc = mul(dag(umu), unu);
-        const M3 ulc = mul(dag(umu_fnu), dag(unu));
-        return madd(mul(mul(dag(umu_fnu), Ln), dag(llc)), mul(mul(ulc, umu), Lm));
-      }
-    }
-  }
+  const int py = __builtin_amdgcn_readfirstlane(parity(y));
+  const size_t Vh = g.Vh;
+  auto link = [&](int q, int dir, int i) { return (q ? C.g64[1] : C.g64[0]) + (size_t)dir * 9 * Vh + i; };
+  const int i0 = cb_index(g, y), im = cb_index(g, ym), in = cb_index(g, yn), imn = cb_index(g, ymn);
+  const double2 *A = link(1 - py, nu, im), *G = link(1 - py, mu, in), *E = link(py, mu, i0), *F = link(py, nu, i0);
+  const double2* Lam = C.Lam + (size_t)plane_index(mu, nu) * 9 * Vh;
+  const bool odd = part & 1, low = part < 2, in_cb = py == C.cb, left = odd != in_cb;  // left: X (P W + W Q)
+  const double2 *X = low ? A : G, *Y = low ? (odd ? E : G) : (odd ? F : A), *Z = low ? F : E;
+  const double2 *P = Lam + (in_cb ? imn : (low ? im : in)), *Q = Lam + (in_cb ? i0 : (low ? in : im));
+  const M3 W = mul(load_m3(left ? Y : X, Vh, left || odd), load_m3(left ? Z : Y, Vh, !left || !odd));
+  const M3 T = madd(mul(load_m3(P, Vh, false), W), mul(W, load_m3(Q, Vh, false)));
+  const M3 O = load_m3(left ? X : Z, Vh, left == odd);
+  const M3 R = left ? mul(O, T) : mul(T, O);
+#pragma unroll
+  for (int k = 0; k < 18; ++k) acc.a[k] = fma(f, R.a[k], acc.a[k]);
 }
 
-// ds[mu](x) += ds_mu(x) - tmp_mu(x - nu);  ds[nu](x) -= ds_nu(x) - tmp_nu(x - mu), scaled by `scale`
-__global__ void __launch_bounds__(128) k_force_loops(LoopCtx C, double scale, double2* __restrict__ ds) {
-  const long V = 2L * C.g.Vh;
-  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= V) return;
-  const int p = s >= C.g.Vh ? 1 : 0;
+// ds[mu](x) += scale sum over nu != mu of +- (ds_mu(x) - tmp_mu(x - nu)) of the plane (mu, nu), + for mu < nu.
+// A work-group is the four directions of 64 sites of one checkerboard, so that mu and the insertion's corners are
+// the same in all lanes of a wave and ds is read and written once; both checkerboards of a region follow each
+// other on one XCD, whose L2 then serves most link and Lambda reads.  Bound by those reads and by two waves per
+// SIMD (250 registers).  The six planes of one Lambda on 16^3x32: 156 us, where a launch per plane that kept all
+// four parts of a site took 336.
+__global__ void __launch_bounds__(256) k_force_loops(LoopCtx C, double scale, double2* __restrict__ ds) {
+  const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = xcd_range(blockIdx.x, gridDim.x);
+  const int i = (l >> 1) * 64 + (int)(threadIdx.x & 63);
+  if (i >= C.g.Vh) return;
+  const int p = l & 1;
   int x[4];
-  cb_coords(C.g, p, (int)(s - (long)p * C.g.Vh), x);
-  int xmn[4], xmm[4];
-  shiftc(C.g, x, C.nu, -1, xmn);
-  shiftc(C.g, x, C.mu, -1, xmm);
-  {
-    const M3 a = loop_terms(C, x, 0), b = loop_terms(C, xmn, 1);
-    double2* d = ds + ((size_t)C.mu * V + s) * 9;
+  cb_coords(C.g, p, i, x);
+  double2* d = ds + ((size_t)mu * 2 * C.g.Vh + (size_t)p * C.g.Vh + i) * 9;
+  M3 acc;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const double2 o = d[k];
-      d[k] = make_double2(o.x + scale * (a.a[2 * k] - b.a[2 * k]), o.y + scale * (a.a[2 * k + 1] - b.a[2 * k + 1]));
-    }
+  for (int k = 0; k < 9; ++k) acc.a[2 * k] = d[k].x, acc.a[2 * k + 1] = d[k].y;
+#pragma unroll 1
+  for (int nu = 0; nu < 4; ++nu) {
+    if (nu == mu) continue;
+    const bool first = mu < nu;
+    const int m = first ? mu : nu, n = first ? nu : mu;
+    int xm[4];
+    shiftc(C.g, x, nu, -1, xm);
+    const double f = first ? scale : -scale;
+    add_part(C, m, n, x, first ? 0 : 2, f, acc);
+    add_part(C, m, n, xm, first ? 1 : 3, -f, acc);
   }
-  {
-    const M3 a = loop_terms(C, x, 2), b = loop_terms(C, xmm, 3);
-    double2* d = ds + ((size_t)C.nu * V + s) * 9;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const double2 o = d[k];
-      d[k] = make_double2(o.x - scale * (a.a[2 * k] - b.a[2 * k]), o.y - scale * (a.a[2 * k + 1] - b.a[2 * k + 1]));
-    }
-  }
+  for (int k = 0; k < 9; ++k) d[k] = make_double2(acc.a[2 * k], acc.a[2 * k + 1]);
 }
 
 // ds_full[mu][cb*Vh + i] += f * ds_cb[mu][i]  (the hopping-term derivative's per-checkerboard layout)
@@ -263,16 +225,10 @@ void launch_loops(Op& op, const double2* Lam, int cb, double scale, double2* ds)
   C.g = op.g;
   C.g64[0] = op.gd->g64[0].as<double2>();
   C.g64[1] = op.gd->g64[1].as<double2>();
+  C.Lam = Lam;
   C.cb = cb;
-  int pl = 0;
-  for (int mu = 0; mu < 3; ++mu)
-    for (int nu = mu + 1; nu < 4; ++nu, ++pl) {
-      C.mu = mu;
-      C.nu = nu;
-      C.Lam = Lam + (size_t)pl * 9 * op.Vh;
-      hipLaunchKernelGGL(k_force_loops, dim3((unsigned)((2 * op.Vh + 127) / 128)), dim3(128), 0, op.stream, C, scale, ds);
-      CMX_HIP(hipGetLastError());
-    }
+  hipLaunchKernelGGL(k_force_loops, dim3((unsigned)(2 * ((op.Vh + 63) / 64))), dim3(256), 0, op.stream, C, scale, ds);
+  CMX_HIP(hipGetLastError());
 }
 
 }  // namespace

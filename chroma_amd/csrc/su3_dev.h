@@ -71,9 +71,12 @@ __device__ __forceinline__ M3 get_link(const Geom& g, const double2* const (&g64
   return u;
 }
 __device__ __forceinline__ void shiftc(const Geom& g, const int (&x)[4], int mu, int d, int (&y)[4]) {
-  y[0] = x[0], y[1] = x[1], y[2] = x[2], y[3] = x[3];
-  y[mu] = (x[mu] + d + g.L[mu]) % g.L[mu];
+  // d = +-1; every element with a constant index, so that the coordinates stay in registers
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int v = x[k] + d;
+    y[k] = k != mu ? x[k] : (v == g.L[k] ? 0 : (v < 0 ? g.L[k] - 1 : v));
+  }
 }
-
 
 }  // namespace cmx
