@@ -302,7 +302,12 @@ void dispatch(const BlasLaunch& b, const int p[4], hipStream_t s, const BatchGri
 }
 
 // ------------------------------------------------------------------------------------------------
+// Threads that sum the partials of one reduction.  A group of 16 waves takes half a microsecond more to start and
+// to meet than one of 4, which 434 partials (3.6 / 4.1 us) and three sums over 1024 (3.7 / 4.6 us) do not repay;
+// three sums over 5760 partials do (6.6 / 5.6 us).  The rule holds per problem, in a batch too, whose group has the
+// threads of its largest problem: the others' add zeros at the end, and the bits are those of the single solve.
 constexpr int FIN_THREADS = 1024;
+__host__ __device__ inline int fin_threads(int nb) { return nb <= 2048 ? 256 : FIN_THREADS; }
 
 // the end of a reliable CG iteration (reliable_cg.cc:150-170)
 __device__ __forceinline__ void rcg_end(double* S, int* F) {
@@ -324,26 +329,25 @@ __device__ __forceinline__ void finalize_body(const FinLaunch& L) {
   const int nb = L.nb, nred = L.nred, prog = L.prog, slot = L.slot;
   double* S = L.S;
   int* F = L.F;
-  // each thread sums partials threadIdx.x, + FIN_THREADS, ... in that order, the sums of an entry side by
-  // side; the loads of four entries are issued before their additions, so that the 5000 to 20000 partials
-  // of a large reduction cost one or two load latencies per sum (with 256 threads and one sum after another
-  // three sums over 5760 partials took 6.6 us)
+  // each of the first `step` threads sums partials threadIdx.x, + step, ... in that order, the sums of an entry side
+  // by side; the loads of four entries are issued before their additions
+  const int step = fin_threads(nb);
   double red[3] = {0, 0, 0};
   auto sums = [&](auto nr) {
     constexpr int NR = decltype(nr)::value;
-    int k = threadIdx.x;
-    for (; k + 3 * FIN_THREADS < nb; k += 4 * FIN_THREADS) {
+    int k = threadIdx.x < step ? threadIdx.x : nb;
+    for (; k + 3 * step < nb; k += 4 * step) {
       double t[4][NR];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < NR; ++r) t[j][r] = partials[(size_t)(k + j * FIN_THREADS) * NR + r];
+        for (int r = 0; r < NR; ++r) t[j][r] = partials[(size_t)(k + j * step) * NR + r];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < NR; ++r) red[r] += t[j][r];
     }
-    for (; k < nb; k += FIN_THREADS)
+    for (; k < nb; k += step)
 #pragma unroll
       for (int r = 0; r < NR; ++r) red[r] += partials[(size_t)k * NR + r];
   };
@@ -710,9 +714,6 @@ void launch_blas(int op, const BlasLaunch& b, const int prec[4], hipStream_t s, 
   }
 }
 
-// Up to 256 partials a thread holds one at most, whatever the size of the group, and block_sum adds the
-// waves in order, so that both sizes of group give the same bits and a batch may take its largest problem's.
-static int fin_threads(int nb) { return nb <= 256 ? 256 : FIN_THREADS; }
 void launch_finalize(const FinLaunch& L, hipStream_t s) { hipLaunchKernelGGL(k_finalize, dim3(1), dim3(fin_threads(L.nb)), 0, s, L); }
 void launch_gather_flags(const int* const* flags, int n, int* out, hipStream_t s) {
   hipLaunchKernelGGL(k_gather_flags, dim3(1), dim3(256), 0, s, flags, n, out);
