@@ -663,6 +663,7 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
   // concurrency from free memory and the per-solve workspace
   size_t free_b = 0, total_b = 0;
   CMX_HIP(hipMemGetInfo(&free_b, &total_b));
+  free_b += scratch_cached();
   size_t need = 0;
   for (Op* o : ops) need = std::max(need, fgmres_workspace_bytes(*o, p));
   int conc = (int)std::max<size_t>(1, std::min<size_t>((size_t)np, (size_t)(0.85 * (double)free_b) / std::max<size_t>(need, 1)));

@@ -406,6 +406,17 @@ DevScratch::~DevScratch() {
     (void)hipFree(p_);  // an error may leave work queued: hipFree waits for it
 }
 
+size_t scratch_cached() {
+  int dev = 0;
+  CMX_HIP(hipGetDevice(&dev));
+  Pool& P = pool();
+  std::lock_guard<std::mutex> lk(P.m);
+  size_t n = 0;
+  for (const Cached& c : P.cache)
+    if (c.dev == dev) n += c.cap;
+  return n;
+}
+
 void xfer_release() {
   Pool& P = pool();
   std::vector<Lane*> lanes;

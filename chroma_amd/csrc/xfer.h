@@ -14,6 +14,9 @@ void host_to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
 void device_to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
 // Gives back the pinned staging buffers, the copy threads and the cached scratch that no call is using
 void xfer_release();
+// device bytes of the current device that the cache holds: free memory to a caller that counts it, since an
+// allocation that fails releases them
+size_t scratch_cached();
 
 // Device memory from the bounded cache of earlier calls' buffers (cap: its size, dev: its device), and back
 // to it; work on a buffer that is given back must have completed
