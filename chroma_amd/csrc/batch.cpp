@@ -25,8 +25,8 @@ template <typename T> LaunchRec make_rec(int kind, const T& v, int nblocks) {
 
 void record_hop(Recorder& r, const HopLaunch& h) {
   LaunchRec x = make_rec(REC_HOP, h, hop_num_blocks(h));
-  // everything that selects the kernel template and the work-group size
-  const int k[8] = {h.prec, h.recon, h.fast, h.prefetch, h.isign, h.epi, h.partials != nullptr, h.block};
+  // everything that selects the kernel template (hop_norm: partials and tail) and the work-group size
+  const int k[8] = {h.prec, h.recon, h.fast, h.prefetch, h.isign, h.epi, h.partials ? 1 + h.tail : 0, h.block};
   std::memcpy(x.key, k, sizeof(k));
   r.recs.push_back(std::move(x));
 }
