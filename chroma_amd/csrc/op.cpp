@@ -372,7 +372,9 @@ HopLaunch Op::hop_base(int prec, int which) const {
   h.recon = recon[prec];
   for (int p_ = 0; p_ < 2; ++p_) h.gauge[p_] = (prec == P64 && recon[P64] == 18) ? gd->g64[p_].p : gauge[prec][p_].p;
   std::memcpy(h.ph, gd->ph, sizeof(h.ph));
-  hop_apply_config(h, hcfg[prec][which]);
+  HopConfig c = hcfg[prec][which];
+  if (prec == P16 && which == 1) c.fast &= ~HOP_SPLIT;  // one arithmetic with the multi-source hop (dslash_multi)
+  hop_apply_config(h, c);
   return h;
 }
 
@@ -646,6 +648,16 @@ void Op::autotune() {
         CMX_HIP(hipGetLastError());
       }
       std::vector<HopConfig> cands;
+      // The plain FP16 hop stays on the plane-grid kernel where that is admitted: dslash_multi runs its arithmetic,
+      // from which the direction-split and site-linear kernels differ by rounding.
+      bool plane_only = false;
+      if (prec == P16 && which == 1) {
+        HopLaunch probe = hop_base(prec, which);
+        HopConfig c;
+        c.fast = 1;
+        hop_apply_config(probe, c);
+        plane_only = (probe.fast & 1) != 0;
+      }
       for (int block : {64, 128, 256}) {
         {  // plane-grid kernel, linear or XCD-slab order, links streamed or not (where admitted)
           for (int fm : {1, 1 | HOP_FAST_STREAM}) {
@@ -653,6 +665,7 @@ void Op::autotune() {
             for (int zb : {1, 4, 8}) cands.push_back(HopConfig{block, 1, zb, 0, fm});
           }
         }
+        if (plane_only) continue;
         if (block == 64) cands.push_back(HopConfig{64, 0, 1, 0, 1 | HOP_SPLIT});
         for (int pf : {0, 1}) {  // site-linear kernel; streamed loads on the single-buffered path
           if (pf && prec == P64) continue;

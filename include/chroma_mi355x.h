@@ -113,7 +113,9 @@ int cmx_dslash_apply(cmx_op op, double* chi, const double* psi, int isign, int c
 /* The hopping term on nrhs sources at once (the 12 spin-colour sources of quarkProp4_a,
  * quarkprop4_w.cc:70-117): chi[k] = D psi[k], consecutive Vh*24-double arrays.  At FP16 storage with
  * 12-real links and real boundary phases each link is loaded once per group of 4 sources; otherwise the
- * single-source kernel runs per source.  Results equal nrhs calls of cmx_dslash_apply. */
+ * single-source kernel runs per source.  Results equal nrhs calls of cmx_dslash_apply: bit for bit with the
+ * untuned and the autotuned launch shapes; to FP32 rounding where cmx_op_set_hop_config chose the site-linear
+ * kernel for the plain hopping term or cmx_op_set_multi_group the matrix cores. */
 int cmx_dslash_multi(cmx_op op, int nrhs, double* chi, const double* psi, int isign, int cb, int prec);
 
 /* Even-odd blocks on full-lattice host arrays (V*24 doubles), FP64
