@@ -650,10 +650,10 @@ int cmx_op_get_hop_config(cmx_op h, int prec, int cfg[6]) {
     CMX_REQUIRE(cfg && prec >= 0 && prec <= 2, CMX_ERR_ARG, "get_hop_config: bad argument");
     const int which = cfg[5] == 2 ? 1 : 0;
     const cmx::HopConfig& c = op.hcfg[prec][which];
-    // the kernel actually admitted for this operator (the plane-grid kernel needs 12-real links,
-    // real boundary phases and a field below 2 GiB; otherwise the site-linear kernel runs)
+    // the kernel actually admitted for this operator (the plane-grid and direction-split kernels need 12-real
+    // links, real boundary phases and a field below 2 GiB; otherwise the site-linear kernel runs)
     cfg[0] = c.block, cfg[1] = c.tiled, cfg[2] = c.zb, cfg[3] = c.prefetch;
-    cfg[4] = op.hop_base(prec, which).fast & 3;  // the direction-split kernel (small lattices) shows as plane-grid
+    cfg[4] = op.hop_base(prec, which).fast;
   });
 }
 
@@ -677,7 +677,8 @@ int cmx_op_set_hop_config(cmx_op h, int prec, const int cfg[6]) {
     cmx::Op& op = O(h);
     CMX_REQUIRE(cfg && prec >= 0 && prec <= 2, CMX_ERR_ARG, "set_hop_config: bad argument");
     CMX_REQUIRE(cfg[0] == 64 || cfg[0] == 128 || cfg[0] == 256, CMX_ERR_ARG, "set_hop_config: block must be 64, 128 or 256");
-    CMX_REQUIRE((cfg[1] == 0 || cfg[1] == 1) && cfg[2] >= 1 && (cfg[3] == 0 || cfg[3] == 1) && cfg[4] >= 0 && cfg[4] <= 3,
+    CMX_REQUIRE((cfg[1] == 0 || cfg[1] == 1) && cfg[2] >= 1 && (cfg[3] == 0 || cfg[3] == 1) &&
+                    ((cfg[4] >= 0 && cfg[4] <= 3) || cfg[4] == (1 | cmx::HOP_SPLIT)),
                 CMX_ERR_ARG,
                 "set_hop_config: bad tiling / prefetch flags");
     CMX_REQUIRE(cfg[5] >= 0 && cfg[5] <= 2, CMX_ERR_ARG, "set_hop_config: target must be 0, 1 or 2");

@@ -1057,7 +1057,7 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
   {
     const HopLaunch h = ops[0]->hop_base(ps);
     bres.hop_block = h.block;
-    bres.hop_fast = h.fast & 3;
+    bres.hop_fast = h.fast;
   }
 
   // passes: every problem, then (true-residual mode) the problems whose FP64 residual is above target,

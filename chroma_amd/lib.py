@@ -491,7 +491,7 @@ class Operator:
 
     def hop_config(self, prec, target=1):
         """Launch shape of the EO operator's kernels (target 1) or of the plain hopping term (2);
-        `fast` is the kernel admitted for this operator (bit 0 plane-grid, bit 1 streamed loads)."""
+        `fast` is the kernel admitted for this operator (bit 0 plane-grid, bit 1 streamed loads; 5 direction-split)."""
         cfg = (ctypes.c_int * 6)(0, 0, 0, 0, 0, int(target))
         check(lib().cmx_op_get_hop_config(self.h, int(prec), cfg))
         return dict(block=cfg[0], tiled=cfg[1], zb=cfg[2], prefetch=cfg[3], fast=cfg[4])
@@ -508,7 +508,7 @@ class Operator:
 
     def set_hop_config(self, prec, block=256, tiled=0, zb=1, prefetch=0, fast=0, target=0):
         """fast: 0 site-linear kernel, 1 plane-grid kernel; +2 with the read-once loads (links, clover,
-        xpay input) streamed non-temporally."""
+        xpay input) streamed non-temporally; 5 direction-split kernel."""
         cfg = (ctypes.c_int * 6)(int(block), int(tiled), int(zb), int(prefetch), int(fast), int(target))
         check(lib().cmx_op_set_hop_config(self.h, int(prec), cfg))
 

@@ -248,9 +248,11 @@ int cmx_solve_multishift(cmx_op op, const cmx_solver_params* p, int nshift, cons
  * bit for bit; as many run at once as their workspaces fit in free device memory.  psi[i] is the initial
  * guess on entry; res[i].solve_seconds is the device time of the whole batch. */
 typedef struct {
-  int tune;   /* 1: time candidate launch shapes for the batch (plane-grid or site-linear hopping
-                 kernel, 64/128/256 threads) and keep the fastest; 0: the operators' own shapes, which
-                 must select the same kernel on every problem */
+  int tune;   /* 1: time candidate launch shapes for the batch (direction-split, plane-grid or site-linear
+                 hopping kernel, 64/128/256 threads) and keep the fastest, for this and later batches of the
+                 same lattices, kinds and shared gauge fields (the last 64 such make-ups are kept);
+                 0: the operators' own shapes, which must select the same kernel on every problem where any
+                 of them was set or autotuned; untuned shapes that differ run in a grid per kernel */
   int graph;  /* 1: replay the batched iterations from a captured HIP graph */
   int max_concurrent; /* FGMRES-DR: at most this many solves in flight (0: as many as fit in free device
                          memory); a waiting solve takes over the context of a finished one on the same
@@ -263,7 +265,8 @@ typedef struct {
   int n_stages;          /* kernels per batched iteration                                         */
   long blocks_per_iter;  /* work-groups per batched iteration                                     */
   int hop_block;         /* hopping-kernel launch shape used: threads per work-group              */
-  int hop_fast;          /* 0 site-linear, 1 plane-grid; +2 with streamed read-once loads        */
+  int hop_fast;          /* 0 site-linear, 1 plane-grid; +2 with streamed read-once loads; 5 direction-split
+                            (the first problem's, where they differ)                              */
 } cmx_batch_result;
 int cmx_solve_batch(const cmx_op* ops, int n, const cmx_solver_params* p, const cmx_batch_params* bp,
                     double* const* psi, const double* const* chi, int mdagm, cmx_solver_result* res,
@@ -387,9 +390,13 @@ int cmx_mg_coarse_apply(cmx_op op, const double* in, double* out);
  * cfg = {threads per work-group (64, 128, 256), tiled work-group order (0/1), z planes per tile,
  * double-buffered direction loads (0/1), kernel (0 site-linear, 1 plane-grid -- 12-real links, real
  * boundary phases, fields below 2 GiB; +2 with the loads of data read once per launch -- links,
- * clover, xpay input -- streamed non-temporally), target (0 both, 1 the EO operator's fused kernels,
- * 2 the plain hopping term; for get, 2 reads the plain-hop shape and 0/1 the operator's)}.  No counterpart in the
- * reference beyond QUDA's AutotuneDslash flag (syssolver_quda_clover_params.cc:93-99). */
+ * clover, xpay input -- streamed non-temporally; 5 direction-split, admitted as plane-grid is and below 2^24
+ * sites per checkerboard, 64 threads' sites per work-group whatever cfg[0..3] say, never for the plain FP16
+ * hopping term), target (0 both, 1 the EO operator's fused kernels,
+ * 2 the plain hopping term; for get, 2 reads the plain-hop shape and 0/1 the operator's)}.  get reports the kernel
+ * that runs: where the one asked for is not admitted, plane-grid in place of direction-split and site-linear in
+ * place of both.  What get returns for a target may be set for that target.  The three kernels' results differ by
+ * rounding.  No counterpart in the reference beyond QUDA's AutotuneDslash flag (syssolver_quda_clover_params.cc:93-99). */
 int cmx_op_get_hop_config(cmx_op op, int prec, int cfg[6]);
 int cmx_op_set_hop_config(cmx_op op, int prec, const int cfg[6]);
 int cmx_op_autotune(cmx_op op);
