@@ -203,6 +203,18 @@ def _d(a):
     return a.ctypes.data_as(_dp)
 
 
+def _holds(a, n):
+    """Refuses an array of fewer than the n complex numbers that the library reads or writes in it."""
+    if a.size < n:
+        raise ValueError(f"array of {a.size} complex numbers where the lattice needs {n}")
+    return a
+
+
+def _result(like, n):
+    """A result of the shape of `like`, of which the library writes the first n numbers; zeros behind them."""
+    return np.empty(like.shape, np.complex128) if _holds(like, n).size == n else np.zeros(like.shape, np.complex128)
+
+
 _initialised = False
 
 
@@ -239,7 +251,10 @@ def gauge_stout_smear(L, U, nstep, rho, smear_dirs=15):
     whose bit is set in smear_dirs (15: all, 7: spatial); returns a new complex128[4, V, 3, 3]."""
     init()
     U = np.ascontiguousarray(U, np.complex128)
-    out = np.empty_like(U)
+    n = 36 * int(np.prod(L))
+    out = _result(U, n)
+    if out.size > n:
+        out.ravel()[n:] = U.ravel()[n:]
     check(lib().cmx_gauge_stout_smear_to(_dims(L), _d(U), _d(out), int(nstep), float(rho), int(smear_dirs)))
     return out
 
@@ -353,20 +368,20 @@ class Operator:
 
     def __call__(self, psi, isign=PLUS, prec=DOUBLE):
         psi = np.ascontiguousarray(psi, np.complex128)
-        chi = np.empty_like(psi)
+        chi = _result(psi, 12 * self.nsub)
         check(lib().cmx_op_apply(self.h, _d(chi), _d(psi), int(isign), int(prec)))
         return chi
 
     def dslash(self, psi_cb, isign, cb, prec=DOUBLE):
         psi_cb = np.ascontiguousarray(psi_cb, np.complex128)
-        chi = np.empty_like(psi_cb)
+        chi = _result(psi_cb, 6 * self.V)
         check(lib().cmx_dslash_apply(self.h, _d(chi), _d(psi_cb), int(isign), int(cb), int(prec)))
         return chi
 
     def dslash_multi(self, psis_cb, isign, cb, prec=HALF):
         """D on n sources at once: psis_cb complex[n, Vh, 4, 3]."""
         psis_cb = np.ascontiguousarray(psis_cb, np.complex128)
-        chi = np.empty_like(psis_cb)
+        chi = _result(psis_cb, 6 * self.V * psis_cb.shape[0])
         check(lib().cmx_dslash_multi(self.h, int(psis_cb.shape[0]), _d(chi), _d(psis_cb), int(isign), int(cb),
                                      int(prec)))
         return chi
@@ -530,8 +545,10 @@ class Operator:
         chi = np.ascontiguousarray(chi, np.complex128)
         single = chi.ndim == 3
         chis = chi[None] if single else chi
-        psis = np.empty_like(chis) if psi is None else np.ascontiguousarray(psi, np.complex128).reshape(chis.shape).copy()
         nrhs = chis.shape[0]
+        psis = _result(chis, 12 * self.nsub * nrhs)
+        if psi is not None:
+            psis[...] = np.ascontiguousarray(psi, np.complex128).reshape(chis.shape)
         p = SolverParams(int(solver), int(maxit), float(rsd), float(delta), int(sloppy_prec), int(check_every),
                          int(bool(verbose)), int(bool(true_residual)), int(n_krylov), int(n_defl), int(precond),
                          int(precond_iters), float(precond_rsd), float(precond_omega), int(reorth), int(basis_prec),
@@ -554,7 +571,7 @@ class Operator:
         shifts = np.ascontiguousarray(shifts, np.float64)
         rsd = np.ascontiguousarray(np.broadcast_to(np.asarray(rsd, np.float64), shifts.shape))
         ns = len(shifts)
-        psis = np.empty((ns,) + chi.shape, np.complex128)
+        psis = _result(np.broadcast_to(chi, (ns,) + chi.shape), 12 * self.nsub * ns)
         p = SolverParams(CG, int(maxit), float(rsd.max()), 0.1, DOUBLE, 0, int(bool(verbose)), 0, 16, 0, 0, 4,
                          1e-12, 1.0, 1, -1, 0.0, 0)
         res = (SolverResult * ns)()
@@ -575,8 +592,10 @@ def solve_batch(ops, chis, psis=None, solver=RELIABLE_CG, rsd=1e-10, maxit=10000
     assert len(chis) == n
     chis = [np.ascontiguousarray(c, np.complex128) for c in chis]
     fn = lib().cmx_solve_batch_from_zero if psis is None else lib().cmx_solve_batch
-    psis = [np.empty_like(c) for c in chis] if psis is None else \
+    psis = [_result(c, 12 * o.nsub) for o, c in zip(ops, chis)] if psis is None else \
         [np.ascontiguousarray(x, np.complex128).copy() for x in psis]
+    for o, c, x in zip(ops, chis, psis):
+        _holds(c, 12 * o.nsub), _holds(x, 12 * o.nsub)
     p = SolverParams(int(solver), int(maxit), float(rsd), float(delta), int(sloppy_prec), int(check_every),
                      0, int(bool(true_residual)), int(n_krylov), int(n_defl), int(precond), int(precond_iters),
                      float(precond_rsd), float(precond_omega), int(reorth), int(basis_prec), float(cycle_reduction),
@@ -657,7 +676,7 @@ def net_set_variant(op, prec, variant):
 
 def net_apply(op, v, prec=SINGLE):
     v = np.ascontiguousarray(v, np.complex128)
-    out = np.empty_like(v)
+    out = _result(v, 12 * op.nsub)
     check(lib().cmx_net_apply(op.h, int(prec), _d(out), _d(v)))
     return out
 
