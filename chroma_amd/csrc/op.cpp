@@ -210,8 +210,10 @@ std::shared_ptr<GaugeData> make_gauge(const int dims[4], const double* const lin
 Op::~Op() {
   for (auto& e : graphs) (void)hipGraphExecDestroy(e.exec);
   if (stream && !shared_stream) (void)hipStreamDestroy(stream);
-  if (shared_stream) {
+  if (shared_stream && std::uncaught_exceptions() == 0) {
     pinned_give(hS);
+  } else if (shared_stream) {
+    if (hS) (void)hipHostFree(hS);  // an error may leave a copy into it queued: hipHostFree waits for it
   } else {
     if (hS) (void)hipHostFree(hS);
     if (hF) (void)hipHostFree(hF);
