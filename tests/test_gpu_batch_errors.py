@@ -18,8 +18,13 @@ def test_after_an_error(solver, sloppy):
     chis = [random_fermion(2 * Vh, 10 + k)[Vh:] for k in range(3)]
     kw = dict(solver=solver, rsd=1e-8, sloppy_prec=sloppy, tune=False)
     want = [p.tobytes() for p in cmx.solve_batch([op] * 3, chis, **kw)[0]]
-    for maxit in (2, 5):
+    bad = [chis[0], np.full_like(chis[1], np.nan), chis[2]]
+    raised = 0
+    for src, maxit in ((chis, 2), (bad, 500), (chis, 5), (bad, 500)):
         print("batch error", solver, sloppy, maxit, flush=True)
-        with pytest.raises(cmx.CmxError):
-            cmx.solve_batch([op] * 3, chis, maxit=maxit, **kw)
+        try:  # CG returns what it has at MaxIter, the other solvers raise
+            cmx.solve_batch([op] * 3, src, maxit=maxit, **kw)
+        except cmx.CmxError:
+            raised += 1
         assert [p.tobytes() for p in cmx.solve_batch([op] * 3, chis, **kw)[0]] == want
+    assert raised >= 2
