@@ -115,7 +115,9 @@ struct MesonArgs {
   double2* part;   // [slice of this launch][chunk][momentum][n]
 };
 
-// the phase factors of each direction, from the product k (x - origin) reduced mod L in integers
+// The phase factors of each direction, from the product k (x - origin) reduced in integers: mod L, then to the
+// nearest quarter turn, so that the argument of sincospi stays within 1/4 and its rounding does not show (the whole
+// sum over a slice depends on the factor of one direction coherently).
 __global__ void __launch_bounds__(256) k_meson_phase(MesonArgs A) {
   const int nx = A.g.L[0] + A.g.L[1] + A.g.L[2];
   const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x), m = blockIdx.y;
@@ -124,9 +126,13 @@ __global__ void __launch_bounds__(256) k_meson_phase(MesonArgs A) {
   const int x = q - (d > 0 ? A.g.L[0] : 0) - (d > 1 ? A.g.L[1] : 0);
   const long L = A.g.L[d];
   long r = ((long)A.moms[3 * m + d] * (x - A.g.org[d])) % L;
-  double2 p;
-  sincospi(2.0 * (double)r / (double)L, &p.y, &p.x);
-  A.phase[(size_t)m * nx + q] = p;
+  if (r < 0) r += L;
+  const int j = (int)(4.0 * (double)r / (double)L + 0.5);
+  const long e = 4 * r - j * L;  // r / L = j / 4 + e / (4 L), |e| <= L / 2
+  double s, c;
+  sincospi((double)e / (double)(2 * L), &s, &c);
+  A.phase[(size_t)m * nx + q] = (j & 1) ? ((j & 2) ? make_double2(s, -c) : make_double2(-s, c))
+                                        : ((j & 2) ? make_double2(-c, -s) : make_double2(c, s));
 }
 
 __device__ __forceinline__ double2 cmul2(double2 a, double2 b) {
@@ -252,18 +258,31 @@ template <int NM, bool SAME> __global__ void __launch_bounds__(256, 2) k_meson(M
   }
 }
 
-// out[n][m0 + m][t_eff] = sum over the slice's chunks, in order (deterministic); one lane per (m, n) of a slice
+// s + z with the rounding error of the sum added to e
+__device__ __forceinline__ void two_sum(double& s, double& e, double z) {
+  const double t = s + z, b = t - s;
+  e += (s - (t - b)) + (z - b);
+  s = t;
+}
+
+// out[n][m0 + m][t_eff] = sum over the slice's chunks, in order (deterministic); one lane per (m, n) of a slice.
+// The sum is compensated: the chunks of a coherent sum (the pion at zero momentum) are all alike, and the rounding of
+// the plain sum over some forty of them was most of the result's error (8x10x6x8: 2.2e-16 of the correlators'
+// norm, with it 0.7e-16).
 __global__ void __launch_bounds__(256) k_meson_reduce(MesonArgs A, int m0, int nmom_all, double2* __restrict__ out) {
   const int t = A.t0 + (int)blockIdx.x, q = (int)(blockIdx.y * blockDim.x + threadIdx.x);
   if (q >= A.nmom * 16) return;
   const int m = q >> 4, n = q & 15;
   const double2* p = A.part + (size_t)blockIdx.x * A.nchunk * A.nmom * 16 + q;
-  double2 s = make_double2(0, 0);
+  double2 s = make_double2(0, 0), e = make_double2(0, 0);
+#pragma unroll 8
   for (int c = 0; c < A.nchunk; ++c) {
     const double2 z = p[(size_t)c * A.nmom * 16];
-    s.x += z.x;
-    s.y += z.y;
+    two_sum(s.x, e.x, z.x);
+    two_sum(s.y, e.y, z.y);
   }
+  s.x += e.x;
+  s.y += e.y;
   const int teff = (t - A.g.org[3] % A.g.L[3] + A.g.L[3]) % A.g.L[3];
   out[((size_t)n * nmom_all + m0 + m) * A.g.L[3] + teff] = s;
 }
