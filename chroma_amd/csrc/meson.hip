@@ -12,6 +12,7 @@
 // Propagators: [site][sink spin*3 + colour][source spin*3 + colour] complex, sites in the host order.
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -139,7 +140,9 @@ __device__ __forceinline__ double2 cmul2(double2 a, double2 b) {
   return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 
-template <int NM, bool SAME> __global__ void __launch_bounds__(256, 2) k_meson(MesonArgs A) {
+// DIRECT: both propagators start on 16 bytes, as the direct loads' elements must; a caller's device arrays need only
+// the 8 of a double, and otherwise pass through registers
+template <int NM, bool SAME, bool DIRECT> __global__ void __launch_bounds__(256, 2) k_meson(MesonArgs A) {
   constexpr int SB = MESON_SITES * 144;  // 256 threads x 9 elements of 16 B
   __shared__ __align__(16) double2 stage[2][SAME ? 1 : 2][SB];
   __shared__ double2 shp[2][MESON_SITES * NM];
@@ -161,12 +164,18 @@ template <int NM, bool SAME> __global__ void __launch_bounds__(256, 2) k_meson(M
       const int v = min(v0 + sl, vend - 1);
       const int cb = v >= Vsh ? 1 : 0;
       const size_t at = ((size_t)cb * A.g.Vh + (size_t)t * Vsh + (v - cb * Vsh)) * 144 + e;
-      const int w = (tid & ~63) + 256 * j;  // a wave's 64 elements are consecutive in LDS
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s1 + at),
-                                       (__attribute__((address_space(3))) void*)&stage[buf][0][w], 16, 0, 0);
-      if constexpr (!SAME)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s2 + at),
-                                         (__attribute__((address_space(3))) void*)&stage[buf][1][w], 16, 0, 0);
+      if constexpr (DIRECT) {
+        const int w = (tid & ~63) + 256 * j;  // a wave's 64 elements are consecutive in LDS
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s1 + at),
+                                         (__attribute__((address_space(3))) void*)&stage[buf][0][w], 16, 0, 0);
+        if constexpr (!SAME)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s2 + at),
+                                           (__attribute__((address_space(3))) void*)&stage[buf][1][w], 16, 0, 0);
+      } else {
+        const double *d1 = reinterpret_cast<const double*>(A.s1), *d2 = reinterpret_cast<const double*>(A.s2);
+        stage[buf][0][q] = make_double2(d1[2 * at], d1[2 * at + 1]);
+        if constexpr (!SAME) stage[buf][1][q] = make_double2(d2[2 * at], d2[2 * at + 1]);
+      }
     }
     if (tid < MESON_SITES * NM) {
       const int m = m0 + tid % NM, v = v0 + tid / NM;
@@ -319,10 +328,10 @@ size_t meson_bytes(const ProjGeom& g, int nchunk, int nm, int nt) {
 
 template <int NM> void launch_meson(const MesonArgs& A, int nt, hipStream_t st) {
   const dim3 grid((unsigned)(nt * A.nchunk), (unsigned)((A.nmom + NM - 1) / NM));
-  if (A.s1 == A.s2)
-    hipLaunchKernelGGL((k_meson<NM, true>), grid, dim3(256), 0, st, A);
-  else
-    hipLaunchKernelGGL((k_meson<NM, false>), grid, dim3(256), 0, st, A);
+  const bool direct = ((reinterpret_cast<uintptr_t>(A.s1) | reinterpret_cast<uintptr_t>(A.s2)) & 15) == 0;
+  auto k = A.s1 == A.s2 ? (direct ? k_meson<NM, true, true> : k_meson<NM, true, false>)
+                        : (direct ? k_meson<NM, false, true> : k_meson<NM, false, false>);
+  hipLaunchKernelGGL(k, grid, dim3(256), 0, st, A);
 }
 
 // All momenta and slices, in passes whose partial correlators fit `bytes` of scratch
