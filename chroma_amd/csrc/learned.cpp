@@ -425,6 +425,21 @@ void adam(std::vector<cf>& w, std::vector<float>& m, std::vector<float>& v, cons
 
 void learned_precond_apply(Op& op, int prec, const Vec& in, Vec& out) { forward(op, prec, in, out); }
 
+// the batch's mixed fields and block outputs of m sources
+static void batch_buffers(Op& op, PtcBuffers& b, int prec, int m) {
+  const size_t gbytes = (size_t)8 * 3 * op.Vh * 8;
+  while ((int)b.Gb.size() < m) b.Gb.emplace_back(gbytes);
+  auto &mid0 = b.midb[prec][0], &mid1 = b.midb[prec][1];
+  while ((int)mid0.size() < m) mid0.emplace_back(), mid1.emplace_back();
+  for (int k = 0; k + 1 < (int)op.net->blk.size(); ++k)
+    for (int i = 0; i < m; ++i) scratch_vec((k & 1) ? mid1[i] : mid0[i], prec, op.subset_sites());
+}
+
+void learned_reserve_batch(Op& op, int prec, int ns) {
+  if (!op.net || !op.eo() || ptc_buffers(op).variant[prec] == 2) return;
+  batch_buffers(op, ptc_buffers(op), prec, std::min(ns, PTC_MAXSRC));
+}
+
 void learned_precond_apply_batch(Op& op, int prec, const std::vector<const Vec*>& in, const std::vector<Vec*>& out) {
   const int ns = (int)in.size();
   CMX_REQUIRE(ns == (int)out.size() && ns >= 1, CMX_ERR_ARG, "learned preconditioner: batch size mismatch");
@@ -439,13 +454,10 @@ void learned_precond_apply_batch(Op& op, int prec, const std::vector<const Vec*>
   }
   const int n = op.subset_sites();
   const int nb = (int)op.net->blk.size();
-  const size_t gbytes = (size_t)8 * 3 * op.Vh * 8;
   for (int off = 0; off < ns; off += PTC_MAXSRC) {
     const int m = std::min(PTC_MAXSRC, ns - off);
-    while ((int)b.Gb.size() < m) b.Gb.emplace_back(gbytes);
-    auto& mid0 = b.midb[prec][0];
-    auto& mid1 = b.midb[prec][1];
-    while ((int)mid0.size() < m) mid0.emplace_back(), mid1.emplace_back();
+    batch_buffers(op, b, prec, m);
+    auto &mid0 = b.midb[prec][0], &mid1 = b.midb[prec][1];
     std::vector<const Vec*> src(m);
     for (int i = 0; i < m; ++i) src[i] = in[off + i];
     for (int k = 0; k < nb; ++k) {

@@ -39,8 +39,13 @@ struct DevBuf {
     }
     bytes = n;
   }
-  // from the scratch cache; work on it must have completed when it is released
+  // from the scratch cache, unless too large for it (a batch has dozens of such vectors at once: passing through the
+  // cache they would push everything else out); work on it must have completed when it is released
   void alloc_scratch(size_t n) {
+    if (n > SCRATCH_LARGE) {
+      alloc(n);
+      return;
+    }
     release();
     p = scratch_take(n, cap_, dev_);
     bytes = n;
@@ -225,6 +230,8 @@ void net_apply_host(Op& op, int prec, double* out, const double* in);
 void net_set_variant(Op& op, int prec, int variant);
 void net_grad_host(Op& op, int prec, const double* v, const double* e, double* loss, double* gwc, double* gw0);
 void net_train(Op& op, const cmx_train_params& tp, cmx_train_result& res);
+// allocates what learned_precond_apply_batch of ns sources will use
+void learned_reserve_batch(Op& op, int prec, int ns);
 // out = P(in): the attached network applied to one vector at precision prec (the learned preconditioner)
 void learned_precond_apply(Op& op, int prec, const Vec& in, Vec& out);
 // P(in[i]) -> out[i] for several sources: one launch per kernel and block for all of them, each source's

@@ -639,7 +639,8 @@ size_t fgmres_workspace_bytes(const Op& op, const cmx_solver_params& p) {
   b += (size_t)(2 * total + 1 + 2 * nd + 1 + (nd > 0 && pb != P64 ? 1 : 0)) * spinor_bytes(pb, n);
   if (pb != ps) b += 2 * spinor_bytes(ps, n);
   if (p.precond == CMX_PRECOND_MR) b += 2 * spinor_bytes(ps, n);
-  b += 2 * spinor_bytes(ps, n);  // the operator's even-checkerboard temporaries of a solver context
+  if (p.precond == CMX_PRECOND_MG) b += 2 * spinor_bytes(ps, n);
+  b += 2 * spinor_bytes(ps, n) + spinor_bytes(P64, n);  // the operator's temporaries of a solver context
   // the batched network: a mixed field (8 paths x 3 colours x 8 B per site) and two block outputs per source
   if (p.precond == CMX_PRECOND_LEARNED) b += (size_t)192 * n + 2 * spinor_bytes(ps, n);
   return b;
@@ -689,7 +690,10 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
   std::vector<int> pending, active;
   std::vector<char> packed(np, 0), unpacked(np, 0);
   for (int i = 0; i < np; ++i) pending.push_back(i);
-  // the source and guess on the device and the workspace allocated
+  // The source and guess on the device and everything allocated that the solve will use.  hipMalloc is not free
+  // there: memory that an earlier call has just released is handed out again only once the driver has cleared it,
+  // at some 34 GB/s, so that twelve learned solves on 48^3x96 right after twelve plain ones waited 0.2 to 0.4 s for
+  // the buffers of their first tick.
   auto prepare = [&](int i) {
     Op& op = *ctx[i];
     const int n = op.subset_sites();
@@ -698,6 +702,9 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
     op.work(2, P64, n);
     op.work(3, P64, n);
     FgmresDR::reserve(op, q[i]);
+    op.ensure_prec(p.sloppy_prec);
+    if (op.eo()) op.tmp(p.sloppy_prec, 0), op.tmp(P64, 0);
+    if (p.precond == CMX_PRECOND_MG) op.work(310, p.sloppy_prec, n), op.work(311, p.sloppy_prec, n);
     packed[i] = 1;
   };
   // the timed region: device time of the solves, without the host transfers of the solves that start
@@ -742,6 +749,13 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
   };
   // the first wave is prepared before the timed region
   for (int k = 0; k < std::min(conc, np); ++k) prepare(k);
+  if (p.precond == CMX_PRECOND_LEARNED && (p.basis_prec < 0 || p.basis_prec == p.sloppy_prec)) {
+    int ns = 0;  // the solves that one network launch will cover
+    for (int k = 0; k < std::min(conc, np); ++k)
+      ns += ctx[k]->gd == ctx[0]->gd && ctx[k]->net == ctx[0]->net && ctx[k]->ptc == ctx[0]->ptc &&
+            ctx[k]->stream == ctx[0]->stream;
+    if (ns >= 2) learned_reserve_batch(*ctx[0], p.sloppy_prec, ns);
+  }
   sync_all();
   // a solve that has stopped: its result and true residual, a true-residual restart, or its solution
   // to the host (and a solver context of the batch's own frees its workspace)

@@ -22,6 +22,8 @@ size_t scratch_cached();
 // to it; work on a buffer that is given back must have completed
 void* scratch_take(size_t bytes, size_t& cap, int& dev);
 void scratch_give(void* p, size_t cap, int dev);
+// Buffers above this are not worth caching where many live at once: a sixteenth of what the cache holds
+constexpr size_t SCRATCH_LARGE = (size_t)256 << 20;
 // Small pinned host blocks (PINNED_BLOCK bytes), cached likewise
 constexpr size_t PINNED_BLOCK = 8192;
 void* pinned_take();
