@@ -397,6 +397,7 @@ struct HopLaunch {
                      // else the site-linear kernel of hop_kernel.h; bit 1 (HOP_FAST_STREAM): the
                      // loads of data read once per launch (links, clover, the xpay input) carry the
                      // non-temporal hint
+  int slabs;         // plane-grid kernel, linear order: each XCD owns a contiguous eighth of the planes
   float inv_lxh;     // 1 / (Lx/2), for the fast kernel's plane decomposition
   float inv_ly, inv_lz;  // 1 / Ly, 1 / Lz (direction-split kernel)
   float sgn[4][2];   // real det(U) phase per direction: [bulk | last slice]

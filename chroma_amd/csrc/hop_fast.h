@@ -465,10 +465,8 @@ __device__ __forceinline__ void hop_fast_body(const HopLaunch& h, int blk) {
   // work-group -> (xy tile, plane).  Work-group b runs on XCD b mod 8; with the tiled order each
   // XCD owns a contiguous slab of Lt/8 time slices and walks it (xy tile, z within a block of
   // tile_zb planes, t, z block), so the z +- 1 and t +- 1 neighbours are re-read from its own L2.
-  // The linear order (Lt not a multiple of 8) gives each XCD a contiguous eighth of the planes: handing
-  // them out round-robin instead brings every spinor into several L2s (the EO clover operator at
-  // 24^3x48: 355 us FP64, 173 us FP32, 84 us FP16 round-robin at 256 threads, 248, 116 and 55 us in slabs
-  // at 64 threads).
+  // The linear order gives each XCD a contiguous eighth of the planes (h.slabs) or hands the planes out
+  // round-robin: by the size of a time slice, see hop_slab_order.
   const int gx = (Pl + (int)blockDim.x - 1) / (int)blockDim.x;
   int bx, z, t;
   {
@@ -484,7 +482,7 @@ __device__ __forceinline__ void hop_fast_body(const HopLaunch& h, int blk) {
       z = (q / h.tile_t8) * h.tile_zb + zi;
       t = xcd * h.tile_t8 + tl;
     } else {
-      const int l = xcd_range(b, gx * Lz * Lt);
+      const int l = h.slabs ? xcd_range(b, gx * Lz * Lt) : b;
       bx = l % gx;
       const int plane_ = l / gx;
       z = plane_ % Lz;

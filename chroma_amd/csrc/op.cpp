@@ -36,6 +36,20 @@ int hop_num_blocks(const HopLaunch& h) {
   return (h.g.Vh + h.block - 1) / h.block;
 }
 
+// Order of the plane-grid kernel's linear launch: slabs of planes (an eighth of the lattice per XCD, so that the z and
+// t neighbours are re-read from its own L2) where a time slice of spinors and links stays in reach of the L2, planes
+// round-robin over the XCDs where it does not (presumably because the XCDs then read the same slices at the same time,
+// which one read into the Infinity Cache serves).  EO clover operator, us, slabs / round-robin, each with its best
+// block, by sites of a checkerboard's time slice: FP64 16384 (32^3x64) 807 / 870, (32^3x96) 1216 / 1178, 23328 (36^3x60)
+// 1123 / 1075, 32000 (40^3x60) 1660 / 1470, 42592 (44^3x60) 2298 / 1968, 55296 (48^3x96) 4746 / 4025, 131072 (64^3x48)
+// 5780 / 4691; FP32 32000 742 / 732, 42592 1008 / 984, 55296 2044 / 2006, 131072 2766 / 2302; FP16 16384 182 / 192, 23328
+// 261 / 267, 32000 351 / 347, 42592 491 / 480, 55296 1052 / 1013, 131072 1291 / 1169.  The hop alone, FP64: 23328 352 / 386,
+// 32000 498 / 495, 55296 1608 / 1343; FP16: 32000 118 / 125, 42592 165 / 161, 55296 352 / 348, 131072 425 / 395.
+static bool hop_slab_order(const Geom& g, int prec, int which) {
+  const long slice = (long)g.Lxh * g.L[1] * g.L[2];
+  return slice < (prec == P64 && which == 0 ? 20000 : 40000);
+}
+
 // The launch shape before any tuning (which: 0 the EO operator's kernels, 1 the plain hopping term).
 // The direction-split kernel (hop_split.h) where a wave per 64 sites leaves the chip waiting on latency: at
 // FP64 and FP32 storage up to 340 MB per launch, at FP16 up to 40000 sites.  EO clover operator, us, split
@@ -43,9 +57,12 @@ int hop_num_blocks(const HopLaunch& h) {
 // 24^3x48 (605 MB) 267 / 248; FP32 8^3x16 8.7 / 14.0, 16^3x32 21.2 / 22.7, 24^3x48 (303 MB) 107 / 116;
 // FP16 8^3x16 9.5 / 14.5, 12^3x24 12.4 / 18.3, 16^4 (32768 sites) 13.3 / 13.4, 16^3x32 (65536) 18.2 / 16.1;
 // the plain FP16 hop stays on the plane-grid kernel, whose arithmetic the multi-source hop shares.
-// Else the plane-grid kernel: one wave per work-group where an xy plane is a multiple of 64 sites, else the
-// block that idles the fewest lanes of it (the larger of equals); XCD slabs in blocks of 8 z planes where
-// the lattice admits them; read-once loads streamed once a launch's data no longer fits the 256 MB Infinity
+// Else the plane-grid kernel.  Where its linear order is round-robin (hop_slab_order), that order and the largest block
+// that idles at most an eighth more lanes than 64 threads do (operator, FP64 and FP16, 256 / 128 / 64 threads: 40^3x60
+// 1568 / 1470 / 1481, 48^3x96 FP16 1020 / 1030 / 1031 and the hop 348 / 361 / 366; the tiled order takes 1059 and 353).
+// On smaller slices one wave per work-group where an xy plane is a multiple of 64 sites, else the
+// block that idles the fewest lanes of it (the larger of equals), and XCD slabs in blocks of 8 z planes where
+// the lattice admits them.  Read-once loads streamed once a launch's data no longer fits the 256 MB Infinity
 // Cache, below which streaming throws away what the next launch re-reads (EO clover operator, us, streamed
 // against not: 24^3x48 FP16 67 / 55, 151 MB per launch; 32^3x64 FP16 182 / 212, 478 MB; the hop alone:
 // 24^3x48 FP64 81 / 87, 382 MB).
@@ -70,6 +87,12 @@ HopConfig hop_default_config(const Geom& g, int prec, bool clover, int which) {
     c.zb = 1;
     c.fast = 1 | HOP_SPLIT;
     return c;
+  }
+  if (!hop_slab_order(g, prec, which)) {
+    c.tiled = 0;
+    c.block = 64;
+    for (int b : {128, 256})
+      if (8 * lanes(b) <= 9 * lanes(64)) c.block = b;
   }
   c.fast = 1 | (bytes > 310e6 ? HOP_FAST_STREAM : 0);
   return c;
@@ -377,6 +400,7 @@ HopLaunch Op::hop_base(int prec, int which) const {
   HopConfig c = hcfg[prec][which];
   if (prec == P16 && which == 1) c.fast &= ~HOP_SPLIT;  // one arithmetic with the multi-source hop (dslash_multi)
   hop_apply_config(h, c);
+  h.slabs = hop_slab_order(g, prec, which);
   return h;
 }
 

@@ -27,5 +27,17 @@ int main() {
     for (int k : r.recs[0].key) std::printf(" %d", k);
     std::printf("\n");
   }
+  const int lat[][4] = {{32, 32, 32, 64}, {36, 36, 36, 60}, {40, 40, 40, 60}, {48, 48, 48, 96}, {64, 64, 64, 48}, {16, 16, 16, 32}};
+  for (const auto& L : lat)
+    for (int prec : {(int)cmx::P64, (int)cmx::P32, (int)cmx::P16})
+      for (int which : {0, 1}) {
+        cmx::Geom g;
+        std::memset(&g, 0, sizeof(g));
+        for (int m = 0; m < 4; ++m) g.L[m] = L[m];
+        g.Lxh = L[0] / 2;
+        g.Vh = L[0] / 2 * L[1] * L[2] * L[3];
+        const cmx::HopConfig c = cmx::hop_default_config(g, prec, true, which);
+        std::printf("shape %d %d %d %d %d %d %d\n", L[0], L[3], prec, which, c.block, c.tiled, c.fast);
+      }
   return 0;
 }
