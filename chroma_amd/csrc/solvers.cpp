@@ -169,8 +169,10 @@ int run_batches(Op& op, const cmx_solver_params& p, long tag, const Vec& psi, co
 // holds (F_DONE with F_UPDR: the next iterations' kernels return at once) until update() has run, so the
 // host needs the flags only to launch the update.  On small lattices it reads them one iteration behind the
 // launches, which keeps the device busy over the read-back (15 to 20 us of a 60 to 90 us iteration); the
-// one iteration queued behind a held one exits at once.  On large ones such an exit costs more (20 us per
-// launch of 16384 work-groups, against an iteration of 0.5 ms) and the host waits for each iteration.
+// one iteration queued behind a held one exits at once.  On large ones such an exit costs as much as the wait (20 us
+// per launch of 16384 work-groups) and the host waits for each iteration.  Reliable CG in FP16, nine updates,
+// behind / waiting, ms: 8^3x16 2.02 / 2.16, 16^3x32 3.58 / 3.76, 24^3x28 (193536 sites) 7.52 / 7.63, 24^3x48 11.84 /
+// 11.94, 32^3x64 34.6 / 34.7, 48^3x96 179.7 / 179.6.
 template <typename Inner, typename Update, typename Say>
 void run_held(Op& op, const cmx_solver_params& p, Inner&& inner, Update&& update, Say&& say) {
   const bool ahead = op.subset_sites() <= 200000 && !p.verbose;
@@ -639,8 +641,7 @@ size_t fgmres_workspace_bytes(const Op& op, const cmx_solver_params& p) {
   b += (size_t)(2 * total + 1 + 2 * nd + 1 + (nd > 0 && pb != P64 ? 1 : 0)) * spinor_bytes(pb, n);
   if (pb != ps) b += 2 * spinor_bytes(ps, n);
   if (p.precond == CMX_PRECOND_MR) b += 2 * spinor_bytes(ps, n);
-  if (p.precond == CMX_PRECOND_MG) b += 2 * spinor_bytes(ps, n);
-  b += 2 * spinor_bytes(ps, n) + spinor_bytes(P64, n);  // the operator's temporaries of a solver context
+  b += 2 * spinor_bytes(ps, n);  // the operator's even-checkerboard temporaries of a solver context
   // the batched network: a mixed field (8 paths x 3 colours x 8 B per site) and two block outputs per source
   if (p.precond == CMX_PRECOND_LEARNED) b += (size_t)192 * n + 2 * spinor_bytes(ps, n);
   return b;
@@ -661,7 +662,9 @@ void solve_batch_fgmres(const std::vector<Op*>& ops, const cmx_solver_params& p,
   auto sync_all = [&]() {
     for (hipStream_t s : streams) CMX_HIP(hipStreamSynchronize(s));
   };
-  // concurrency from free memory and the per-solve workspace
+  // Concurrency from free memory and the per-solve workspace.  The 15 % left over are the operator's own buffers, the
+  // FP64 temporary of the residuals among them: counting that as well (18.6 instead of 17.6 GB per solve) makes twelve
+  // learned solves on 48^3x96 run in two waves.
   size_t free_b = 0, total_b = 0;
   CMX_HIP(hipMemGetInfo(&free_b, &total_b));
   free_b += scratch_cached();
@@ -1210,7 +1213,9 @@ void solve_batch(const std::vector<Op*>& ops, const cmx_solver_params& p, const 
         }
       } else {
         // as run_held: a problem holds at an iteration whose FP64 update is due; the flags are read one
-        // iteration behind the launches, and the gated update runs when some problem holds
+        // iteration behind the launches, and the gated update runs when some problem holds.  At every size: the
+        // problems that do not hold use the iteration (twelve sources, behind / waiting, ms: 8^3x16 3.27 / 3.43,
+        // 24^3x48 116.5 / 115.8, 32^3x64 388.7 / 387.2, 48^3x96 1752 / 1772)
         for (hipEvent_t& e : ev.e) CMX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         bool stale = false;  // the coming snapshot precedes an update that covers all that hold in it
         auto issue = [&](long j) {
