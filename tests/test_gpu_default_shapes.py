@@ -27,6 +27,7 @@ def test_default_shapes(L, kind):
         op = cmx.Operator(cmx.Gauge(L, U), kind, mass, 1.0, sloppy_prec=sloppy)
         for prec in (cmx.DOUBLE, sloppy):
             print("default shape", L, kind, prec, op.hop_config(prec), flush=True)
+            assert op.hop_config(prec)["fast"] == 5  # all of these lattices are small enough for the direction-split kernel
             for isign in (+1, -1):
                 assert rel(op(psi[lo:], isign, prec), ref_op(psi, isign)[lo:]) < TOL[prec]
         # |M p|^2 over every work-group: CG reaches its residual only with the right sums

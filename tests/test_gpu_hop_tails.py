@@ -34,6 +34,7 @@ def test_solver_tails(kernel, kind):
         op = cmx.Operator(cmx.Gauge(L, U), kind, mass, 1.0, sloppy_prec=cmx.HALF if prec == cmx.HALF else cmx.SINGLE)
         if kernel != "default":
             op.set_hop_config(prec, block=64, fast=1 if kernel == "plane" else 0)
+        assert op.hop_config(prec)["fast"] == {"default": 5, "plane": 1, "linear": 0}[kernel]  # 5: direction-split
         print("tails", kernel, kind, solver, prec, op.hop_config(prec), flush=True)
         psi_ref, n_ref, _, _ = ref_op.solve(chi, solver=ORACLE[solver], rsd=rsd, maxit=500)
         psi, res = op.solve(chi[lo:], solver=solver, rsd=rsd, maxit=500, delta=0.1, sloppy_prec=prec)
