@@ -55,7 +55,10 @@ static bool hop_slab_order(const Geom& g, int prec, int which) {
 // FP64 and FP32 storage up to 340 MB per launch, at FP16 up to 40000 sites.  EO clover operator, us, split
 // against the best plane-grid shape: FP64 8^3x16 10.6 / 15.3, 12^3x24 17.6 / 24.0, 20^3x40 102 / 120,
 // 24^3x48 (605 MB) 267 / 248; FP32 8^3x16 8.7 / 14.0, 16^3x32 21.2 / 22.7, 24^3x48 (303 MB) 107 / 116;
-// FP16 8^3x16 9.5 / 14.5, 12^3x24 12.4 / 18.3, 16^4 (32768 sites) 13.3 / 13.4, 16^3x32 (65536) 18.2 / 16.1;
+// FP16 8^3x16 9.5 / 14.5, 12^3x24 12.4 / 18.3, 16^4 (32768 sites) 13.3 / 13.4, 16^3x32 (65536) 18.2 / 16.1.
+// The lines lie inside those intervals; close to them the kernels differ by up to a tenth: FP64 20^3x44 (321 MB) 119 /
+// 133, 24^3x28 (353) 137 / 148, 24^3x32 (403) 162 / 165, 22^3x44 (427) 180 / 178; FP32 24^3x54 (340) 131 / 135, 28^3x36
+// (360) 145 / 148, 28^3x44 (440) 180 / 174; FP16 16^3x18 (36864 sites) 15.6 / 14.3, 16^3x20 (40960) 16.0 / 14.8;
 // the plain FP16 hop stays on the plane-grid kernel, whose arithmetic the multi-source hop shares.
 // Else the plane-grid kernel.  Where its linear order is round-robin (hop_slab_order), that order and the largest block
 // that idles at most an eighth more lanes than 64 threads do (operator, FP64 and FP16, 256 / 128 / 64 threads: 40^3x60

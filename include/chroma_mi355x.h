@@ -69,6 +69,9 @@ typedef struct cmx_op_s* cmx_op;
 
 /* ---- lifecycle: initQuda / endQuda hooks (lib/init/chroma_init.cc:215-250, 308-312) ----------- */
 int cmx_init(int device);
+/* Also gives back what the library keeps between calls for the next one's arrays: at most 4 GiB of device scratch,
+ * two sets of 32 MB of pinned slots per device and their threads.  Another allocator of the process gets that memory
+ * only through this call (an allocation of the library's own that fails releases it as well). */
 int cmx_finalize(void);
 const char* cmx_last_error(void);
 int cmx_version(void);
