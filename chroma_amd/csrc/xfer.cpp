@@ -3,9 +3,11 @@
 // slot on the caller's stream, so that the host copies of all threads, the page faults of fresh arrays and
 // the DMA overlap.  The link runs at 57 GB/s each way; every DMA costs some 14 us beside its bytes, so
 // slots are large (4 MB), and waking a thread costs 20 to 50 us, so small arrays use the calling thread
-// alone.  Measured (us, hipMemcpyAsync of pageable memory against this): 256 KB up 107 / 34, 2 MB down
-// 137 / 98, 12 MB down into fresh pages 1177 / 462, 64 MB up 2199 / 1502, down 3784 / 1544, fresh
-// 6183 / 1913, 256 MB up 8939 / 5821, fresh 25180 / 6322.  Chunks that hold only zero bits (an initial
+// alone, and below 1 MB the runtime's own staging is faster.  Measured (us, hipMemcpyAsync of pageable memory against
+// this): up and down again, with buffers used before and in turn, 96 KB 43 / 52, 192 KB 52 / 82, 384 KB 69 / 96,
+// 768 KB 102 / 126, 1152 KB 145 to 170 / 143 to 151, 1536 KB 169 to 194 / 157 to 168, into fresh pages 768 KB 253 / 266,
+// 1152 KB 405 / 367; 2 MB down 137 / 98, 12 MB down into fresh pages 1177 / 462, 64 MB up 2199 / 1502, down 3784 / 1544,
+// fresh 6183 / 1913, 256 MB up 8939 / 5821, fresh 25180 / 6322.  Chunks that hold only zero bits (an initial
 // guess of zero, a point source) are cleared on the device instead of sent.
 //
 // The threads and slots live in a Lane; a call takes a free one, makes one if none is free (at most
@@ -32,7 +34,7 @@ namespace cmx {
 namespace {
 
 constexpr size_t SLOT = (size_t)4 << 20;     // bytes per pinned slot
-constexpr size_t SMALL = (size_t)64 << 10;   // below this the runtime's own path is as fast
+constexpr size_t SMALL = (size_t)1 << 20;    // below this the runtime's own path is faster
 constexpr size_t MIN_CHUNK = (size_t)128 << 10;
 constexpr int MAX_WORKERS = 4, MAX_LANES = 2;
 

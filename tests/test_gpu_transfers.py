@@ -11,8 +11,8 @@ from tests.util import random_fermion
 
 pytestmark = pytest.mark.gpu
 
-# checkerboards of 0.05, 0.07, 3.98, 4.4, 7.96, 8.8 and 16.7 MB
-LATTICES = [(4, 4, 4, 8), (4, 4, 6, 8), (12, 12, 16, 18), (12, 12, 16, 20), (16, 16, 18, 18), (16, 16, 18, 20),
+# checkerboards of 0.05, 0.07, 0.98, 1.08, 3.98, 4.4, 7.96, 8.8 and 16.7 MB
+LATTICES = [(4, 4, 4, 8), (4, 4, 6, 8), (8, 8, 8, 20), (8, 8, 8, 22), (12, 12, 16, 18), (12, 12, 16, 20), (16, 16, 18, 18), (16, 16, 18, 20),
             (16, 16, 20, 34)]
 
 
