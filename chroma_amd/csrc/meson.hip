@@ -103,12 +103,14 @@ struct ProjGeom {
 // Gamma, 256 colour products per site) and read them back per momentum took 2.17 ms, this takes 0.34.
 constexpr int MESON_SITES = 16;
 constexpr int MESON_NM = 8;  // momenta per pass over the propagators
+constexpr size_t MESON_SLAB = (size_t)1 << 30;  // bytes of a host propagator on the device at a time
 
 struct MesonArgs {
   ProjGeom g;
   const double2 *s1, *s2, *coef;
   const int* moms;
   int nmom;    // momenta of this launch
+  int tb, nt;  // the propagators hold the nt time slices from tb on
   int t0;      // first time slice of this launch
   int nchunk;  // work-groups per time slice
   int groups;  // groups of MESON_SITES sites per work-group
@@ -163,7 +165,7 @@ template <int NM, bool SAME, bool DIRECT> __global__ void __launch_bounds__(256,
       const int q = tid + 256 * j, sl = q / 144, e = q - sl * 144;
       const int v = min(v0 + sl, vend - 1);
       const int cb = v >= Vsh ? 1 : 0;
-      const size_t at = ((size_t)cb * A.g.Vh + (size_t)t * Vsh + (v - cb * Vsh)) * 144 + e;
+      const size_t at = ((size_t)(cb * A.nt + (t - A.tb)) * Vsh + (v - cb * Vsh)) * 144 + e;
       if constexpr (DIRECT) {
         const int w = (tid & ~63) + 256 * j;  // a wave's 64 elements are consecutive in LDS
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A.s1 + at),
@@ -334,11 +336,13 @@ template <int NM> void launch_meson(const MesonArgs& A, int nt, hipStream_t st) 
   hipLaunchKernelGGL(k, grid, dim3(256), 0, st, A);
 }
 
-// All momenta and slices, in passes whose partial correlators fit `bytes` of scratch
-void run_meson(const ProjGeom& g, const double2* s1, const double2* s2, const double2* coef, const int* moms, int nmom,
-               double2* part, size_t bytes, double2* out, hipStream_t st) {
+// All momenta of the time slices tb .. tb + ntb - 1, which s1 and s2 hold (even sites, then odd sites, each by t), in passes
+// whose partial correlators fit `bytes` of scratch
+void run_meson(const ProjGeom& g, int tb, int ntb, const double2* s1, const double2* s2, const double2* coef,
+               const int* moms, int nmom, double2* part, size_t bytes, double2* out, hipStream_t st) {
   MesonArgs A;
   A.g = g;
+  A.tb = tb, A.nt = ntb;
   A.s1 = s1, A.s2 = s2, A.coef = coef;
   meson_chunks(g, A.nchunk, A.groups);
   const size_t slice = sizeof(double2) * 16 * (size_t)A.nchunk;  // per momentum
@@ -349,16 +353,16 @@ void run_meson(const ProjGeom& g, const double2* s1, const double2* s2, const do
   while (mstep > 1 && meson_bytes(g, A.nchunk, mstep, 1) > bytes) mstep = (mstep + 1) / 2;
   CMX_REQUIRE(meson_bytes(g, A.nchunk, mstep, 1) <= bytes, CMX_ERR_STATE, "meson_2pt: scratch too small");
   const size_t table = sizeof(double2) * (size_t)nx * mstep;
-  const int tstep = (int)std::min<size_t>(g.L[3], (bytes - table) / (slice * mstep));
+  const int tstep = (int)std::min<size_t>(ntb, (bytes - table) / (slice * mstep));
   A.phase = part, A.part = part + (size_t)nx * mstep;
   for (int m0 = 0; m0 < nmom; m0 += mstep) {
     A.moms = moms + 3 * m0;
     A.nmom = std::min(mstep, nmom - m0);
-    A.t0 = 0;
+    A.t0 = tb;
     hipLaunchKernelGGL(k_meson_phase, dim3((unsigned)((nx + 255) / 256), (unsigned)A.nmom), dim3(256), 0, st, A);
     CMX_HIP(hipGetLastError());
-    for (int t0 = 0; t0 < g.L[3]; t0 += tstep) {
-      const int nt = std::min(tstep, g.L[3] - t0);
+    for (int t0 = tb; t0 < tb + ntb; t0 += tstep) {
+      const int nt = std::min(tstep, tb + ntb - t0);
       A.t0 = t0;
       switch (A.nmom) {
         case 1: launch_meson<1>(A, nt, st); break;
@@ -394,19 +398,38 @@ void meson_2pt(const int dims[4], const double* prop1, const double* prop2, cons
   CMX_REQUIRE(nmom >= 1 && nmom <= 4096 && moms, CMX_ERR_ARG, "meson_2pt: 1..4096 momenta");
   const ProjGeom g = proj_geom(dims, origin);
   const std::vector<double2> coefs = meson_coefs();
-  const size_t pbytes = sizeof(double) * 288 * (size_t)g.V;
+  // Host propagators pass through the device in ranges of time slices whose buffers the scratch cache holds: one of
+  // 4.8 GB (32^3x64) was allocated and freed by every call, and hipMalloc then waited for the driver to clear what the
+  // call before had freed (247 ms per call back to back, 103 without the wait).  A slice's sums do not depend on the range.
+  const size_t slice = sizeof(double) * 288 * (size_t)g.L[0] * g.L[1] * g.L[2];
   const bool same = prop2 == prop1;
+  const int nslab = (int)std::min<size_t>(g.L[3], std::max<size_t>(1, MESON_SLAB / slice));
+  const size_t pbytes = slice * nslab;
   int nchunk, groups;
   meson_chunks(g, nchunk, groups);
   const size_t least = meson_bytes(g, nchunk, 1, 1), whole = meson_bytes(g, nchunk, std::min(nmom, 64), g.L[3]);
   DevScratch d1(pbytes), d2(same ? 0 : pbytes), dp(std::max(least, std::min(whole, MESON_SCRATCH_PART))), dt(sizeof(double2) * coefs.size()),
       dm(sizeof(int) * 3 * (size_t)nmom), dout(sizeof(double2) * 16 * (size_t)nmom * g.L[3]);
-  host_to_device(d1.get(), prop1, pbytes, 0);
-  if (!same) host_to_device(d2.get(), prop2, pbytes, 0);
   CMX_HIP(hipMemcpy(dt.get(), coefs.data(), dt.bytes(), hipMemcpyHostToDevice));
   CMX_HIP(hipMemcpy(dm.get(), moms, dm.bytes(), hipMemcpyHostToDevice));
-  run_meson(g, d1.as<double2>(), same ? d1.as<double2>() : d2.as<double2>(), dt.as<double2>(), dm.as<int>(), nmom,
-            dp.as<double2>(), dp.bytes(), dout.as<double2>(), 0);
+  for (int t = 0; t < g.L[3]; t += nslab) {
+    const int nt = std::min(nslab, g.L[3] - t);
+    const size_t half = slice / 2 * nt;  // a checkerboard's part, on the host and on the device
+    auto up = [&](const DevScratch& d, const double* prop) {
+      for (int cb = 0; cb < 2; ++cb)
+        host_to_device(d.as<char>() + cb * half,
+                       reinterpret_cast<const char*>(prop) + ((size_t)cb * g.L[3] + t) * (slice / 2), half, 0);
+    };
+    if (nt == g.L[3]) {
+      host_to_device(d1.get(), prop1, 2 * half, 0);
+      if (!same) host_to_device(d2.get(), prop2, 2 * half, 0);
+    } else {
+      up(d1, prop1);
+      if (!same) up(d2, prop2);
+    }
+    run_meson(g, t, nt, d1.as<double2>(), same ? d1.as<double2>() : d2.as<double2>(), dt.as<double2>(), dm.as<int>(),
+              nmom, dp.as<double2>(), dp.bytes(), dout.as<double2>(), 0);
+  }
   CMX_HIP(hipMemcpy(corr, dout.get(), dout.bytes(), hipMemcpyDeviceToHost));
 }
 
@@ -437,7 +460,7 @@ void meson_2pt_noalloc(const int dims[4], const double* prop1, const double* pro
   int dev = 0;
   CMX_HIP(hipGetDevice(&dev));
   char* base = static_cast<char*>(g_scratch_ptr[dev]);
-  run_meson(g, reinterpret_cast<const double2*>(prop1), reinterpret_cast<const double2*>(prop2),
+  run_meson(g, 0, g.L[3], reinterpret_cast<const double2*>(prop1), reinterpret_cast<const double2*>(prop2),
             reinterpret_cast<const double2*>(base + MESON_SCRATCH_PART), moms, nmom, reinterpret_cast<double2*>(base),
             MESON_SCRATCH_PART, reinterpret_cast<double2*>(corr), stream);
 }
