@@ -128,9 +128,10 @@ __global__ void __launch_bounds__(256) k_meson_phase(MesonArgs A) {
   const int d = q < A.g.L[0] ? 0 : (q < A.g.L[0] + A.g.L[1] ? 1 : 2);
   const int x = q - (d > 0 ? A.g.L[0] : 0) - (d > 1 ? A.g.L[1] : 0);
   const long L = A.g.L[d];
-  long r = ((long)A.moms[3 * m + d] * (x - A.g.org[d])) % L;
+  const long k = (long)A.moms[3 * m + d] * (x - A.g.org[d]);
+  long r = k == (int)k ? (int)k % (int)L : k % L;  // a 32-bit remainder takes a fraction of a 64-bit one's time
   if (r < 0) r += L;
-  const int j = (int)(4.0 * (double)r / (double)L + 0.5);
+  const int j = (int)(4.0f * (float)r * __builtin_amdgcn_rcpf((float)L) + 0.5f);  // off by one at a tie at most
   const long e = 4 * r - j * L;  // r / L = j / 4 + e / (4 L), |e| <= L / 2
   double s, c;
   sincospi((double)e / (double)(2 * L), &s, &c);
@@ -286,11 +287,16 @@ __global__ void __launch_bounds__(256) k_meson_reduce(MesonArgs A, int m0, int n
   const int m = q >> 4, n = q & 15;
   const double2* p = A.part + (size_t)blockIdx.x * A.nchunk * A.nmom * 16 + q;
   double2 s = make_double2(0, 0), e = make_double2(0, 0);
-#pragma unroll 8
-  for (int c = 0; c < A.nchunk; ++c) {
-    const double2 z = p[(size_t)c * A.nmom * 16];
-    two_sum(s.x, e.x, z.x);
-    two_sum(s.y, e.y, z.y);
+  for (int c = 0; c < A.nchunk; c += 8) {  // eight loads in flight, of few work-groups too
+    double2 z[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      z[j] = c + j < A.nchunk ? p[(size_t)(c + j) * A.nmom * 16] : make_double2(0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      two_sum(s.x, e.x, z[j].x);
+      two_sum(s.y, e.y, z[j].y);
+    }
   }
   s.x += e.x;
   s.y += e.y;
