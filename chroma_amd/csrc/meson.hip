@@ -100,7 +100,7 @@ struct ProjGeom {
 // Gamma and the momenta never meet per site.  At the end the lanes' sums are combined over sites and spins
 // (fixed order) and the work-group writes its 16 x NM partial correlators.
 // 24^3x48, 7 momenta, S_1 = S_2: two kernels that stored the 16 site correlators (one trace per lane and
-// Gamma, 256 colour products per site) and read them back per momentum took 2.17 ms, this takes 0.34.
+// Gamma, 256 colour products per site) and read them back per momentum took 2.17 ms, this takes 0.33.
 constexpr int MESON_SITES = 16;
 constexpr int MESON_NM = 8;  // momenta per pass over the propagators
 constexpr size_t MESON_SLAB = (size_t)1 << 30;  // bytes of a host propagator on the device at a time
